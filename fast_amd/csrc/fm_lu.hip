@@ -38,6 +38,7 @@ template <bool CART> constexpr int lu_ci() { return CART ? FM_LU_CI_CART : FM_LU
 #endif
 #include <algorithm>
 #include <array>
+#include <type_traits>
 #include <vector>
 
 namespace fm {
@@ -221,6 +222,14 @@ __device__ __forceinline__ double lu_ldc(const double* p) {
     return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 __device__ __forceinline__ void lu_stc(double* p, double v) {
+    __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+// the same through a pointer known to be device memory
+typedef __attribute__((address_space(1))) double lu_gdouble;
+__device__ __forceinline__ double lu_ldg(const lu_gdouble* p) {
+    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ void lu_stg(lu_gdouble* p, double v) {
     __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 __device__ __forceinline__ bool lu_any_pending(const double* v, int n) {
@@ -838,29 +847,40 @@ __global__ __launch_bounds__(64) void k_lu_pipe(KZ z, LuArgs a, const double* __
 }
 
 // ---------------------------------------------------------------------------------------
-// Streaming schedule (LU_STREAM, Cartesian zones).  One wave per pencil of 8 x 8 (j, k) lines,
-// sweeping the whole i extent of the LU box as a skewed wavefront: lane (jj, kk) handles cell
-// ii = s - jj - kk of its line at step s of the lower sweep, and ii = R - 1 - s - jj - kk at step
-// s of the upper sweep (R = ni + 14), so the cell it needs from the line before it in j (k) was
+// Streaming schedule (LU_STREAM).  One workgroup of six waves per pencil of 8 x 8 (j, k) lines,
+// sweeping the whole i extent of the LU box as a skewed wavefront: lane (jj, kk) of every wave stands
+// for cell ii = s - jj - kk of its line at step s of the lower sweep, and ii = R - 1 - s - jj - kk at
+// step s of the upper sweep (R = ni + 14), so the cell it needs from the line before it in j (k) was
 // finished one step earlier by lane L -/+ 1 (L -/+ 8).
 //
-//  * The wave solves its 64 cells (the reference's neighbour terms and division) and forms the
-//    three products of each for its consumers in i, j and k: the i product stays in the lane's
-//    registers, the j product moves one lane by a DPP row shift, the k product eight lanes by
-//    ds_bpermute.  No barrier: the wave runs the pencil alone.
+//  * A step is a chain of two halves, each ended by a barrier that orders LDS only.  First half:
+//    waves 0-2 solve one equation of the 64 cells each and wave 3 two (the reference's neighbour terms
+//    and division), from the three products of the step before in LDS.  Second half: waves 0-2 form
+//    the i, j and k products of the solution and put them where the lanes that consume them read
+//    them in the next step, wave 3 stores the results (with the Newton update).  Wave 4 copies the
+//    rows of later steps into LDS, wave 5 brings in the products of the previous pencils.
+//  * Why: a sweep is a chain of ni + nj + nk - 2 steps (plus the hand-overs), and a wave issues one
+//    instruction every five cycles (measured), so a step lasts as long as its longest wave's
+//    instructions.  One wave doing all of it took 0.95 us a step (~850 instructions); two halves of
+//    ~55 and ~65 instructions take 0.40 us.  Products formed by waves that each solve every equation
+//    (one barrier a step) took 0.55 us; rows loaded into registers by each wave 0.57 us (four waves
+//    reading the same rows kept the CU's vector memory path busy for half of the step).
+//    Lower + upper sweep, one wave -> this: 256 x 8 x 8 0.60 -> 0.23 ms, 256 x 128 x 128 1.56 -> 0.81,
+//    256^3 2.93 -> 1.97 ms (there 180 + 238 bytes a cell at 3.2 and 3.8 TB/s bound it), channel
+//    257 x 129 x 33 (3dfull) 1.58 -> 0.68, 513 x 257 x 65 3.23 -> 1.77 ms.
 //  * Inputs come from a skewed, pencil-major copy made before the sweeps (k_lu_pack): row r of a
 //    pencil holds, for each lane, the cell r - jj - kk of its line (right-hand side, state, the
-//    coefficients: 16 doubles), so a step reads whole 512-byte rows, one per array, and every byte
-//    fetched is used.  The wave loads the rows kLuStAhead steps ahead into registers.  The lower
-//    sweep writes dW* back into the right-hand-side rows; the upper sweep reads it from there and
-//    writes dW and the Newton-updated state into the rows it has read, which k_lu_unpack copies
+//    coefficients: 16 doubles), so a step's row is contiguous and every byte fetched is used.  The
+//    lower sweep writes dW* back into the right-hand-side rows; the upper sweep reads it from there
+//    and writes dW and the Newton-updated state into the rows it has read, which k_lu_unpack copies
 //    to the zone arrays.
 //  * Pencils hand their j-face (k-face) products to the next pencil in sweep order through a
-//    global exchange, one value per (pencil, lane, variable, cell), with agent-scope stores; the
-//    consumer lanes load them two steps ahead and re-read values that are still the pending
-//    pattern (bounded waits, error word).  The exchange is filled with the pending pattern before
-//    each sweep (one fill kernel: cheaper than agent-scope stores giving every slot back, whose
-//    write-through holds up the loads issued after them).
+//    global exchange, one value per (pencil, lane, variable, cell), with agent-scope stores; wave 5 of
+//    the consumer loads them two steps ahead and re-reads values that are still the pending
+//    pattern (bounded waits, error word).  A hand-over costs the 8 steps of the pencil's lines and
+//    about 3 us.  The exchange is filled with the pending pattern before each sweep (one fill kernel:
+//    cheaper than agent-scope stores giving every slot back, whose write-through holds up the loads
+//    issued after them).
 //  * Pencils are taken from a counter in diagonal order (reversed for the upper sweep): a pencil
 //    only waits on pencils handed out before it, so there is no deadlock whatever the dispatch
 //    order.
@@ -873,29 +893,17 @@ __global__ __launch_bounds__(64) void k_lu_pipe(KZ z, LuArgs a, const double* __
 // k products 16-24 (lu_normal)
 template <bool CART> constexpr int lu_skf() { return CART ? 16 : 25; }
 __device__ __forceinline__ int lu_skf_of(const KZ& z) { return z.typ == 2 ? 16 : 25; }
-// 1: the B matrices of a step are formed one step ahead (while the step before waits), 0: at the
-// step (as fast at 256^3, and fewer instructions)
-#ifndef FM_LU_ST_COEF_AHEAD
-#define FM_LU_ST_COEF_AHEAD 0
-#endif
-// rows in flight per wave
-#ifndef FM_LU_ST_AHEAD
-#define FM_LU_ST_AHEAD 4
-#endif
-constexpr int kLuStAhead = FM_LU_ST_AHEAD;
-// steps of slack a consumer lane builds up once it had to wait for the previous pencil
-#ifndef FM_LU_ST_SLACK
-#define FM_LU_ST_SLACK 1
-#endif
-constexpr int kLuStSlack = FM_LU_ST_SLACK;
-// s_sleep arguments (units of 64 cycles) of the wait for the slack step and of the re-reads
-#ifndef FM_LU_ST_SLEEP_SLACK
-#define FM_LU_ST_SLEEP_SLACK 4
-#endif
-#ifndef FM_LU_ST_SLEEP_RETRY
-#define FM_LU_ST_SLEEP_RETRY 2
-#endif
-// steps ahead at which a lane loads the products of the previous pencil (divides kLuStAhead)
+// place of array f in a row: the density and 1 / coe5 change places, so that the two arrays the
+// lower sweep does not read (density and coe5) make one aligned pair
+__device__ __forceinline__ constexpr int lu_sk_pos(int f) { return f == 5 ? 14 : f == 14 ? 5 : f; }
+// ring slots of rows per pencil: the rows of the next step and of the RING - 2 steps after it are in
+// LDS or on their way (3dcart 8 slots of 8 KB, 3dfull 4 of 13 KB; 4 to 8 and 3 to 5 slots measure alike).
+// The ring starts the workgroup's LDS and ends below its first 64 KB + 16 B (lu_copy_1k).
+template <bool CART> constexpr int lu_ring() { return CART ? 8 : 4; }
+// steps of slack the halo wave builds up once it had to wait for a previous pencil (0 to 2 measure
+// alike, 4 costs 5 %), and the s_sleep argument (units of 64 cycles) between its re-reads
+constexpr int kLuStSlack = 1, kLuStSleep = 4;
+// steps ahead at which the halo wave loads the products of the previous pencils (1 or 2)
 constexpr int kLuStHalo = 2;
 
 __device__ __forceinline__ long lu_sk_row(int t, int r, int R, int nfld) { return ((long)t * R + r) * nfld * 64; }
@@ -908,39 +916,12 @@ long lu_skew_size(bool cart, int ni, int nj, int nk) {
 // arrays the pack copies, in launch order: the right-hand side, the state (unless a.w_ready), the
 // coefficients, the normals (3dfull, unless a.n_ready)
 
-// exchange slot of value e of cell ii of lane l8 on the j (face 0) or k (face 1) side of the
-// consuming pencil t.  The eight lanes of a face handle cells with the same ii + l8 at one step
-// (in either sweep), so the slots are ordered by ii + l8, then value, then lane: a step reads and
-// writes 64 contiguous bytes per value.
-__device__ __forceinline__ long lu_st_slot(int face, int t, int l8, int e, int ii, int ntile, int ni) {
-    return ((((long)face * ntile + t) * (ni + 7) + ii + l8) * 5 + e) * 8 + l8;
-}
-
+// Exchange: value e of cell ii on line l8 of the j (face 0) or k (face 1) side of consuming pencil t
+// at (((face ntile + t) (ni + 7) + ii + l8) 5 + e) 8 + l8.  The eight lines of a face handle cells with
+// the same ii + l8 at one step (in either sweep), so a step's 40 values are contiguous.
 __host__ __device__ long lu_stream_exchange_size(int ni, int nj, int nk) {
     long nt = (long)((nj + 7) / 8) * ((nk + 7) / 8);
     return 2 * nt * 40 * (long)(ni + 7);
-}
-
-// the value of the lane before this one in j in sweep order: L - 1 (lower) or L + 1 (upper), by
-// a row shift inside rows of 16 lanes (lanes on the first line of the pencil get a value they do
-// not use: they take the j neighbour from the exchange)
-template <bool LOWER>
-__device__ __forceinline__ double lu_from_jprev(double v) {
-    constexpr int ctl = LOWER ? 0x111 : 0x101;   // row_shr:1 / row_shl:1
-    const long long b = __double_as_longlong(v);
-    const int lo = __builtin_amdgcn_update_dpp((int)b, (int)b, ctl, 0xf, 0xf, false);
-    const int hi = __builtin_amdgcn_update_dpp((int)(b >> 32), (int)(b >> 32), ctl, 0xf, 0xf, false);
-    return __longlong_as_double(((long long)hi << 32) | (unsigned int)lo);
-}
-// the value of the lane before this one in k in sweep order: L - 8 (lower) or L + 8 (upper);
-// lanes on the first k line read their own value (they take the k neighbour from the exchange)
-template <bool LOWER>
-__device__ __forceinline__ double lu_from_kprev(double v, int lane) {
-    const long long b = __double_as_longlong(v);
-    const int src = (LOWER ? (lane >= 8 ? lane - 8 : lane) : (lane < 56 ? lane + 8 : lane)) << 2;
-    const int lo = __builtin_amdgcn_ds_bpermute(src, (int)b);
-    const int hi = __builtin_amdgcn_ds_bpermute(src, (int)(b >> 32));
-    return __longlong_as_double(((long long)hi << 32) | (unsigned int)lo);
 }
 
 // The skewed copy: workgroup (t, y, f) writes array f of rows [64 y, 64 y + 64) of pencil t.  Line
@@ -987,7 +968,7 @@ __device__ __forceinline__ void lu_pack_rows(const KZ& z, const LuArgs& a, int n
         T[w + 4 * m][lane] = x;
     }
     __syncthreads();
-    double* __restrict__ dst = a.skw + f * 64 + lane;
+    double* __restrict__ dst = a.skw + lu_sk_pos(f) * 64 + lane;
 #pragma unroll
     for (int m = 0; m < 16; m++) {
         const int rr = w + 4 * m, r = r0 + rr;
@@ -1050,7 +1031,7 @@ __device__ __forceinline__ void lu_unpack_rows(const KZ& z, const LuArgs& a, int
     const long nd = z.nd;
     const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
     const int nfld = lu_skf_of(z);
-    const double* __restrict__ src = a.skw + f * 64 + lane;
+    const double* __restrict__ src = a.skw + lu_sk_pos(f) * 64 + lane;
     double v[16];
 #pragma unroll
     for (int m = 0; m < 16; m++) {
@@ -1102,272 +1083,365 @@ __global__ __launch_bounds__(256) void k_lu_fill_list(const LuZone* __restrict__
         a.stx[e] = __longlong_as_double(kLuPending);
 }
 
-// One pencil (jt, kt) of a sweep, in sweep-order tile coordinates.
+// LDS of a pencil, in doubles: the rows in flight (lu_ring() slots of lu_skf() arrays, rounded up to
+// whole 1 KB copies), then the products a step hands to the next one (value e of the i, j or k product
+// d = 0, 1, 2, at the lane that consumes it: [5 d + e][lane]) and the solution of the step ([e][lane])
+template <bool CART> constexpr int lu_slot_doubles() { return (lu_skf<CART>() + 1) / 2 * 128; }
+template <bool CART> constexpr int lu_lds_doubles() { return lu_ring<CART>() * lu_slot_doubles<CART>() + 20 * 64; }
+constexpr int kLuStThreads = 6 * 64;
+
+// End of a half step: the LDS writes of every wave are visible to the others.  Only LDS is ordered: a
+// __syncthreads() would also wait for the wave's global stores and loads in flight.
+__device__ __forceinline__ void lu_step_barrier() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
+// 1 KB from device memory straight into LDS: lane l copies the 16 bytes at src + 16 l to LDS byte
+// dst + 16 l.  In asm, with no register written, because the compiler would wait for every copy in
+// flight before the wave's next LDS read; lu_copy_wait counts them instead (the wave that copies
+// makes no other vector memory access inside the sweep).  dst stays below 64 KB.
+__device__ __forceinline__ void lu_copy_1k(const lu_gdouble* src, int lane16, int dst) {
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(dst), "v"(lane16), "s"(src)
+                 : "memory", "m0");
+}
+template <int N>
+__device__ __forceinline__ void lu_copy_wait() {
+    static_assert(N <= 63, "vmcnt holds 6 bits");
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
+}
+
+// What the sweep waves share of pencil (jt, kt), in sweep-order tile coordinates
 template <bool CART, bool LOWER>
-__device__ __forceinline__ void lu_pencil(const KZ& z, const LuArgs& a, int jt, int kt, int ntj, int ntk) {
-    constexpr int NF = lu_skf<CART>();
-    const int L = threadIdx.x, jj = L & 7, kk = L >> 3;
-    const int ni = a.i1 - a.i0 + 1, nj = a.j1 - a.j0 + 1, nk = a.k1 - a.k0 + 1;
-    const int R = ni + 14;
-    const int ntile = ntj * ntk;
-    const LUC<> c = lu_const<double>(z);
-    double* __restrict__ X = a.stx;
-    double* __restrict__ SK = a.skw;
-    int* err = a.sync + 1;
-    const bool kalias = !LOWER && a.rop_k != a.rop;
-    const bool newton = !LOWER && a.newton;
-    const double tci = z.ti[0], tcj = z.tj[0], tck = z.tk[0];
-    const double cvinv = 1. / z.cv, cvinv2 = 0.5 * cvinv;
+struct LuPencil {
+    int jt, kt, ntj, ntk, ni, nj, nk, R, ntile, tileid, L, jj, kk;
+    lu_gdouble* X;           // exchange
+    lu_gdouble* SK;          // rows
+    double* S;               // LDS: rows, products, solution
+    double* P;
+    double* W;
+    bool lane_ok;
+    static constexpr int NF = lu_skf<CART>(), RING = lu_ring<CART>(), SLOT = lu_slot_doubles<CART>();
     // first and last line of a pencil in sweep order
-    const int first = LOWER ? 0 : 7, last = LOWER ? 7 : 0;
-    {
-        const int tileid = jt + ntj * kt;
-        const int oj = jt * 8 + jj, ok = kt * 8 + kk;
-        const bool lane_ok = oj < nj && ok < nk;
-        // the lane's neighbours in j and k before it in sweep order, inside the LU box
-        const bool hjn = LOWER ? oj > 0 : oj + 1 < nj;
-        const bool hkn = LOWER ? ok > 0 : ok + 1 < nk;
-        // the lanes of the first line in j (k) take the products of the previous pencil; those of
-        // the last line hand theirs to the next pencil
-        const bool get_j = lane_ok && jj == first && hjn;
-        const bool get_k = lane_ok && kk == first && hkn;
-        const bool put_j = lane_ok && jj == last && (LOWER ? oj + 1 < nj : oj > 0);
-        const bool put_k = lane_ok && kk == last && (LOWER ? ok + 1 < nk : ok > 0);
-        const int tj_next = put_j ? (LOWER ? jt + 1 : jt - 1) + ntj * kt : 0;
-        const int tk_next = put_k ? jt + ntj * (LOWER ? kt + 1 : kt - 1) : 0;
-        // value e of cell ii on the lane's face: hjp + (ii * 5 + e) * 8 (hkp)
-        double* hjp = X + lu_st_slot(0, tileid, kk, 0, 0, ntile, ni);
-        double* hkp = X + lu_st_slot(1, tileid, jj, 0, 0, ntile, ni);
-        // the lane's cell at step s
-        auto cell = [&](int s) { return (LOWER ? s : R - 1 - s) - jj - kk; };
+    static constexpr int first = LOWER ? 0 : 7, last = LOWER ? 7 : 0;
+    __device__ __forceinline__ LuPencil(const LuArgs& a, int jt_, int kt_, int ntj_, int ntk_, double* S_)
+        : jt(jt_), kt(kt_), ntj(ntj_), ntk(ntk_), ni(a.i1 - a.i0 + 1), nj(a.j1 - a.j0 + 1), nk(a.k1 - a.k0 + 1),
+          R(ni + 14), ntile(ntj_ * ntk_), tileid(jt_ + ntj_ * kt_), L(threadIdx.x & 63), jj(L & 7), kk(L >> 3),
+          X((lu_gdouble*)a.stx), SK((lu_gdouble*)a.skw), S(S_), P(S_ + RING * SLOT), W(P + 15 * 64),
+          lane_ok(jt_ * 8 + jj < nj && kt_ * 8 + kk < nk) {}
+    // steps, an even number (the last one may hold no cell)
+    __device__ __forceinline__ int steps() const { return (R + 1) & ~1; }
+    // row and cell of the lane at step s
+    __device__ __forceinline__ int row(int s) const { return LOWER ? s : R - 1 - s; }
+    __device__ __forceinline__ int cell(int s) const { return row(s) - jj - kk; }
+    __device__ __forceinline__ bool active(int s) const { return lane_ok && (unsigned)cell(s) < (unsigned)ni; }
+    __device__ __forceinline__ lu_gdouble* row_ptr(int s) const { return SK + lu_sk_row(tileid, row(s), R, NF); }
+};
 
-        // the rows of steps s .. s + kLuStAhead - 1 in flight (slot s % kLuStAhead); the lower sweep
-        // reads neither the density nor coe5
-        double in[kLuStAhead][NF];
-        auto rows = [&](int s, int q) {
-            const int sc = s < R ? s : R - 1;
-            const double* __restrict__ p = SK + lu_sk_row(tileid, LOWER ? sc : R - 1 - sc, R, NF) + L;
-#pragma unroll
-            for (int f = 0; f < NF; f++)
-                if (!(LOWER && (f == 5 || f == 15))) in[q][f] = p[f * 64];
-        };
-        // halo products of step s, kLuStHalo steps ahead (buffer s % kLuStHalo), loaded by the
-        // lanes that take them (the exchange is read by those lanes only: no other lane touches it)
-        double hj[kLuStHalo][5], hk[kLuStHalo][5];
-        auto hload = [&](int s, int bsel) {
-            const int ii = cell(s);
-            const bool v = s < R && ii >= 0 && ii < ni;
-            if (get_j && v) {
-#pragma unroll
-                for (int e = 0; e < 5; e++) hj[bsel][e] = lu_ldc(hjp + (ii * 5 + e) * 8);
-            }
-            if (get_k && v) {
-#pragma unroll
-                for (int e = 0; e < 5; e++) hk[bsel][e] = lu_ldc(hkp + (ii * 5 + e) * 8);
-            }
-        };
-        // the products of the previous step: i (own next cell), and the j and k products of the
-        // lanes before, already moved
-        double pi[5], bj[5], bk[5];
-#pragma unroll
-        for (int e = 0; e < 5; e++) { pi[e] = 0.; bj[e] = 0.; bk[e] = 0.; }
+// ROLE 0-2: equation ROLE of every cell, then the i, j or k product; ROLE 3: equations 3 and 4, then
+// the results.  KAL: the k products see the updated state (in-place sub-iterations).
+template <bool CART, bool LOWER, bool KAL, int ROLE>
+__device__ __forceinline__ void lu_sweep_wave(const KZ& z, const LuArgs& a, const LuPencil<CART, LOWER>& pc) {
+    constexpr int RING = LuPencil<CART, LOWER>::RING, SLOT = LuPencil<CART, LOWER>::SLOT;
+    constexpr int E0 = ROLE, NE = ROLE == 3 ? 2 : 1;      // the equations of this wave
+    constexpr bool PROD = ROLE < 3;
+    const int L = pc.L, ni = pc.ni, nj = pc.nj, nk = pc.nk, jt = pc.jt, kt = pc.kt, ntj = pc.ntj;
+    const int oj = jt * 8 + pc.jj, ok = kt * 8 + pc.kk;
+    const LUC<> c = lu_const<double>(z);
+    const bool newton = !LOWER && a.newton;
+    const double tc = CART ? (ROLE == 0 ? z.ti[0] : ROLE == 1 ? z.tj[0] : z.tk[0]) : 0.;
+    const double cvinv = 1. / z.cv, cvinv2 = 0.5 * cvinv, cv = z.cv;
+    // the lane's neighbours in j and k before it in sweep order, inside the LU box
+    const bool hjn = LOWER ? oj > 0 : oj + 1 < nj;
+    const bool hkn = LOWER ? ok > 0 : ok + 1 < nk;
+    // a pencil with lanes that have none (elsewhere only the first 15 steps hold lanes whose cell
+    // has no i neighbour)
+    const bool edge = LOWER ? jt == 0 || kt == 0 : jt == ntj - 1 || kt == pc.ntk - 1;
 
+    // what this wave uses of a row: right-hand side, xal, 1 / coe5 (upper: coe5) of its equations;
+    // state, coe and normal of its product; state and density for the update
+    struct Row { double x[NE], al, dg, c5, w[4], cd, n[3], ro; };
+    constexpr bool kUpdates = !LOWER && (ROLE == 3 || (KAL && ROLE == 2));
+    auto read_row = [&](int s, Row& r) {
+        const double* q = pc.S + (s % RING) * SLOT + L;
 #pragma unroll
-        for (int q = 0; q < kLuStAhead; q++) rows(q, q);
+        for (int e = 0; e < NE; e++) r.x[e] = q[(E0 + e) * 64];
+        r.dg = q[lu_sk_pos(14) * 64];
+        r.al = q[lu_sk_pos(10) * 64];
+        if (!LOWER) r.c5 = q[lu_sk_pos(15) * 64];
+        if (kUpdates) r.ro = q[lu_sk_pos(5) * 64];
+        if (PROD || kUpdates) {
 #pragma unroll
-        for (int q = 0; q < kLuStHalo; q++) hload(q, q);
-        // the B matrices of the three products of a step, formed before it waits on its
-        // neighbours (they do not depend on the solution; with in-place sub-iterations the k
-        // matrix takes the updated state and is formed with the product)
-        LuB<double> B0, B1, B2;
-        auto coefs = [&](int qn) {
-            const double u = in[qn][6], v = in[qn][7], w = in[qn][8], t = in[qn][9];
-            const double ci = LOWER ? in[qn][11] : -in[qn][11], cj = LOWER ? in[qn][12] : -in[qn][12];
-            const double ck = LOWER ? in[qn][13] : -in[qn][13];
-            if (CART) {
-                B0 = lu_coef<true, 0, double>(c, u, v, w, t, ci, tci, 0., 0.);
-                B1 = lu_coef<true, 1, double>(c, u, v, w, t, cj, tcj, 0., 0.);
-                if (!(newton && kalias)) B2 = lu_coef<true, 2, double>(c, u, v, w, t, ck, tck, 0., 0.);
+            for (int e = 0; e < 4; e++) r.w[e] = q[lu_sk_pos(6 + e) * 64];
+        }
+        if (PROD) {
+            r.cd = q[lu_sk_pos(11 + ROLE) * 64];
+            if (!CART) {
+#pragma unroll
+                for (int e = 0; e < 3; e++) r.n[e] = q[lu_sk_pos(16 + 3 * ROLE + e) * 64];
             }
-            // (3dfull: the full 5 x 5 matrices are formed at their step, registers being short)
+        }
+    };
+    // mjr_newton.for: the Newton-updated state of a cell with increment x
+    auto update = [&](const Row& r, const double x[5], double o[5]) {
+        const double r0 = r.ro, u = r.w[0], v = r.w[1], w = r.w[2], t = r.w[3];
+        const double r1 = r0 + x[0];
+        const double r_1 = 1. / r1;
+        const double u1 = (r0 * u + x[1]) * r_1, v1 = (r0 * v + x[2]) * r_1, w1 = (r0 * w + x[3]) * r_1;
+        const double roe_old = r0 * (cv * t + 0.5 * (u * u + v * v + w * w));
+        o[0] = r1; o[1] = u1; o[2] = v1; o[3] = w1;
+        o[4] = (roe_old + x[4]) * r_1 * cvinv - cvinv2 * (u1 * u1 + v1 * v1 + w1 * w1);
+    };
+
+    // the products this wave hands on: inside the pencil to lane `to`, across it (last line) to
+    // the next pencil's exchange
+    const bool last_line = ROLE == 1 ? pc.jj == pc.last : ROLE == 2 ? pc.kk == pc.last : false;
+    const int to = L + (ROLE == 1 ? (LOWER ? 1 : -1) : ROLE == 2 ? (LOWER ? 8 : -8) : 0);
+    const bool put = last_line && (ROLE == 1 ? (LOWER ? oj + 1 < nj : oj > 0) : (LOWER ? ok + 1 < nk : ok > 0));
+    const int tnext = ROLE == 1 ? (LOWER ? jt + 1 : jt - 1) + ntj * kt : jt + ntj * (LOWER ? kt + 1 : kt - 1);
+    lu_gdouble* xp = pc.X + ((ROLE == 2 ? (long)pc.ntile : 0) + tnext) * (ni + 7) * 40 + (ROLE == 1 ? pc.kk : pc.jj);
+
+    // (two barriers before the first step: the first row in place, then read by every wave before its
+    // slot is filled again)
+    Row cur, nxt;
+    lu_step_barrier();
+    read_row(0, cur);
+    lu_step_barrier();
+    // step s; EDGE: lanes may lack a neighbour
+    auto step = [&](int s, auto at_edge) {
+        constexpr bool EDGE = decltype(at_edge)::value;
+        // the equations of this wave: the products of the step before, then, while they arrive, the
+        // matrix of this wave's product
+        double b[3][NE];
+#pragma unroll
+        for (int d = 0; d < 3; d++)
+#pragma unroll
+            for (int e = 0; e < NE; e++) b[d][e] = pc.P[(5 * d + E0 + e) * 64 + L];
+        __builtin_amdgcn_sched_barrier(0);
+        const double cs = LOWER ? cur.cd : -cur.cd;
+        const double t0 = CART ? tc : cur.n[0], t1 = CART ? 0. : cur.n[1], t2 = CART ? 0. : cur.n[2];
+        LuB<double> B;
+        constexpr bool kLate = KAL && ROLE == 2;
+        if (PROD && !kLate) B = lu_coef<CART, ROLE % 3, double>(c, cur.w[0], cur.w[1], cur.w[2], cur.w[3], cs, t0, t1, t2);
+        // the sweep's sign products (coe * 0.5 negated for the upper sweep equals coe * -0.5)
+        // and scaled right-hand side
+        const double xal = LOWER ? cur.al : -cur.al;
+        double x1[NE];
+#pragma unroll
+        for (int e = 0; e < NE; e++) x1[e] = LOWER ? cur.x[e] : cur.x[e] * cur.c5;
+        __builtin_amdgcn_sched_barrier(0);
+        // neighbour terms in the reference order: lower 3dcart J, K, I; lower 3dfull and upper
+        // K, J, I
+        const int ii = pc.cell(s);
+        const bool has[3] = {LOWER ? ii > 0 : ii + 1 < ni, hjn, hkn};
+#pragma unroll
+        for (int qq = 0; qq < 3; qq++) {
+            constexpr int D0 = LOWER && CART ? 1 : 2, D1 = LOWER && CART ? 2 : 1;
+            const int D = qq == 0 ? D0 : qq == 1 ? D1 : 0;
+#pragma unroll
+            for (int e = 0; e < NE; e++) {
+                const double xn = x1[e] + b[D][e] * xal;
+                x1[e] = !EDGE || has[D] ? xn : x1[e];
+            }
+        }
+#pragma unroll
+        for (int e = 0; e < NE; e++) pc.W[(E0 + e) * 64 + L] = x1[e] * cur.dg;
+        lu_step_barrier();
+        // the solution of the step; while it arrives, the row of the next step is asked for
+        double x[5];
+#pragma unroll
+        for (int e = 0; e < 5; e++) x[e] = pc.W[e * 64 + L];
+        read_row(s + 1, nxt);
+        __builtin_amdgcn_sched_barrier(0);
+        if (PROD) {
+            if (kLate) {
+                double o[5];
+                update(cur, x, o);
+                B = lu_coef<CART, 2, double>(c, o[1], o[2], o[3], o[4], cs, t0, t1, t2);
+            }
+            double p[5];
+            lu_apply<CART, ROLE % 3, double>(B, x, p);
+            if (!last_line) {
+#pragma unroll
+                for (int e = 0; e < 5; e++) pc.P[(5 * ROLE + e) * 64 + to] = p[e];
+            }
+            if (ROLE > 0) {
+                const int m = LOWER ? s - 7 : pc.R - 1 - s;
+                if (put && pc.active(s)) {
+#pragma unroll
+                    for (int e = 0; e < 5; e++) lu_stg(xp + (long)m * 40 + e * 8, p[e]);
+                }
+            }
+        } else if (pc.active(s)) {
+            // lower: dW* into the right-hand-side row the upper sweep reads; upper: dW and the
+            // updated state into the row (its copy in LDS was complete a step ago)
+            lu_gdouble* p = pc.row_ptr(s) + L;
+#pragma unroll
+            for (int e = 0; e < 5; e++) p[e * 64] = x[e];
+            if (newton) {
+                double o[5];
+                update(cur, x, o);
+#pragma unroll
+                for (int e = 0; e < 5; e++) p[lu_sk_pos(5 + e) * 64] = o[e];
+            }
+        }
+        cur = nxt;
+        lu_step_barrier();
+    };
+    // the steps whose lanes may lack a neighbour, two at a time, then the others
+    const int steps = pc.steps(), nedge = edge ? steps : 16;
+    for (int s = 0; s < nedge; s += 2) {
+        step(s, std::true_type());
+        step(s + 1, std::true_type());
+    }
+    for (int s = nedge; s < steps; s += 2) {
+        step(s, std::false_type());
+        step(s + 1, std::false_type());
+    }
+}
+
+// The row of step s goes into ring slot s % RING (past the end, the first row again, not used).  In
+// step s every wave reads the row of step s + 1 after the middle of the step, so the slot of step s
+// takes the row of step s + RING, and the row of step s + 2 is in place when the step ends.
+template <bool CART, bool LOWER>
+__device__ __forceinline__ void lu_rows_wave(const LuPencil<CART, LOWER>& pc) {
+    constexpr int NF = LuPencil<CART, LOWER>::NF, RING = LuPencil<CART, LOWER>::RING, SLOT = LuPencil<CART, LOWER>::SLOT;
+    // 1 KB copies of a row: the lower sweep skips the pair (density, coe5)
+    constexpr int kPairs = (NF + 1) / 2, kCopies = kPairs - (LOWER ? 1 : 0);
+    const int base = (int)(unsigned)(size_t)(__attribute__((address_space(3))) double*)pc.S;
+    auto copy_row = [&](int s) {
+        const lu_gdouble* src = pc.row_ptr(s < pc.R ? s : 0);
+        const int dst = base + (s % RING) * SLOT * 8;
+#pragma unroll
+        for (int h = 0; h < kPairs; h++) {
+            if (LOWER && h == 7) continue;
+            if (2 * h + 1 < NF || pc.L < 32) lu_copy_1k(src + h * 128, pc.L * 16, dst + h * 1024);
+        }
+    };
+    for (int q = 0; q < RING; q++) copy_row(q);
+    lu_copy_wait<kCopies * (RING - 2)>();
+    lu_step_barrier();
+    lu_step_barrier();
+    const int steps = pc.steps();
+    for (int s = 0; s < steps; s++) {
+        copy_row(s + RING);
+        lu_step_barrier();
+        lu_copy_wait<kCopies * (RING - 2)>();
+        lu_step_barrier();
+    }
+    lu_copy_wait<0>();
+}
+
+// The products of the previous pencils for step s + 1, into the products in LDS in the second half of
+// step s.  Lane q < 40 takes value q / 8 of line q % 8 of each face: 320 contiguous bytes a step and
+// face, loaded kLuStHalo steps ahead.
+template <bool CART, bool LOWER>
+__device__ __forceinline__ void lu_halo_wave(const LuArgs& a, const LuPencil<CART, LOWER>& pc) {
+    const int L = pc.L, l8 = L & 7, ni = pc.ni, first = pc.first;
+    const bool fromj = L < 40 && (LOWER ? pc.jt > 0 : pc.jt + 1 < pc.ntj) && pc.kt * 8 + l8 < pc.nk;
+    const bool fromk = L < 40 && (LOWER ? pc.kt > 0 : pc.kt + 1 < pc.ntk) && pc.jt * 8 + l8 < pc.nj;
+    const lu_gdouble* hjp = pc.X + (long)pc.tileid * (ni + 7) * 40 + L;
+    const lu_gdouble* hkp = pc.X + ((long)pc.ntile + pc.tileid) * (ni + 7) * 40 + L;
+    double hj[kLuStHalo], hk[kLuStHalo];
+    auto face_row = [&](int s) { return LOWER ? s : pc.R - 8 - s; };
+    auto hload = [&](int s, int b) {
+        const int m = face_row(s);
+        const bool v = (unsigned)(m - l8) < (unsigned)ni;
+        hj[b] = 0.; hk[b] = 0.;
+        if (fromj && v) hj[b] = lu_ldg(hjp + (long)m * 40);
+        if (fromk && v) hk[b] = lu_ldg(hkp + (long)m * 40);
+    };
+    // the halo of step s (buffer b), once no value is pending
+    auto halo = [&](int s, int b) {
+        auto pend = [&]() {
+            return (__double_as_longlong(hj[b]) == kLuPending) | (__double_as_longlong(hk[b]) == kLuPending);
         };
-#if FM_LU_ST_COEF_AHEAD
-        coefs(0);
-#endif
-        for (int s0 = 0; s0 < R; s0 += kLuStAhead) {
-#pragma unroll
-            for (int q = 0; q < kLuStAhead; q++) {
-                const int s = s0 + q;
-                const int ii = cell(s);
-                const bool act = s < R && lane_ok && ii >= 0 && ii < ni;
-                const int hb = q % kLuStHalo;
-#if !FM_LU_ST_COEF_AHEAD
-                coefs(q);
-#endif
-                // the inputs of the step (lanes without a cell read zeros or stale values, never
-                // used)
-                double x[5], wv[5];
-#pragma unroll
-                for (int e = 0; e < 5; e++) {
-                    x[e] = in[q][e];
-                    wv[e] = LOWER && e == 0 ? 0. : in[q][5 + e];
+        if (__builtin_amdgcn_ballot_w64(pend())) {
+            // the previous pencil is about to pass this step: wait until it has also handed over
+            // the cells kLuStSlack steps ahead (it writes its cells in order), so that the steps
+            // after this one find their values in place instead of waiting a round trip each
+            int* err = a.sync + 1;
+            int spins = 0;
+            const int s2 = s + kLuStSlack < ni + 6 ? s + kLuStSlack : ni + 6, m2 = face_row(s2);
+            const bool v2 = (unsigned)(m2 - l8) < (unsigned)ni;
+            for (;;) {
+                double pj = 0., pk = 0.;
+                if (fromj && v2) pj = lu_ldg(hjp + (long)m2 * 40);
+                if (fromk && v2) pk = lu_ldg(hkp + (long)m2 * 40);
+                hload(s, b);
+                const bool p2 = (__double_as_longlong(pj) == kLuPending) | (__double_as_longlong(pk) == kLuPending);
+                if (!__builtin_amdgcn_ballot_w64(pend() | p2)) break;
+                if (++spins > kLuSpinMax ||
+                    ((spins & 63) == 1 && __hip_atomic_load(err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))) {
+                    if (L == 0) __hip_atomic_store(err, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                    break;
                 }
-                // the sweep's divisor, sign products (coe * 0.5 negated for the upper sweep equals
-                // coe * -0.5) and scaled right-hand side
-                const double xal = LOWER ? in[q][10] : -in[q][10], diag = in[q][14];
-                const double ck = LOWER ? in[q][13] : -in[q][13];
-                if (!LOWER) {
-#pragma unroll
-                    for (int e = 0; e < 5; e++) x[e] = x[e] * in[q][15];
-                }
-                // halo products of the previous pencils: while any lane still holds the pending
-                // pattern, the wave re-reads its values (bounded)
-                const bool uj = get_j && act, uk = get_k && act;
-                {
-                    auto pend = [&]() {
-                        bool p = false;
-#pragma unroll
-                        for (int e = 0; e < 5; e++)
-                            p = p | (uj & (__double_as_longlong(hj[hb][e]) == kLuPending)) |
-                                (uk & (__double_as_longlong(hk[hb][e]) == kLuPending));
-                        return p;
-                    };
-                    if (__builtin_amdgcn_ballot_w64(pend())) {
-                        int spins = 0;
-                        // the previous pencil is about to pass this step: wait until it has also
-                        // handed over the cell kLuStSlack steps ahead (it writes its cells in
-                        // order), so that the next steps find their values in place instead of
-                        // waiting one round trip each
-                        {
-                            const int iia = LOWER ? min(ii + kLuStSlack, ni - 1) : max(ii - kLuStSlack, 0);
-                            const double* pa = (uj ? hjp : hkp) + (iia * 5 + 4) * 8;
-                            const bool wa = uj || uk;
-                            double va = wa ? lu_ldc(pa) : 0.;
-                            while (__builtin_amdgcn_ballot_w64(wa && __double_as_longlong(va) == kLuPending)) {
-                                if (++spins > kLuSpinMax ||
-                                    ((spins & 63) == 1 && __hip_atomic_load(err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)))
-                                    break;
-                                __builtin_amdgcn_s_sleep(FM_LU_ST_SLEEP_SLACK);
-                                if (wa) va = lu_ldc(pa);
-                            }
-#pragma unroll
-                            for (int d = 1; d < kLuStHalo; d++) hload(s + d, (hb + d) % kLuStHalo);
-                        }
-                        do {
-                            if (++spins > kLuSpinMax ||
-                                ((spins & 63) == 1 && __hip_atomic_load(err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))) {
-                                if (L == 0) __hip_atomic_store(err, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                                break;
-                            }
-                            __builtin_amdgcn_s_sleep(FM_LU_ST_SLEEP_RETRY);
-                            hload(s, hb);
-                            // every access of the wave done: the steps after this rare path keep
-                            // exact memory counters
-                            __builtin_amdgcn_s_waitcnt(0);
-                        } while (__builtin_amdgcn_ballot_w64(pend()));
-                    }
-                }
-#pragma unroll
-                for (int e = 0; e < 5; e++) {
-                    bj[e] = jj == first ? hj[hb][e] : bj[e];
-                    bk[e] = kk == first ? hk[hb][e] : bk[e];
-                }
-                const bool hi = LOWER ? ii > 0 : ii + 1 < ni;
-                // neighbour terms in the reference order: lower 3dcart J, K, I; lower 3dfull and
-                // upper K, J, I
-#pragma unroll
-                for (int qq = 0; qq < 3; qq++) {
-                    const int D = (LOWER && CART) ? (qq == 0 ? 1 : qq == 1 ? 2 : 0) : (qq == 0 ? 2 : qq == 1 ? 1 : 0);
-                    const bool has = D == 0 ? hi : D == 1 ? hjn : hkn;
-#pragma unroll
-                    for (int e = 0; e < 5; e++) {
-                        const double bb = D == 0 ? pi[e] : D == 1 ? bj[e] : bk[e];
-                        const double xn = x[e] + bb * xal;
-                        x[e] = has ? xn : x[e];
-                    }
-                }
-#pragma unroll
-                for (int e = 0; e < 5; e++) x[e] = x[e] * diag;
-                const double uu = wv[1], vv = wv[2], ww = wv[3], tt = wv[4];
-                // the i and j products (the j product moves one lane by DPP)
-                double pk[5], pj[5];
-                if (CART) {
-                    lu_apply<true, 0, double>(B0, x, pi);
-                    lu_apply<true, 1, double>(B1, x, pj);
-                } else {
-                    const double ci = LOWER ? in[q][11] : -in[q][11], cj = LOWER ? in[q][12] : -in[q][12];
-                    lu_prod<false, 0, double>(c, uu, vv, ww, tt, ci, in[q][16], in[q][17], in[q][18], x, pi);
-                    lu_prod<false, 1, double>(c, uu, vv, ww, tt, cj, in[q][19], in[q][20], in[q][21], x, pj);
-                }
-#pragma unroll
-                for (int e = 0; e < 5; e++) bj[e] = lu_from_jprev<LOWER>(pj[e]);
-                double o[5] = {0., 0., 0., 0., 0.};
-                if (newton) {
-                    // mjr_newton.for: the Newton-updated state; in place (kalias) the k products
-                    // see it
-                    const double r0 = wv[0];
-                    const double r1 = r0 + x[0];
-                    const double r_1 = 1. / r1;
-                    const double u1 = (r0 * uu + x[1]) * r_1, v1 = (r0 * vv + x[2]) * r_1, w1 = (r0 * ww + x[3]) * r_1;
-                    const double roe_old = r0 * (z.cv * tt + 0.5 * (uu * uu + vv * vv + ww * ww));
-                    const double t1 = (roe_old + x[4]) * r_1 * cvinv - cvinv2 * (u1 * u1 + v1 * v1 + w1 * w1);
-                    o[0] = r1; o[1] = u1; o[2] = v1; o[3] = w1; o[4] = t1;
-                }
-                // the k product (moves eight lanes by ds_bpermute)
-                if (newton && kalias) {
-                    if (CART) lu_prod<true, 2, double>(c, o[1], o[2], o[3], o[4], ck, tck, 0., 0., x, pk);
-                    else lu_prod<false, 2, double>(c, o[1], o[2], o[3], o[4], ck, in[q][22], in[q][23], in[q][24], x, pk);
-                } else if (CART) {
-                    lu_apply<true, 2, double>(B2, x, pk);
-                } else {
-                    lu_prod<false, 2, double>(c, uu, vv, ww, tt, ck, in[q][22], in[q][23], in[q][24], x, pk);
-                }
-#pragma unroll
-                for (int e = 0; e < 5; e++) bk[e] = lu_from_kprev<LOWER>(pk[e], L);
-                if (act) {
-                    // lower: dW* into the right-hand-side row the upper sweep reads; upper: dW and
-                    // the updated state into the row just read
-                    double* __restrict__ p = SK + lu_sk_row(tileid, LOWER ? s : R - 1 - s, R, NF) + L;
-#pragma unroll
-                    for (int e = 0; e < 5; e++) p[e * 64] = x[e];
-                    if (newton) {
-#pragma unroll
-                        for (int e = 0; e < 5; e++) p[(5 + e) * 64] = o[e];
-                    }
-                }
-                // the face products for the next pencils
-                if (put_j && act) {
-#pragma unroll
-                    for (int e = 0; e < 5; e++) lu_stc(X + lu_st_slot(0, tj_next, kk, e, ii, ntile, ni), pj[e]);
-                }
-                if (put_k && act) {
-#pragma unroll
-                    for (int e = 0; e < 5; e++) lu_stc(X + lu_st_slot(1, tk_next, jj, e, ii, ntile, ni), pk[e]);
-                }
-                hload(s + kLuStHalo, hb);
-                // the row kLuStAhead steps ahead into the slot just read
-                rows(s + kLuStAhead, q);
-#if FM_LU_ST_COEF_AHEAD
-                coefs((q + 1) % kLuStAhead);
-#endif
+                __builtin_amdgcn_s_sleep(kLuStSleep);
             }
+#pragma unroll
+            for (int d = 1; d < kLuStHalo; d++) hload(s + d, (b + d) % kLuStHalo);
+            // every access of the wave done: the steps after this rare path keep exact memory
+            // counters
+            __builtin_amdgcn_s_waitcnt(0);
+        }
+    };
+    auto hand_in = [&](int b) {
+        if (L < 40) {
+            pc.P[(5 + (L >> 3)) * 64 + first + 8 * l8] = hj[b];
+            pc.P[(10 + (L >> 3)) * 64 + l8 + 8 * first] = hk[b];
+        }
+    };
+#pragma unroll
+    for (int q = 0; q < kLuStHalo; q++) hload(q, q);
+    halo(0, 0);
+    hand_in(0);
+    hload(kLuStHalo, 0);
+    lu_step_barrier();
+    lu_step_barrier();
+    const int steps = pc.steps();
+    for (int s0 = 0; s0 < steps; s0 += 2) {
+#pragma unroll
+        for (int q = 0; q < 2; q++) {
+            constexpr int H = kLuStHalo;
+            halo(s0 + q + 1, (q + 1) % H);
+            lu_step_barrier();
+            hand_in((q + 1) % H);
+            hload(s0 + q + 1 + H, (q + 1) % H);
+            lu_step_barrier();
         }
     }
 }
 
+// One pencil (jt, kt) of a sweep by a workgroup of six waves, in sweep-order tile coordinates.
+template <bool CART, bool LOWER>
+__device__ __forceinline__ void lu_pencil(const KZ& z, const LuArgs& a, int jt, int kt, int ntj, int ntk, double* S) {
+    const int role = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+    const LuPencil<CART, LOWER> pc(a, jt, kt, ntj, ntk, S);
+    if (role == 4) lu_rows_wave<CART, LOWER>(pc);
+    else if (role == 5) lu_halo_wave<CART, LOWER>(a, pc);
+    else if (role == 0) lu_sweep_wave<CART, LOWER, false, 0>(z, a, pc);
+    else if (role == 1) lu_sweep_wave<CART, LOWER, false, 1>(z, a, pc);
+    else if (role == 3) lu_sweep_wave<CART, LOWER, false, 3>(z, a, pc);
+    else if (LOWER || !a.newton || a.rop_k == a.rop) lu_sweep_wave<CART, LOWER, false, 2>(z, a, pc);
+    else lu_sweep_wave<CART, LOWER, true, 2>(z, a, pc);
+}
 
 template <bool CART, bool LOWER>
-__global__ __launch_bounds__(64) void k_lu_stream(KZ z, LuArgs a, int ntj, int ntk) {
+__global__ void __launch_bounds__(kLuStThreads) __attribute__((amdgpu_waves_per_eu(3))) k_lu_stream(KZ z, LuArgs a, int ntj, int ntk) {
+    __shared__ __align__(16) double S[lu_lds_doubles<CART>()];
+    __shared__ int ticket;
     const int ntile = ntj * ntk;
     for (;;) {
-        int tk0 = 0;
-        if (threadIdx.x == 0) tk0 = atomicAdd(a.sync, 1);
-        const int t = __builtin_amdgcn_readfirstlane(tk0);
+        // (the waves have read the last ticket before the first step of its pencil)
+        if (threadIdx.x == 0) ticket = atomicAdd(a.sync, 1);
+        __syncthreads();
+        const int t = __builtin_amdgcn_readfirstlane(ticket);
         if (t >= ntile) break;
         int jt, kt;
         lu_tile_of(t, ntj, ntk, jt, kt);
         if (!LOWER) { jt = ntj - 1 - jt; kt = ntk - 1 - kt; }
-        lu_pencil<CART, LOWER>(z, a, jt, kt, ntj, ntk);
+        lu_pencil<CART, LOWER>(z, a, jt, kt, ntj, ntk, S);
     }
 }
 
@@ -1376,12 +1450,14 @@ __global__ __launch_bounds__(64) void k_lu_stream(KZ z, LuArgs a, int ntj, int n
 // pencils mirrored, so in either sweep a pencil only waits on pencils of its zone handed out before
 // it.  Each zone has its own rows, exchange and error word.
 template <bool CART, bool LOWER>
-__global__ __launch_bounds__(64) void k_lu_stream_list(const LuZone* __restrict__ zones,
-                                                       const LuWork* __restrict__ work, int nwork, int* counter) {
+__global__ void __launch_bounds__(kLuStThreads) __attribute__((amdgpu_waves_per_eu(3)))
+k_lu_stream_list(const LuZone* __restrict__ zones, const LuWork* __restrict__ work, int nwork, int* counter) {
+    __shared__ __align__(16) double S[lu_lds_doubles<CART>()];
+    __shared__ int ticket;
     for (;;) {
-        int tk0 = 0;
-        if (threadIdx.x == 0) tk0 = atomicAdd(counter, 1);
-        const int t = __builtin_amdgcn_readfirstlane(tk0);
+        if (threadIdx.x == 0) ticket = atomicAdd(counter, 1);
+        __syncthreads();
+        const int t = __builtin_amdgcn_readfirstlane(ticket);
         if (t >= nwork) break;
         const LuWork w = work[t];
         const KZ& z = zones[w.zone].z;
@@ -1389,7 +1465,7 @@ __global__ __launch_bounds__(64) void k_lu_stream_list(const LuZone* __restrict_
         const int ntj = (a.j1 - a.j0 + 8) / 8, ntk = (a.k1 - a.k0 + 8) / 8;
         int jt = w.bj, kt = w.bk;
         if (!LOWER) { jt = ntj - 1 - jt; kt = ntk - 1 - kt; }
-        lu_pencil<CART, LOWER>(z, a, jt, kt, ntj, ntk);
+        lu_pencil<CART, LOWER>(z, a, jt, kt, ntj, ntk, S);
     }
 }
 
@@ -1481,14 +1557,14 @@ void stream(const KZ& z, const LuArgs& a, hipStream_t st) {
     int cus = 0, dev = 0, per = 0;
     if (hipGetDevice(&dev) != hipSuccess ||
         hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) cus = 256;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, (const void*)k_lu_stream<CART, true>, 64, 0) != hipSuccess || per < 1)
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, (const void*)k_lu_stream<CART, true>, kLuStThreads, 0) != hipSuccess || per < 1)
         per = 1;
     long cap = (long)per * cus;
     unsigned grid = (unsigned)((long)ntj * ntk < cap ? (long)ntj * ntk : cap);
     hipLaunchKernelGGL(k_fill_lin, dim3((unsigned)((nx + 255) / 256)), dim3(256), 0, st, a.stx, nx, kLuPending, a.sync);
-    hipLaunchKernelGGL((k_lu_stream<CART, true>), dim3(grid), dim3(64), 0, st, z, a, ntj, ntk);
+    hipLaunchKernelGGL((k_lu_stream<CART, true>), dim3(grid), dim3(kLuStThreads), 0, st, z, a, ntj, ntk);
     hipLaunchKernelGGL(k_fill_lin, dim3((unsigned)((nx + 255) / 256)), dim3(256), 0, st, a.stx, nx, kLuPending, a.sync);
-    hipLaunchKernelGGL((k_lu_stream<CART, false>), dim3(grid), dim3(64), 0, st, z, a, ntj, ntk);
+    hipLaunchKernelGGL((k_lu_stream<CART, false>), dim3(grid), dim3(kLuStThreads), 0, st, z, a, ntj, ntk);
     // dW back only if asked (inside fm_compute it is copied once, after the last time step)
     const int f0 = lu_unpack_first(a), f1 = lu_unpack_end(a);
     hipLaunchKernelGGL(k_lu_unpack, dim3((unsigned)(ntj * ntk), (unsigned)((ni + 14 + 63) / 64), (unsigned)(f1 - f0)),
@@ -1600,7 +1676,7 @@ void launch_lu_stream_list(bool cart, const LuZone* zones, int nz, const LuWork*
     if (hipGetDevice(&dev) != hipSuccess ||
         hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) cus = 256;
     const void* kfn = cart ? (const void*)k_lu_stream_list<true, true> : (const void*)k_lu_stream_list<false, true>;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, kfn, 64, 0) != hipSuccess || per < 1) per = 1;
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, kfn, kLuStThreads, 0) != hipSuccess || per < 1) per = 1;
     const long cap = (long)per * cus;
     const unsigned grid = (unsigned)(nwork < cap ? nwork : cap);
     if (npack > 0)
@@ -1609,11 +1685,11 @@ void launch_lu_stream_list(bool cart, const LuZone* zones, int nz, const LuWork*
     for (int lower = 1; lower >= 0; lower--) {
         hipLaunchKernelGGL(k_lu_fill_list, dim3((unsigned)nz, 64), dim3(256), 0, st, zones, counter);
         if (cart) {
-            if (lower) hipLaunchKernelGGL((k_lu_stream_list<true, true>), dim3(grid), dim3(64), 0, st, zones, work, nwork, counter);
-            else hipLaunchKernelGGL((k_lu_stream_list<true, false>), dim3(grid), dim3(64), 0, st, zones, work, nwork, counter);
+            if (lower) hipLaunchKernelGGL((k_lu_stream_list<true, true>), dim3(grid), dim3(kLuStThreads), 0, st, zones, work, nwork, counter);
+            else hipLaunchKernelGGL((k_lu_stream_list<true, false>), dim3(grid), dim3(kLuStThreads), 0, st, zones, work, nwork, counter);
         } else {
-            if (lower) hipLaunchKernelGGL((k_lu_stream_list<false, true>), dim3(grid), dim3(64), 0, st, zones, work, nwork, counter);
-            else hipLaunchKernelGGL((k_lu_stream_list<false, false>), dim3(grid), dim3(64), 0, st, zones, work, nwork, counter);
+            if (lower) hipLaunchKernelGGL((k_lu_stream_list<false, true>), dim3(grid), dim3(kLuStThreads), 0, st, zones, work, nwork, counter);
+            else hipLaunchKernelGGL((k_lu_stream_list<false, false>), dim3(grid), dim3(kLuStThreads), 0, st, zones, work, nwork, counter);
         }
     }
     if (nunpack > 0)
