@@ -931,22 +931,61 @@ __global__ void k_cfl_partial(KZ z, const double* __restrict__ rop, double* __re
     if (tid == 0) { part[blockIdx.x * 3] = smax[0]; part[blockIdx.x * 3 + 1] = smin[0]; part[blockIdx.x * 3 + 2] = ssum[0]; }
 }
 
-__global__ void k_cfl_final(const double* __restrict__ part, int nblk, double* __restrict__ out) {
-    if (threadIdx.x != 0) return;
-    double m = 0., n = 1e8, s = 0.;
-    for (int b = 0; b < nblk; b++) { m = dmax(m, part[3 * b]); n = dmin(n, part[3 * b + 1]); s += part[3 * b + 2]; }
-    out[0] = m; out[1] = n; out[2] = s;
+// Second pass of a reduction: nblk partial results of N values each.  A workgroup brings them into LDS
+// (kFinalBlocks at a time); then each wave runs one kind of operation,
+// its lanes one value each, block by block: the order of the partial results, and so the bits, are
+// those of one thread going through them.  The chain is one LDS read and one operation a block
+// instead of a trip to memory: 512 blocks 177 -> 16 us (norms), 70 -> 11 us (CFL).
+constexpr int kFinalBlocks = 256, kFinalThreads = 256;
+
+template <int N, typename Op>
+__device__ __forceinline__ void reduce_blocks(const double* __restrict__ part, int nblk, double* buf, Op op) {
+    for (int b0 = 0; b0 < nblk; b0 += kFinalBlocks) {
+        const int nb = nblk - b0 < kFinalBlocks ? nblk - b0 : kFinalBlocks;
+        for (int t = threadIdx.x; t < nb * N; t += kFinalThreads) buf[t] = part[b0 * N + t];
+        __syncthreads();
+        op(nb);
+        __syncthreads();
+    }
 }
 
-__global__ void k_norm_final(const double* __restrict__ part, int nblk, double* __restrict__ out) {
-    if (threadIdx.x != 0) return;
-    double s[5] = {0, 0, 0, 0, 0}, m[5] = {0, 0, 0, 0, 0};
-    for (int b = 0; b < nblk; b++)
-        for (int e = 0; e < 5; e++) {
-            s[e] += part[b * 10 + e];
-            if (part[b * 10 + 5 + e] > m[e]) m[e] = part[b * 10 + 5 + e];
+__global__ void __launch_bounds__(kFinalThreads) k_cfl_final(const double* __restrict__ part, int nblk, double* __restrict__ out) {
+    __shared__ double buf[kFinalBlocks * 3];
+    const int w = threadIdx.x >> 6;         // 0 largest, 1 smallest, 2 sum
+    double v = w == 1 ? 1e8 : 0.;
+    reduce_blocks<3>(part, nblk, buf, [&](int nb) {
+        if (threadIdx.x == 0) {
+#pragma unroll 16
+            for (int b = 0; b < nb; b++) v = dmax(v, buf[3 * b]);
+        } else if (threadIdx.x == 64) {
+#pragma unroll 16
+            for (int b = 0; b < nb; b++) v = dmin(v, buf[3 * b + 1]);
+        } else if (threadIdx.x == 128) {
+#pragma unroll 16
+            for (int b = 0; b < nb; b++) v += buf[3 * b + 2];
         }
-    for (int e = 0; e < 5; e++) { out[e] = s[e]; out[5 + e] = m[e]; }
+    });
+    if ((threadIdx.x & 63) == 0 && w < 3) out[w] = v;
+}
+
+__global__ void __launch_bounds__(kFinalThreads) k_norm_final(const double* __restrict__ part, int nblk, double* __restrict__ out) {
+    __shared__ double buf[kFinalBlocks * 10];
+    const int w = threadIdx.x >> 6, e = threadIdx.x & 63;     // wave 0 sums, wave 1 largest; equation e
+    double v = 0.;
+    reduce_blocks<10>(part, nblk, buf, [&](int nb) {
+        if (e >= 5) return;
+        if (w == 0) {
+#pragma unroll 16
+            for (int b = 0; b < nb; b++) v += buf[10 * b + e];
+        } else if (w == 1) {
+#pragma unroll 16
+            for (int b = 0; b < nb; b++) {
+                const double p = buf[10 * b + 5 + e];
+                if (p > v) v = p;
+            }
+        }
+    });
+    if (e < 5 && w < 2) out[5 * w + e] = v;
 }
 
 // Kinetic energy and volume sums over the interior (POST/computePT_enstrophy.cpp, tke part)
@@ -1160,12 +1199,12 @@ void launch_coins_list(const CoinsZone* zones, int nz, int nblk, hipStream_t st)
 
 void launch_norms(const KZ& z, const double* dr, double* part, int nblk, double* out, hipStream_t st) {
     hipLaunchKernelGGL(k_norm_partial, dim3(nblk), dim3(256), 0, st, z, dr, part);
-    hipLaunchKernelGGL(k_norm_final, dim3(1), dim3(64), 0, st, part, nblk, out);
+    hipLaunchKernelGGL(k_norm_final, dim3(1), dim3(kFinalThreads), 0, st, part, nblk, out);
 }
 
 void launch_cfl(const KZ& z, const double* rop, double* part, int nblk, double* out, hipStream_t st) {
     hipLaunchKernelGGL(k_cfl_partial, dim3(nblk), dim3(256), 0, st, z, rop, part);
-    hipLaunchKernelGGL(k_cfl_final, dim3(1), dim3(64), 0, st, part, nblk, out);
+    hipLaunchKernelGGL(k_cfl_final, dim3(1), dim3(kFinalThreads), 0, st, part, nblk, out);
 }
 
 void launch_tke(const KZ& z, const double* ro, double* part, int nblk, hipStream_t st) {
