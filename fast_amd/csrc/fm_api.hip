@@ -80,7 +80,7 @@ struct Zone {
 struct fm_ctx {
     int device;
     int lu_schedule;         // LU_PIPELINE or LU_BLOCKS
-    int res_schedule;        // RES_CELLS, RES_FACES, RES_KCOL or RES_AUTO (per zone)
+    int res_schedule;        // RES_CELLS, RES_FACES, RES_KCOL or RES_AUTO
     hipStream_t stream;
     std::vector<Zone*> zones;
     hipEvent_t e0, e1;
@@ -113,7 +113,7 @@ struct fm_ctx {
     hipEvent_t fork_ev;
     int lu_batch;            // batch the LU of several zones (default on)
     int lu_fp32;             // mixed precision: LU-SGS sweep arithmetic in FP32 (default off)
-    int res_kcol_n;          // tile shapes: k-column length of RES_KCOL (0: built-in)
+    int res_kcol_n;          // tile shapes: cells up k per residual workgroup (0: by the zone's size)
     int lu_flow_grid;        //   workgroups of a dataflow sweep (0: all that are resident)
     // time steps captured as HIP graphs (FM_OPT_GRAPH): one per distinct configuration
     // inside fm_compute: the streaming LU-SGS leaves dW in its skewed rows (copied back once at
@@ -565,14 +565,6 @@ static int ensure_exchange(fm_ctx* c, Zone* z) {
 
 // Dataflow LU schedule: the face exchange (sized for the largest LU box, interior plus a wall
 // layer per side) and the block order of the LU box b (rebuilt when the box changes).
-// The residual schedule of a zone: the context's, or with RES_AUTO six faces per cell on
-// Cartesian zones and columns up k on curvilinear ones (the faster of the two on each mesh kind,
-// measured on TGV 256^3 and the 257 x 129 x 33 channel)
-static int res_schedule_of(const fm_ctx* c, const Zone* z) {
-    if (c->res_schedule != RES_AUTO) return c->res_schedule;
-    return z->k.typ == 2 ? RES_CELLS : RES_KCOL;
-}
-
 // Streaming LU schedule of a zone: the pencil exchange, sized for the largest LU box and
 // filled with the pending pattern once (the sweeps leave it that way).
 static bool uses_stream(const fm_ctx* c, const Zone* z) {
@@ -769,7 +761,7 @@ static int substep(fm_ctx* c, Zone* z, int nitcfg, int first_it, int lssiter_ver
     if (k.kflu == 2 && nitcfg == 1) launch_wiggle(k, ro_ssiter, st);
     RhsArgs a;
     memset(&a, 0, sizeof a);
-    a.schedule = res_schedule_of(c, z);
+    a.schedule = c->res_schedule;
     a.kcol_n = c->res_kcol_n;
     if (k.kflu == 5) {
         int rc = wall_corrections(z, a);
@@ -1029,7 +1021,7 @@ extern "C" int fm_flux_balance(fm_ctx* c, int zone, int level, double* drodm) {
     launch_coe(k, rop, 0, 0, b, k.iflow == 2, st);
     if (k.kflu == 2) launch_wiggle(k, rop, st);
     RhsArgs a;
-    if (int rc = balance_args(z, rop, a, res_schedule_of(c, z))) return rc;
+    if (int rc = balance_args(z, rop, a, c->res_schedule)) return rc;
     a.kcol_n = c->res_kcol_n;
     z->dw_pending = 0;
     HIPCHK(hipMemsetAsync(k.drodm, 0, sizeof(double) * 5 * (size_t)k.nd, st));
@@ -1751,7 +1743,7 @@ extern "C" int fm_time_phase(fm_ctx* c, int zone, int phase, int reps, float* ms
     double* ro = z->ro[0];
     RhsArgs a;
     memset(&a, 0, sizeof a);
-    a.schedule = res_schedule_of(c, z);
+    a.schedule = c->res_schedule;
     a.kcol_n = c->res_kcol_n;
     if (k.kflu == 5) {
         int rc = wall_corrections(z, a);

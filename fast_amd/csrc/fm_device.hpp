@@ -47,6 +47,26 @@ __device__ __forceinline__ double dmax(double a, double b) { return a > b ? a : 
 __device__ __forceinline__ double dmin(double a, double b) { return a < b ? a : b; }
 __device__ __forceinline__ double dsign(double a, double b) { return copysign(fabs(a), b); }
 
+// the value lane L + DI holds (DPP wave shifts; the last lanes of the wave get their own value)
+template <int DI>
+__device__ __forceinline__ double from_lane(double v) {
+    static_assert(DI >= -1 && DI <= 1, "shift of a wave");
+    if (DI == 0) return v;
+    constexpr int ctl = DI > 0 ? 0x130 : 0x138;   // wave_shl:1 / wave_shr:1
+    const long long b = __double_as_longlong(v);
+    const int lo = __builtin_amdgcn_update_dpp((int)b, (int)b, ctl, 0xf, 0xf, false);
+    const int hi = __builtin_amdgcn_update_dpp((int)(b >> 32), (int)(b >> 32), ctl, 0xf, 0xf, false);
+    return __longlong_as_double(((long long)hi << 32) | (unsigned int)lo);
+}
+
+// A barrier that makes the LDS accesses of every wave before it visible after it.  Only LDS is ordered: a
+// __syncthreads() may also wait for the wave's global stores and loads in flight.
+__device__ __forceinline__ void lds_barrier() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
 // Constants of the flux template header (template_FluxAndBalance.for:100-190)
 struct FluxConst {
     double gam, rgp, gam1, gam3, psiroe, tmin_1, c1, c2, c3, opt0, c4, c5, c6, cvisq, wig_cte;
@@ -78,28 +98,49 @@ __device__ __forceinline__ FluxConst flux_const(const KZ& z) {
     return f;
 }
 
+// Where a face flux reads its stencil from: values of the cell (DI, DJ, DK) away from the flux's own
+// cell, and the face vectors and volumes at the same place of the metric grid.  MemCell reads all of
+// them from memory.
+struct MemCell {
+    const KZ& z;
+    const double* __restrict__ rop;
+    long l, lt;
+    __device__ __forceinline__ MemCell(const KZ& z_, const double* rop_, long l_, long lt_) : z(z_), rop(rop_), l(l_), lt(lt_) {}
+    template <int DI, int DJ, int DK> __device__ __forceinline__ long at() const { return l + DI + DJ * z.incj + DK * z.inck; }
+    template <int DI, int DJ, int DK> __device__ __forceinline__ double q(int e) const { return rop[at<DI, DJ, DK>() + e * z.nd]; }
+    template <int DI, int DJ, int DK> __device__ __forceinline__ double mu() const { return z.xmut[at<DI, DJ, DK>()]; }
+    __device__ __forceinline__ double wig(int d) const { return z.wig[l + d * z.nd]; }
+    template <int DI, int DJ, int DK> __device__ __forceinline__ double met(const double* __restrict__ t, int m) const {
+        return t[lt + DI * z.mi + DJ * z.mj + DK * z.mk + m * z.ndm];
+    }
+};
+
+// value e of the cell M places along direction D (M = 0: the cell itself)
+template <int D, int M, typename Cell>
+__device__ __forceinline__ double along(const Cell& c, int e) {
+    return c.template q<(D == 0 ? M : 0), (D == 1 ? M : 0), (D == 2 ? M : 0)>(e);
+}
+
 // MUSCL states (Slope/{o1,o3,minmod}_slope_var.for); qm right, qp left of face (l-inc, l)
-template <int SLOPE>
-__device__ __forceinline__ void slope_state(const FluxConst& f, const double* __restrict__ rop,
-                                            long nd, long l, long inc, double qm[5], double qp[5]) {
-    long nm = l - inc, nm2 = l - 2 * inc, np = l + inc;
+template <int SLOPE, int D, typename Cell>
+__device__ __forceinline__ void slope_state(const FluxConst& f, const Cell& cell, double qm[5], double qp[5]) {
     if (SLOPE == 1) {
 #pragma unroll
-        for (int e = 0; e < 5; e++) { qm[e] = rop[l + e * nd]; qp[e] = rop[nm + e * nd]; }
+        for (int e = 0; e < 5; e++) { qm[e] = along<D, 0>(cell, e); qp[e] = along<D, -1>(cell, e); }
     } else if (SLOPE == 2) {
 #pragma unroll
         for (int e = 0; e < 5; e++) {
-            const double* q = rop + e * nd;
-            double a = q[l], b = q[nm], c = q[np], d = q[nm2];
+            double a = along<D, 0>(cell, e), b = along<D, -1>(cell, e);
+            double c = along<D, 1>(cell, e), d = along<D, -2>(cell, e);
             qm[e] = f.c4 * a + f.c5 * b + f.c6 * c;
             qp[e] = f.c4 * b + f.c6 * d + f.c5 * a;
         }
     } else {
-        double roff = .5 * dmax(0., dmin(rop[l + 4 * nd] * f.tmin_1 - .5, 1.));
+        double roff = .5 * dmax(0., dmin(along<D, 0>(cell, 4) * f.tmin_1 - .5, 1.));
 #pragma unroll
         for (int e = 0; e < 5; e++) {
-            const double* q = rop + e * nd;
-            double a = q[l], b = q[nm], c = q[np], d = q[nm2];
+            double a = along<D, 0>(cell, e), b = along<D, -1>(cell, e);
+            double c = along<D, 1>(cell, e), d = along<D, -2>(cell, e);
             double delm = a - b, delp = c - a, delq = b - d;
             double sg = dsign(1., delm);
             double slp = roff * (sg * dmax(0., dmin(fabs(delm), sg * delp)));
@@ -113,11 +154,9 @@ __device__ __forceinline__ void slope_state(const FluxConst& f, const double* __
 
 // Inviscid face flux: Roe (etat_roe_GD.for + Vit_ent/fludiffer_*), AUSM+(P)
 // (AUSM/fluFaceEuler.for) and SENSEUR (SENSOR/fluFaceEuler.for), 3dcart or 3dfull.
-template <int KFLU, bool CART, int D>
-__device__ __forceinline__ void inviscid_flux(const FluxConst& f, const double* __restrict__ rop,
-                                              const double* __restrict__ wig, long nd, long l,
-                                              const double tn[3], double sn, const double qm[5],
-                                              const double qp[5], double flu[5]) {
+template <int KFLU, bool CART, int D, typename Cell>
+__device__ __forceinline__ void inviscid_flux(const FluxConst& f, const Cell& cell, const double tn[3], double sn,
+                                              const double qm[5], const double qp[5], double flu[5]) {
     if (KFLU == 5) {
         double gam = f.gam, rgp = f.rgp, gam1 = f.gam1, psiroe = f.psiroe;
         double r1 = qp[0];
@@ -213,14 +252,14 @@ __device__ __forceinline__ void inviscid_flux(const FluxConst& f, const double* 
         }
         double u, tdu;
         if (KFLU == 1) {
-            double c = rgp * f.gam * rop[l + 4 * nd];
+            double c = rgp * f.gam * cell.template q<0, 0, 0>(4);
             double son = sqrt(qn1 * qn1 / c);
             double tam = f.c3 * son + sn;
             double tam1 = dmax(0., tam) * f.c2;
             u = 0.25 * (qn1 + qn2) - tam1 * (p2 - p1);
             tdu = dmax(fabs(u), f.c1 * sn) * f.wig_cte;
         } else {
-            double wg = wig[l + D * nd];
+            double wg = cell.wig(D);
             u = 0.25 * (qn1 + qn2) - f.c2 * sn * (p2 - p1) * (f.opt0 * wg + 1. - f.opt0);
             tdu = dmax(fabs(u), f.c1 * sn) * wg;
         }
@@ -238,102 +277,89 @@ __device__ __forceinline__ void inviscid_flux(const FluxConst& f, const double* 
 }
 
 // Centred viscous flux on a Cartesian zone (fluvisq_3dcart_{i,j,k}.for)
-template <int D>
 // gv (optional): the face gradients (u, v, w, T) x (x, y, z) the flux was built from, and the
 // face's volinv in gv[12]; components this direction does not form stay as they were
-__device__ __forceinline__ void visc_cart(const FluxConst& f, const KZ& z, const double* __restrict__ rop,
-                                          const double* __restrict__ xmut, long l, double flu[5],
+template <int D, typename Cell>
+__device__ __forceinline__ void visc_cart(const FluxConst& f, const Cell& cell, double flu[5],
                                           double* gv = nullptr) {
-    long nd = z.nd, incj = z.incj, inck = z.inck;
-    const double* U = rop + nd; const double* V = rop + 2 * nd;
-    const double* W = rop + 3 * nd; const double* T = rop + 4 * nd;
     double tcx = f.tc[0], tcy = f.tc[1], tcz = f.tc[2];
     double xmutvol, xktvol, fv, fv5, f1, f2, f3, f4, f5, f6, div, fvs;
-    if (D == 0) {
-        long il = l - 1, ir = l;
-        long l220 = l - 1 - incj, l020 = l - incj, l210 = l - 1 + incj, l010 = l + incj;
-        long l202 = l - 1 - inck, l002 = l - inck, l201 = l - 1 + inck, l001 = l + inck;
+    if constexpr (D == 0) {
         double tix = tcx, tjy = .25 * tcy, tkz = .25 * tcz;
         double gUx, gUy, gUz, gVx, gVy, gWx, gWz, gTx;
-        f1 = U[il]; f2 = U[ir]; fvs = f1 + f2;
-        f3 = fvs + U[l220] + U[l020]; f4 = fvs + U[l210] + U[l010];
-        f5 = fvs + U[l202] + U[l002]; f6 = fvs + U[l201] + U[l001];
+        f1 = cell.template q<-1, 0, 0>(1); f2 = cell.template q<0, 0, 0>(1); fvs = f1 + f2;
+        f3 = fvs + cell.template q<-1, -1, 0>(1) + cell.template q<0, -1, 0>(1); f4 = fvs + cell.template q<-1, 1, 0>(1) + cell.template q<0, 1, 0>(1);
+        f5 = fvs + cell.template q<-1, 0, -1>(1) + cell.template q<0, 0, -1>(1); f6 = fvs + cell.template q<-1, 0, 1>(1) + cell.template q<0, 0, 1>(1);
         gUx = (f2 - f1) * tix; gUy = (f4 - f3) * tjy; gUz = (f6 - f5) * tkz;
-        f1 = V[il]; f2 = V[ir]; fvs = f1 + f2;
-        f3 = fvs + V[l220] + V[l020]; f4 = fvs + V[l210] + V[l010];
+        f1 = cell.template q<-1, 0, 0>(2); f2 = cell.template q<0, 0, 0>(2); fvs = f1 + f2;
+        f3 = fvs + cell.template q<-1, -1, 0>(2) + cell.template q<0, -1, 0>(2); f4 = fvs + cell.template q<-1, 1, 0>(2) + cell.template q<0, 1, 0>(2);
         gVx = (f2 - f1) * tix; gVy = (f4 - f3) * tjy;
-        f1 = W[il]; f2 = W[ir]; fvs = f1 + f2;
-        f5 = fvs + W[l202] + W[l002]; f6 = fvs + W[l201] + W[l001];
+        f1 = cell.template q<-1, 0, 0>(3); f2 = cell.template q<0, 0, 0>(3); fvs = f1 + f2;
+        f5 = fvs + cell.template q<-1, 0, -1>(3) + cell.template q<0, 0, -1>(3); f6 = fvs + cell.template q<-1, 0, 1>(3) + cell.template q<0, 0, 1>(3);
         gWx = (f2 - f1) * tix; gWz = (f6 - f5) * tkz;
-        f1 = T[il]; f2 = T[ir];
+        f1 = cell.template q<-1, 0, 0>(4); f2 = cell.template q<0, 0, 0>(4);
         gTx = (f2 - f1) * tix;
         div = (gUx + gVy + gWz) * f.cvisq;
         f1 = gUx - div; f2 = gUy + gVx; f3 = gUz + gWx;
-        xmutvol = (xmut[ir] + xmut[il]) * f.volinv;
+        xmutvol = (cell.template mu<0, 0, 0>() + cell.template mu<-1, 0, 0>()) * f.volinv;
         xktvol = xmutvol * f.gam3;
-        fv = -(2. * f1 * tcx) * xmutvol; fv5 = fv * (U[ir] + U[il]); flu[1] = flu[1] + fv;
-        fv = -(f2 * tcx) * xmutvol; fv5 = fv5 + fv * (V[ir] + V[il]); flu[2] = flu[2] + fv;
-        fv = -(f3 * tcx) * xmutvol; fv5 = fv5 + fv * (W[ir] + W[il]); flu[3] = flu[3] + fv;
+        fv = -(2. * f1 * tcx) * xmutvol; fv5 = fv * (cell.template q<0, 0, 0>(1) + cell.template q<-1, 0, 0>(1)); flu[1] = flu[1] + fv;
+        fv = -(f2 * tcx) * xmutvol; fv5 = fv5 + fv * (cell.template q<0, 0, 0>(2) + cell.template q<-1, 0, 0>(2)); flu[2] = flu[2] + fv;
+        fv = -(f3 * tcx) * xmutvol; fv5 = fv5 + fv * (cell.template q<0, 0, 0>(3) + cell.template q<-1, 0, 0>(3)); flu[3] = flu[3] + fv;
         fv = fv5 * 0.5 - (gTx * tcx) * xktvol; flu[4] = flu[4] + fv;
         if (gv) {
             gv[0] = gUx; gv[1] = gUy; gv[2] = gUz; gv[3] = gVx; gv[4] = gVy;
             gv[6] = gWx; gv[8] = gWz; gv[9] = gTx;
         }
-    } else if (D == 1) {
-        long il = l - incj, ir = l;
-        long l022 = l - incj - inck, l002 = l - inck, l021 = l - incj + inck, l001 = l + inck;
-        long l220 = l - 1 - incj, l200 = l - 1, l120 = l + 1 - incj, l100 = l + 1;
+    } else if constexpr (D == 1) {
         double tiy = tcy, tjz = .25 * tcz, tkx = .25 * tcx;
         double gUx, gUy, gVx, gVy, gVz, gWy, gWz, gTy;
-        f1 = U[il]; f2 = U[ir]; fvs = f1 + f2;
-        f5 = fvs + U[l220] + U[l200]; f6 = fvs + U[l120] + U[l100];
+        f1 = cell.template q<0, -1, 0>(1); f2 = cell.template q<0, 0, 0>(1); fvs = f1 + f2;
+        f5 = fvs + cell.template q<-1, -1, 0>(1) + cell.template q<-1, 0, 0>(1); f6 = fvs + cell.template q<1, -1, 0>(1) + cell.template q<1, 0, 0>(1);
         gUx = (f6 - f5) * tkx; gUy = (f2 - f1) * tiy;
-        f1 = V[il]; f2 = V[ir]; fvs = f1 + f2;
-        f3 = fvs + V[l022] + V[l002]; f4 = fvs + V[l021] + V[l001];
-        f5 = fvs + V[l220] + V[l200]; f6 = fvs + V[l120] + V[l100];
+        f1 = cell.template q<0, -1, 0>(2); f2 = cell.template q<0, 0, 0>(2); fvs = f1 + f2;
+        f3 = fvs + cell.template q<0, -1, -1>(2) + cell.template q<0, 0, -1>(2); f4 = fvs + cell.template q<0, -1, 1>(2) + cell.template q<0, 0, 1>(2);
+        f5 = fvs + cell.template q<-1, -1, 0>(2) + cell.template q<-1, 0, 0>(2); f6 = fvs + cell.template q<1, -1, 0>(2) + cell.template q<1, 0, 0>(2);
         gVx = (f6 - f5) * tkx; gVy = (f2 - f1) * tiy; gVz = (f4 - f3) * tjz;
-        f1 = W[il]; f2 = W[ir]; fvs = f1 + f2;
-        f3 = fvs + W[l022] + W[l002]; f4 = fvs + W[l021] + W[l001];
+        f1 = cell.template q<0, -1, 0>(3); f2 = cell.template q<0, 0, 0>(3); fvs = f1 + f2;
+        f3 = fvs + cell.template q<0, -1, -1>(3) + cell.template q<0, 0, -1>(3); f4 = fvs + cell.template q<0, -1, 1>(3) + cell.template q<0, 0, 1>(3);
         gWy = (f2 - f1) * tiy; gWz = (f4 - f3) * tjz;
-        f1 = T[il]; f2 = T[ir];
+        f1 = cell.template q<0, -1, 0>(4); f2 = cell.template q<0, 0, 0>(4);
         gTy = (f2 - f1) * tiy;
         div = (gUx + gVy + gWz) * f.cvisq;
         f2 = gUy + gVx; f4 = gVy - div; f5 = gVz + gWy;
-        xmutvol = (xmut[ir] + xmut[il]) * f.volinv;
+        xmutvol = (cell.template mu<0, 0, 0>() + cell.template mu<0, -1, 0>()) * f.volinv;
         xktvol = xmutvol * f.gam3;
-        fv = -(f2 * tcy) * xmutvol; fv5 = fv * (U[ir] + U[il]); flu[1] = flu[1] + fv;
-        fv = -(2. * f4 * tcy) * xmutvol; fv5 = fv5 + fv * (V[ir] + V[il]); flu[2] = flu[2] + fv;
-        fv = -(f5 * tcy) * xmutvol; fv5 = fv5 + fv * (W[ir] + W[il]); flu[3] = flu[3] + fv;
+        fv = -(f2 * tcy) * xmutvol; fv5 = fv * (cell.template q<0, 0, 0>(1) + cell.template q<0, -1, 0>(1)); flu[1] = flu[1] + fv;
+        fv = -(2. * f4 * tcy) * xmutvol; fv5 = fv5 + fv * (cell.template q<0, 0, 0>(2) + cell.template q<0, -1, 0>(2)); flu[2] = flu[2] + fv;
+        fv = -(f5 * tcy) * xmutvol; fv5 = fv5 + fv * (cell.template q<0, 0, 0>(3) + cell.template q<0, -1, 0>(3)); flu[3] = flu[3] + fv;
         fv = fv5 * 0.5 - (gTy * tcy) * xktvol; flu[4] = flu[4] + fv;
         if (gv) {
             gv[0] = gUx; gv[1] = gUy; gv[3] = gVx; gv[4] = gVy; gv[5] = gVz;
             gv[7] = gWy; gv[8] = gWz; gv[10] = gTy;
         }
     } else {
-        long il = l - inck, ir = l;
-        long l200 = l - 1, l202 = l - 1 - inck, l102 = l + 1 - inck, l100 = l + 1;
-        long l022 = l - incj - inck, l020 = l - incj, l012 = l + incj - inck, l010 = l + incj;
         double tiz = tcz, tky = .25 * tcy, tjx = .25 * tcx;
         double gUx, gUz, gVy, gVz, gWx, gWy, gWz, gTz;
-        f1 = U[il]; f2 = U[ir]; fvs = f1 + f2;
-        f3 = fvs + U[l202] + U[l200]; f4 = fvs + U[l102] + U[l100];
+        f1 = cell.template q<0, 0, -1>(1); f2 = cell.template q<0, 0, 0>(1); fvs = f1 + f2;
+        f3 = fvs + cell.template q<-1, 0, -1>(1) + cell.template q<-1, 0, 0>(1); f4 = fvs + cell.template q<1, 0, -1>(1) + cell.template q<1, 0, 0>(1);
         gUx = (f4 - f3) * tjx; gUz = (f2 - f1) * tiz;
-        f1 = V[il]; f2 = V[ir]; fvs = f1 + f2;
-        f5 = fvs + V[l022] + V[l020]; f6 = fvs + V[l012] + V[l010];
+        f1 = cell.template q<0, 0, -1>(2); f2 = cell.template q<0, 0, 0>(2); fvs = f1 + f2;
+        f5 = fvs + cell.template q<0, -1, -1>(2) + cell.template q<0, -1, 0>(2); f6 = fvs + cell.template q<0, 1, -1>(2) + cell.template q<0, 1, 0>(2);
         gVy = (f6 - f5) * tky; gVz = (f2 - f1) * tiz;
-        f1 = W[il]; f2 = W[ir]; fvs = f1 + f2;
-        f3 = fvs + W[l202] + W[l200]; f4 = fvs + W[l102] + W[l100];
-        f5 = fvs + W[l022] + W[l020]; f6 = fvs + W[l012] + W[l010];
+        f1 = cell.template q<0, 0, -1>(3); f2 = cell.template q<0, 0, 0>(3); fvs = f1 + f2;
+        f3 = fvs + cell.template q<-1, 0, -1>(3) + cell.template q<-1, 0, 0>(3); f4 = fvs + cell.template q<1, 0, -1>(3) + cell.template q<1, 0, 0>(3);
+        f5 = fvs + cell.template q<0, -1, -1>(3) + cell.template q<0, -1, 0>(3); f6 = fvs + cell.template q<0, 1, -1>(3) + cell.template q<0, 1, 0>(3);
         gWx = (f4 - f3) * tjx; gWy = (f6 - f5) * tky; gWz = (f2 - f1) * tiz;
-        f1 = T[il]; f2 = T[ir];
+        f1 = cell.template q<0, 0, -1>(4); f2 = cell.template q<0, 0, 0>(4);
         gTz = (f2 - f1) * tiz;
         div = (gUx + gVy + gWz) * f.cvisq;
         f3 = gUz + gWx; f5 = gVz + gWy; f6 = gWz - div;
-        xmutvol = (xmut[ir] + xmut[il]) * f.volinv;
+        xmutvol = (cell.template mu<0, 0, 0>() + cell.template mu<0, 0, -1>()) * f.volinv;
         xktvol = xmutvol * f.gam3;
-        fv = -f3 * tcz * xmutvol; fv5 = fv * (U[ir] + U[il]); flu[1] = flu[1] + fv;
-        fv = -f5 * tcz * xmutvol; fv5 = fv5 + fv * (V[ir] + V[il]); flu[2] = flu[2] + fv;
-        fv = -2. * f6 * tcz * xmutvol; fv5 = fv5 + fv * (W[ir] + W[il]); flu[3] = flu[3] + fv;
+        fv = -f3 * tcz * xmutvol; fv5 = fv * (cell.template q<0, 0, 0>(1) + cell.template q<0, 0, -1>(1)); flu[1] = flu[1] + fv;
+        fv = -f5 * tcz * xmutvol; fv5 = fv5 + fv * (cell.template q<0, 0, 0>(2) + cell.template q<0, 0, -1>(2)); flu[2] = flu[2] + fv;
+        fv = -2. * f6 * tcz * xmutvol; fv5 = fv5 + fv * (cell.template q<0, 0, 0>(3) + cell.template q<0, 0, -1>(3)); flu[3] = flu[3] + fv;
         fv = fv5 * 0.5 - gTz * tcz * xktvol; flu[4] = flu[4] + fv;
         if (gv) {
             gv[0] = gUx; gv[2] = gUz; gv[4] = gVy; gv[5] = gVz;
@@ -344,70 +370,86 @@ __device__ __forceinline__ void visc_cart(const FluxConst& f, const KZ& z, const
 }
 
 // Centred viscous flux on a curvilinear zone (fluvisq_3dfull_{i,j,k}.for)
-template <int D>
-__device__ __forceinline__ void visc_full(const FluxConst& f, const KZ& z, const double* __restrict__ rop,
-                                          const double* __restrict__ xmut, long l, long lt,
-                                          const double tn[3], double flu[5], double* gv = nullptr) {
-    long nd = z.nd, ndm = z.ndm, incj = z.incj, inck = z.inck, mi = z.mi, mj = z.mj, mk = z.mk;
-    const double* A; const double* B; const double* C;
-    long il, lvol, a0, a1, b0, b1, b2, b3, c0, c1, c2, c3, n3a, n3b, n4a, n4b, n5a, n5b, n6a, n6b;
-    if (D == 0) {
-        A = z.ti; B = z.tj; C = z.tk; il = l - 1; lvol = lt - mi;
-        a0 = lt - mi; a1 = lt + mi; b0 = lt; b1 = lt - mi; b2 = lt + mj; b3 = lt - mi + mj;
-        c0 = lt; c1 = lt - mi; c2 = lt + mk; c3 = lt - mi + mk;
-        n3a = l - 1 - incj; n3b = l - incj; n4a = l - 1 + incj; n4b = l + incj;
-        n5a = l - 1 - inck; n5b = l - inck; n6a = l - 1 + inck; n6b = l + inck;
-    } else if (D == 1) {
-        A = z.tj; B = z.tk; C = z.ti; il = l - incj; lvol = lt - mj;
-        a0 = lt - mj; a1 = lt + mj; b0 = lt; b1 = lt - mj; b2 = lt + mk; b3 = lt - mj + mk;
-        c0 = lt; c1 = lt - mj; c2 = lt + mi; c3 = lt + mi - mj;
-        n3a = l - incj - inck; n3b = l - inck; n4a = l - incj + inck; n4b = l + inck;
-        n5a = l - 1 - incj; n5b = l - 1; n6a = l + 1 - incj; n6b = l + 1;
-    } else {
-        A = z.tk; B = z.ti; C = z.tj; il = l - inck; lvol = lt - mk;
-        a0 = lt - mk; a1 = lt + mk; b0 = lt; b1 = lt - mk; b2 = lt + mi; b3 = lt + mi - mk;
-        c0 = lt; c1 = lt - mk; c2 = lt + mj; c3 = lt + mj - mk;
-        n3a = l - 1 - inck; n3b = l - 1; n4a = l + 1 - inck; n4b = l + 1;
-        n5a = l - incj - inck; n5b = l - incj; n6a = l + incj - inck; n6b = l + incj;
-    }
-    long ir = l;
+template <int D, typename Cell>
+__device__ __forceinline__ void visc_full(const FluxConst& f, const KZ& z, const Cell& cell, const double tn[3],
+                                          double flu[5], double* gv = nullptr) {
+    // (D, then the two directions after it) the face vectors of the cells on both sides, and the
+    // neighbours of the two cells in those directions
     double t0[3], t1[3], u0[3], u1[3], w0[3], w1[3];
 #pragma unroll
     for (int m = 0; m < 3; m++) {
-        t0[m] = .5 * (A[lt + m * ndm] + A[a0 + m * ndm]);
-        t1[m] = .5 * (A[lt + m * ndm] + A[a1 + m * ndm]);
-        u0[m] = .125 * (B[b0 + m * ndm] + B[b1 + m * ndm]);
-        u1[m] = .125 * (B[b2 + m * ndm] + B[b3 + m * ndm]);
-        w0[m] = .125 * (C[c0 + m * ndm] + C[c1 + m * ndm]);
-        w1[m] = .125 * (C[c2 + m * ndm] + C[c3 + m * ndm]);
+        const double* ti = z.ti; const double* tj = z.tj; const double* tk = z.tk;
+        if constexpr (D == 0) {
+            const double a = cell.template met<0, 0, 0>(ti, m);
+            t0[m] = .5 * (a + cell.template met<-1, 0, 0>(ti, m));
+            t1[m] = .5 * (a + cell.template met<1, 0, 0>(ti, m));
+            u0[m] = .125 * (cell.template met<0, 0, 0>(tj, m) + cell.template met<-1, 0, 0>(tj, m));
+            u1[m] = .125 * (cell.template met<0, 1, 0>(tj, m) + cell.template met<-1, 1, 0>(tj, m));
+            w0[m] = .125 * (cell.template met<0, 0, 0>(tk, m) + cell.template met<-1, 0, 0>(tk, m));
+            w1[m] = .125 * (cell.template met<0, 0, 1>(tk, m) + cell.template met<-1, 0, 1>(tk, m));
+        } else if constexpr (D == 1) {
+            const double a = cell.template met<0, 0, 0>(tj, m);
+            t0[m] = .5 * (a + cell.template met<0, -1, 0>(tj, m));
+            t1[m] = .5 * (a + cell.template met<0, 1, 0>(tj, m));
+            u0[m] = .125 * (cell.template met<0, 0, 0>(tk, m) + cell.template met<0, -1, 0>(tk, m));
+            u1[m] = .125 * (cell.template met<0, 0, 1>(tk, m) + cell.template met<0, -1, 1>(tk, m));
+            w0[m] = .125 * (cell.template met<0, 0, 0>(ti, m) + cell.template met<0, -1, 0>(ti, m));
+            w1[m] = .125 * (cell.template met<1, 0, 0>(ti, m) + cell.template met<1, -1, 0>(ti, m));
+        } else {
+            const double a = cell.template met<0, 0, 0>(tk, m);
+            t0[m] = .5 * (a + cell.template met<0, 0, -1>(tk, m));
+            t1[m] = .5 * (a + cell.template met<0, 0, 1>(tk, m));
+            u0[m] = .125 * (cell.template met<0, 0, 0>(ti, m) + cell.template met<0, 0, -1>(ti, m));
+            u1[m] = .125 * (cell.template met<1, 0, 0>(ti, m) + cell.template met<1, 0, -1>(ti, m));
+            w0[m] = .125 * (cell.template met<0, 0, 0>(tj, m) + cell.template met<0, 0, -1>(tj, m));
+            w1[m] = .125 * (cell.template met<0, 1, 0>(tj, m) + cell.template met<0, 1, -1>(tj, m));
+        }
     }
-    double g[4][3];
+    // (the 33 face vectors are read and averaged before any state, which keeps both out of scratch)
+    __builtin_amdgcn_sched_barrier(0);
+    double ql[5], qr[5], g[4][3];
 #pragma unroll
-    for (int e = 0; e < 4; e++) {
-        const double* q = rop + (e + 1) * nd;
-        double f1 = q[il], f2 = q[ir];
-        double f3 = q[ir] + q[il] + q[n3a] + q[n3b];
-        double f4 = q[ir] + q[il] + q[n4a] + q[n4b];
-        double f5 = q[ir] + q[il] + q[n5a] + q[n5b];
-        double f6 = q[ir] + q[il] + q[n6a] + q[n6b];
+    for (int e = 1; e < 5; e++) {
+        const double f1 = ql[e] = along<D, -1>(cell, e), f2 = qr[e] = along<D, 0>(cell, e);
+        double n3a, n3b, n4a, n4b, n5a, n5b, n6a, n6b;
+        if constexpr (D == 0) {
+            n3a = cell.template q<-1, -1, 0>(e); n3b = cell.template q<0, -1, 0>(e);
+            n4a = cell.template q<-1, 1, 0>(e); n4b = cell.template q<0, 1, 0>(e);
+            n5a = cell.template q<-1, 0, -1>(e); n5b = cell.template q<0, 0, -1>(e);
+            n6a = cell.template q<-1, 0, 1>(e); n6b = cell.template q<0, 0, 1>(e);
+        } else if constexpr (D == 1) {
+            n3a = cell.template q<0, -1, -1>(e); n3b = cell.template q<0, 0, -1>(e);
+            n4a = cell.template q<0, -1, 1>(e); n4b = cell.template q<0, 0, 1>(e);
+            n5a = cell.template q<-1, -1, 0>(e); n5b = cell.template q<-1, 0, 0>(e);
+            n6a = cell.template q<1, -1, 0>(e); n6b = cell.template q<1, 0, 0>(e);
+        } else {
+            n3a = cell.template q<-1, 0, -1>(e); n3b = cell.template q<-1, 0, 0>(e);
+            n4a = cell.template q<1, 0, -1>(e); n4b = cell.template q<1, 0, 0>(e);
+            n5a = cell.template q<0, -1, -1>(e); n5b = cell.template q<0, -1, 0>(e);
+            n6a = cell.template q<0, 1, -1>(e); n6b = cell.template q<0, 1, 0>(e);
+        }
+        double f3 = f2 + f1 + n3a + n3b;
+        double f4 = f2 + f1 + n4a + n4b;
+        double f5 = f2 + f1 + n5a + n5b;
+        double f6 = f2 + f1 + n6a + n6b;
 #pragma unroll
         for (int m = 0; m < 3; m++)
-            g[e][m] = (f2 * t1[m] - f1 * t0[m]) + (f4 * u1[m] - f3 * u0[m]) + (f6 * w1[m] - f5 * w0[m]);
+            g[e - 1][m] = (f2 * t1[m] - f1 * t0[m]) + (f4 * u1[m] - f3 * u0[m]) + (f6 * w1[m] - f5 * w0[m]);
     }
+    constexpr int IL = D == 0 ? -1 : 0, JL = D == 1 ? -1 : 0, KL = D == 2 ? -1 : 0;
     double div = (g[0][0] + g[1][1] + g[2][2]) * f.cvisq;
     double f1 = g[0][0] - div, f2 = g[0][1] + g[1][0], f3 = g[0][2] + g[2][0];
     double f4 = g[1][1] - div, f5 = g[1][2] + g[2][1], f6 = g[2][2] - div;
-    double volinv = 1. / (z.vol[lt] + z.vol[lvol]);
-    double xmutvol = (xmut[ir] + xmut[il]) * volinv;
+    double volinv = 1. / (cell.template met<0, 0, 0>(z.vol, 0) + cell.template met<IL, JL, KL>(z.vol, 0));
+    double xmutvol = (cell.template mu<0, 0, 0>() + cell.template mu<IL, JL, KL>()) * volinv;
     double xktvol = xmutvol * f.gam3;
-    const double* U = rop + nd; const double* V = rop + 2 * nd; const double* W = rop + 3 * nd;
     double tcx = tn[0], tcy = tn[1], tcz = tn[2], fv, fv5;
     fv = -(2. * f1 * tcx + f2 * tcy + f3 * tcz) * xmutvol;
-    fv5 = fv * (U[ir] + U[il]); flu[1] = flu[1] + fv;
+    fv5 = fv * (qr[1] + ql[1]); flu[1] = flu[1] + fv;
     fv = -(f2 * tcx + 2. * f4 * tcy + f5 * tcz) * xmutvol;
-    fv5 = fv5 + fv * (V[ir] + V[il]); flu[2] = flu[2] + fv;
+    fv5 = fv5 + fv * (qr[2] + ql[2]); flu[2] = flu[2] + fv;
     fv = -(f3 * tcx + f5 * tcy + 2. * f6 * tcz) * xmutvol;
-    fv5 = fv5 + fv * (W[ir] + W[il]); flu[3] = flu[3] + fv;
+    fv5 = fv5 + fv * (qr[3] + ql[3]); flu[3] = flu[3] + fv;
     fv = fv5 * 0.5 - (g[3][0] * tcx + g[3][1] * tcy + g[3][2] * tcz) * xktvol;
     flu[4] = flu[4] + fv;
     if (gv) {
@@ -419,28 +461,30 @@ __device__ __forceinline__ void visc_full(const FluxConst& f, const KZ& z, const
     }
 }
 
-// Full face flux through the face (l - inc_D, l) of cell (i,j,k)
-template <int KFLU, int SLOPE, bool LAMIN, bool CART, int D>
-__device__ __forceinline__ void face_flux(const FluxConst& f, const KZ& z, const double* __restrict__ rop,
-                                          int i, int j, int k, double flu[5]) {
-    long l = IDX(z, i, j, k);
-    long inc = D == 0 ? 1 : D == 1 ? z.incj : z.inck;
+// Full face flux through the face (l - inc_D, l) of a cell
+template <int KFLU, int SLOPE, bool LAMIN, bool CART, int D, typename Cell>
+__device__ __forceinline__ void face_flux_at(const FluxConst& f, const KZ& z, const Cell& cell, double flu[5]) {
     double qm[5], qp[5], tn[3], sn;
-    long lt = 0;
     if (CART) {
         tn[0] = f.tc[0]; tn[1] = f.tc[1]; tn[2] = f.tc[2]; sn = f.s[D];
     } else {
         const double* t = D == 0 ? z.ti : D == 1 ? z.tj : z.tk;
-        lt = MTR(z, i, j, k);
-        tn[0] = t[lt]; tn[1] = t[lt + z.ndm]; tn[2] = t[lt + 2 * z.ndm];
+#pragma unroll
+        for (int m = 0; m < 3; m++) tn[m] = cell.template met<0, 0, 0>(t, m);
         sn = sqrt(tn[0] * tn[0] + tn[1] * tn[1] + tn[2] * tn[2]);
     }
-    slope_state<SLOPE>(f, rop, z.nd, l, inc, qm, qp);
-    inviscid_flux<KFLU, CART, D>(f, rop, z.wig, z.nd, l, tn, sn, qm, qp, flu);
+    slope_state<SLOPE, D>(f, cell, qm, qp);
+    inviscid_flux<KFLU, CART, D>(f, cell, tn, sn, qm, qp, flu);
     if (LAMIN) {
-        if (CART) visc_cart<D>(f, z, rop, z.xmut, l, flu);
-        else visc_full<D>(f, z, rop, z.xmut, l, lt, tn, flu);
+        if (CART) visc_cart<D>(f, cell, flu);
+        else visc_full<D>(f, z, cell, tn, flu);
     }
+}
+// the same of cell (i, j, k), read from memory
+template <int KFLU, int SLOPE, bool LAMIN, bool CART, int D>
+__device__ __forceinline__ void face_flux(const FluxConst& f, const KZ& z, const double* __restrict__ rop,
+                                          int i, int j, int k, double flu[5]) {
+    face_flux_at<KFLU, SLOPE, LAMIN, CART, D>(f, z, MemCell(z, rop, IDX(z, i, j, k), CART ? 0 : MTR(z, i, j, k)), flu);
 }
 
 }  // namespace fm

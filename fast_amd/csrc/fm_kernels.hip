@@ -400,25 +400,128 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(FM_RES
     res_update(z, a, rop, l, acc);
 }
 
-// Residual, a column of a.kcol_n cells up k per thread: the k face between two cells of the
-// column is evaluated once (as the top face of the lower cell and the bottom face of the upper
-// one), and the planes the k stencils share stay in the cache of the block.  Per cell the sum
-// order is the reference's, so the result is the one of k_residual.
+// Residual from planes in LDS.  The lanes of a wave hold consecutive cells of a row, two ghosts at each
+// end included, so a value at i +- 1 or 2 is in the place of lane +- 1 or 2 and the flux of face i + 1 is
+// lane + 1's.  A workgroup is kPlaneRows waves on as many consecutive rows j.  A wave's lanes run over
+// the rows of its number of every group of kPlaneRows rows one after another (x = group (ni + 4) + i),
+// 60 of 64 lanes with a cell of their own: the lanes lost are the ghosts and 4 a wave whatever ni is.
+// The workgroup walks kcol cells up k with the planes k - 1, k and k + 1 of its rows and of the two rows on
+// each side in LDS and plane k + 2 on its way in registers; a thread keeps the k face between two of
+// its cells.  Per cell: four faces, summed in the reference order.
+//
+// Why: a 64-lane load of 8 bytes takes the CU's vector memory path 16 cycles whether or not it hits, an
+// LDS read 4.  k_residual's 153 loads a cell kept that path busy for 79 % of its time (256^3, AUSM+(P)
+// laminar; vector units 42 %), and on curvilinear zones, with ~380, the registers it held them in spilled.
+// Here a cell costs 12 loads for the planes and 22 for its own update, and four face fluxes instead of six
+// (five for columns of cells).  us before (six faces on 3dcart, columns on 3dfull) and now, laminar:
+// AUSM+(P) 256^3 1778 -> 1143, 161 x 97 x 75 136 -> 80, 64^3 28 -> 29; SENSEUR 161 x 97 x 75 155 -> 78;
+// Roe o3 128^3 493 -> 230, minmod 667 -> 250; curvilinear AUSM+(P) 257 x 129 x 33 436 -> 242,
+// 513 x 257 x 65 3006 -> 1875, 80 x 50 x 20 98 -> 34, Roe 257 x 129 x 33 695 -> 275; Euler 192 x 180 x 168
+// 445 -> 340.  What bounds it now: instruction issue, at two waves a SIMD.
+constexpr int kPlaneRows = 4, kPlaneCells = 60, kPlaneTile = kPlaneRows + 4;
+constexpr int kPlaneSlots = 512;      // workgroups at work at once (two of 74 KB of LDS on each of 256 CUs)
+
+// what a face flux at (0, DJ0, DK0) from the thread's cell reads: state and viscosity from the planes
+// (two cells up k: the thread's own values on their way), the metric from memory at the lane's own i and
+// from the neighbouring lanes at i +- 1
+template <int DJ0, int DK0>
+struct PlaneCell {
+    const KZ& z;
+    const double* m1; const double* p0; const double* p1;     // planes k - 1, k, k + 1 at the thread's cell
+    const double* up;                                         // plane k + 2, the thread's cell
+    long l, lt;
+    template <int DI, int DJ, int DK> __device__ __forceinline__ double get(int e) const {
+        constexpr int K = DK0 + DK;
+        static_assert(K >= -1 && (K <= 1 || (K == 2 && DI == 0 && DJ0 + DJ == 0)), "outside the planes held");
+        if (K == 2) return up[e];
+        return (K < 0 ? m1 : K > 0 ? p1 : p0)[(e * kPlaneTile + DJ0 + DJ) * 64 + DI];
+    }
+    template <int DI, int DJ, int DK> __device__ __forceinline__ double q(int e) const { return get<DI, DJ, DK>(e); }
+    template <int DI, int DJ, int DK> __device__ __forceinline__ double mu() const { return get<DI, DJ, DK>(5); }
+    __device__ __forceinline__ double wig(int d) const { return z.wig[l + DJ0 * z.incj + DK0 * z.inck + d * z.nd]; }
+    template <int DI, int DJ, int DK> __device__ __forceinline__ double met(const double* __restrict__ t, int m) const {
+        return from_lane<DI>(t[lt + (DJ0 + DJ) * z.mj + (DK0 + DK) * z.mk + m * z.ndm]);
+    }
+};
+
+// the metric index of another face: hides from the compiler that it equals the last face's, so that the
+// face vectors two faces share are read again (from the caches) rather than held in registers
+template <bool CART>
+__device__ __forceinline__ long apart(long lt) {
+    if (!CART) asm volatile("" : "+v"(lt));
+    return lt;
+}
+
 template <int KFLU, int SLOPE, bool LAMIN, bool CART>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(FM_RES_WAVES))) k_residual_kcol(KZ z, RhsArgs a) {
-    int i = blockIdx.x * blockDim.x + threadIdx.x + 1;
-    int j = blockIdx.y * blockDim.y + threadIdx.y + 1;
-    const int kn_col = a.kcol_n > 0 ? a.kcol_n : RES_KCOL_N;
-    int k0 = blockIdx.z * kn_col + 1;
-    if (i > z.ni || j > z.nj || k0 > z.nk) return;
+__global__ void __launch_bounds__(64 * kPlaneRows) __attribute__((amdgpu_waves_per_eu(2))) k_residual_planes(KZ z, RhsArgs a, int kcol) {
+    constexpr int NA = LAMIN ? 6 : 5, PLANE = NA * kPlaneTile * 64;
+    __shared__ double P[3 * PLANE + 4];              // (the first and last lanes read two places out)
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    const int nx = (z.nj + kPlaneRows - 1) / kPlaneRows * z.nit;
+    int bx = blockIdx.x, by = blockIdx.y;
+    if (CART) {
+        // consecutive workgroups go to the eight XCDs in turn; this gives XCD c the c-th of eight
+        // near-equal ranges of workgroups, so that the rows two neighbours share are in its L2 (256^3
+        // 1152 -> 1143 us, 161 x 97 x 75 108 -> 103; curvilinear zones, whose metric fills it, lose:
+        // 513 x 257 x 65 1819 -> 2062)
+        const int n = gridDim.x * gridDim.y, id = bx + gridDim.x * by, c = id % 8, per = n / 8, rem = n % 8;
+        const int q = c * per + (c < rem ? c : rem) + id / 8;
+        by = q / gridDim.x; bx = q % gridDim.x;
+    }
+    const int x0 = bx * kPlaneCells + lane - 2, x = x0 < 0 ? 0 : x0 < nx ? x0 : nx - 1;
+    const int g = x / z.nit, i = x - g * z.nit - 1, j0 = g * kPlaneRows + w + 1, j = j0 < z.nj ? j0 : z.nj;
+    const bool own = lane >= 2 && lane < 2 + kPlaneCells && x0 < nx && i >= 1 && i <= z.ni && j0 <= z.nj;
+    const int k0 = by * kcol + 1, k1 = k0 + kcol - 1 < z.nk ? k0 + kcol - 1 : z.nk;
     const double* __restrict__ rop = a.rop;
-    long nd = z.nd;
-    FluxConst f = flux_const(z);
-    double fk[5], flu[5], acc[5];
-    face_flux<KFLU, SLOPE, LAMIN, CART, 2>(f, z, rop, i, j, k0, fk);
-    const int k1 = k0 + kn_col - 1 < z.nk ? k0 + kn_col - 1 : z.nk;
+    const long nd = z.nd;
+    const FluxConst f = flux_const(z);
+    const bool jn = cb_next(j, z.cbj, z.nbj);
+    // the two rows this wave brings in: its own (row w + 2 of the tile) and one of the four around
+    const int hr = w < 2 ? w : w + 4;
+    auto row_j = [&](int r) { const int jr = g * kPlaneRows - 1 + r; return jr < z.nj + 2 ? jr : z.nj + 2; };
+    long lo = IDX(z, i, row_j(w + 2), k0 - 2), lh = IDX(z, i, row_j(hr), k0 - 2);
+    double vo[NA], vh[NA];
+    auto fetch = [&]() {
+#pragma unroll
+        for (int e = 0; e < NA; e++) {
+            const double* __restrict__ q = e < 5 ? rop + e * nd : z.xmut;
+            vo[e] = q[lo]; vh[e] = q[lh];
+        }
+        lo += z.inck; lh += z.inck;
+    };
+    auto keep = [&](double* p) {
+#pragma unroll
+        for (int e = 0; e < NA; e++) {
+            p[2 + (e * kPlaneTile + w + 2) * 64 + lane] = vo[e];
+            p[2 + (e * kPlaneTile + hr) * 64 + lane] = vh[e];
+        }
+    };
+    double *s0 = P, *s1 = P + PLANE, *s2 = P + 2 * PLANE;
+    fetch(); keep(s0);
+    fetch(); keep(s1);
+    fetch(); keep(s2);
+    fetch();
+    lds_barrier();
+    // the k face under the first cell, from the cell before it, then cell by cell
+    long l = IDX(z, i, j, k0 - 1), lt = CART ? 0 : MTR(z, i, j, k0 - 1);
+    double fk[5];
+    const int mine = 2 + (w + 2) * 64 + lane;
+    const double *m1, *p0, *p1;
+    auto planes = [&]() { m1 = s0 + mine; p0 = s1 + mine; p1 = s2 + mine; };
+    auto advance = [&]() {
+        lds_barrier();
+        keep(s0);
+        fetch();
+        double* t = s0; s0 = s1; s1 = s2; s2 = t;
+        l += z.inck; lt += z.mk;
+        lds_barrier();
+        planes();
+    };
+    planes();
+    face_flux_at<KFLU, SLOPE, LAMIN, CART, 2>(f, z, PlaneCell<0, 1>{z, m1, p0, p1, vo, l, lt}, fk);
     for (int k = k0; k <= k1; k++) {
-        long l = IDX(z, i, j, k);
+        advance();
+        double flu[5], acc[5];
         if (a.zero_init) {
 #pragma unroll
             for (int e = 0; e < 5; e++) acc[e] = 0.;
@@ -428,117 +531,41 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(FM_RES
         }
 #pragma unroll
         for (int e = 0; e < 5; e++) acc[e] = acc[e] + fk[e];
-        face_flux<KFLU, SLOPE, LAMIN, CART, 1>(f, z, rop, i, j, k, flu);
+        // (what the faces of a cell share is read again, not held in registers)
+        __builtin_amdgcn_sched_barrier(0);
+        face_flux_at<KFLU, SLOPE, LAMIN, CART, 1>(f, z, PlaneCell<0, 0>{z, m1, p0, p1, vo, l, apart<CART>(lt)}, flu);
 #pragma unroll
         for (int e = 0; e < 5; e++) acc[e] = acc[e] + flu[e];
-        face_flux<KFLU, SLOPE, LAMIN, CART, 0>(f, z, rop, i, j, k, flu);
+        __builtin_amdgcn_sched_barrier(0);
+        face_flux_at<KFLU, SLOPE, LAMIN, CART, 0>(f, z, PlaneCell<0, 0>{z, m1, p0, p1, vo, l, apart<CART>(lt)}, flu);
 #pragma unroll
         for (int e = 0; e < 5; e++) acc[e] = acc[e] + flu[e];
-        face_flux<KFLU, SLOPE, LAMIN, CART, 0>(f, z, rop, i + 1, j, k, flu);
 #pragma unroll
-        for (int e = 0; e < 5; e++) acc[e] = acc[e] - flu[e];
-        const bool jn = cb_next(j, z.cbj, z.nbj), kn = cb_next(k, z.cbk, z.nbk);
-        face_flux<KFLU, SLOPE, LAMIN, CART, 1>(f, z, rop, i, j + 1, k, flu);
+        for (int e = 0; e < 5; e++) acc[e] = acc[e] - from_lane<1>(flu[e]);
+        __builtin_amdgcn_sched_barrier(0);
+        face_flux_at<KFLU, SLOPE, LAMIN, CART, 1>(f, z, PlaneCell<1, 0>{z, m1, p0, p1, vo, l, apart<CART>(lt)}, flu);
         if (!jn) {
 #pragma unroll
             for (int e = 0; e < 5; e++) acc[e] = acc[e] - flu[e];
         }
-        face_flux<KFLU, SLOPE, LAMIN, CART, 2>(f, z, rop, i, j, k + 1, fk);
+        __builtin_amdgcn_sched_barrier(0);
+        face_flux_at<KFLU, SLOPE, LAMIN, CART, 2>(f, z, PlaneCell<0, 1>{z, m1, p0, p1, vo, l, apart<CART>(lt)}, fk);
+        const bool kn = cb_next(k, z.cbk, z.nbk);
         if (!kn) {
 #pragma unroll
             for (int e = 0; e < 5; e++) acc[e] = acc[e] - fk[e];
         }
-        if (KFLU == 5 && a.ncorr > 0) wall_correction<SLOPE, CART>(f, z, rop, a, i, j, k, acc);
-        if (jn) {
-#pragma unroll
-            for (int e = 0; e < 5; e++) acc[e] = acc[e] - flu[e];
-        }
-        if (kn) {
-#pragma unroll
-            for (int e = 0; e < 5; e++) acc[e] = acc[e] - fk[e];
-        }
-        res_update(z, a, rop, l, acc);
-    }
-}
-
-// Residual with every face flux evaluated once.  Block: 64 i-lanes x 5 j-rows of threads
-// marching RES_KC planes in k.  Lane tx of rows 0..3 evaluates the i-face at i0 + tx (its cell
-// i0 + tx takes face i + 1 from lane tx + 1, so a block covers 63 cells); row r evaluates the
-// j-face at j0 + r (row 4 only provides the face above the last cell row); each cell carries
-// the k-face under it from the previous plane.  Per cell the faces are summed in the reference
-// order (template_FluxAndBalance.for:192-271), so the result is the one of k_residual.
-constexpr int RES_KC = 32;
-
-template <int KFLU, int SLOPE, bool LAMIN, bool CART>
-__global__ void __launch_bounds__(320) k_residual_faces(KZ z, RhsArgs a) {
-    __shared__ double fj[2][5][5][64];        // [plane parity][row][eq][lane]
-    const int tx = threadIdx.x, ty = threadIdx.y;
-    const int i = blockIdx.x * 63 + tx + 1;
-    const int j = blockIdx.y * 4 + ty + 1;
-    const int k0 = blockIdx.z * RES_KC + 1;
-    const int k1 = k0 + RES_KC - 1 < z.nk ? k0 + RES_KC - 1 : z.nk;
-    const bool cell = tx < 63 && ty < 4 && i <= z.ni && j <= z.nj;
-    const bool iface = ty < 4 && j <= z.nj && i <= z.ni + 1;
-    const bool jface = tx < 63 && i <= z.ni && j <= z.nj + 1;
-    const double* __restrict__ rop = a.rop;
-    const long nd = z.nd;
-    FluxConst f = flux_const(z);
-    double fk[5] = {0., 0., 0., 0., 0.};
-    if (cell) face_flux<KFLU, SLOPE, LAMIN, CART, 2>(f, z, rop, i, j, k0, fk);
-    for (int k = k0; k <= k1; k++) {
-        const int par = k & 1;
-        double fl[5];
-        if (jface) {
-            face_flux<KFLU, SLOPE, LAMIN, CART, 1>(f, z, rop, i, j, k, fl);
-#pragma unroll
-            for (int e = 0; e < 5; e++) fj[par][ty][e][tx] = fl[e];
-        }
-        double fi[5] = {0., 0., 0., 0., 0.};
-        if (iface) face_flux<KFLU, SLOPE, LAMIN, CART, 0>(f, z, rop, i, j, k, fi);
-        double fi1[5];
-#pragma unroll
-        for (int e = 0; e < 5; e++) fi1[e] = __shfl_down(fi[e], 1, 64);
-        double fk1[5];
-        if (cell) face_flux<KFLU, SLOPE, LAMIN, CART, 2>(f, z, rop, i, j, k + 1, fk1);
-        __syncthreads();
-        if (cell) {
-            const long l = IDX(z, i, j, k);
-            double acc[5];
-            if (a.zero_init) {
-#pragma unroll
-                for (int e = 0; e < 5; e++) acc[e] = 0.;
-            } else {
-#pragma unroll
-                for (int e = 0; e < 5; e++) acc[e] = z.drodm[l + e * nd] * a.coefH;
-            }
-#pragma unroll
-            for (int e = 0; e < 5; e++) acc[e] = acc[e] + fk[e];
-#pragma unroll
-            for (int e = 0; e < 5; e++) acc[e] = acc[e] + fj[par][ty][e][tx];
-#pragma unroll
-            for (int e = 0; e < 5; e++) acc[e] = acc[e] + fi[e];
-#pragma unroll
-            for (int e = 0; e < 5; e++) acc[e] = acc[e] - fi1[e];
-            const bool jn = cb_next(j, z.cbj, z.nbj), kn = cb_next(k, z.cbk, z.nbk);
-            if (!jn) {
-#pragma unroll
-                for (int e = 0; e < 5; e++) acc[e] = acc[e] - fj[par][ty + 1][e][tx];
-            }
-            if (!kn) {
-#pragma unroll
-                for (int e = 0; e < 5; e++) acc[e] = acc[e] - fk1[e];
-            }
+        if (own) {
+            if (KFLU == 5 && a.ncorr > 0) wall_correction<SLOPE, CART>(f, z, rop, a, i, j, k, acc);
             if (jn) {
 #pragma unroll
-                for (int e = 0; e < 5; e++) acc[e] = acc[e] - fj[par][ty + 1][e][tx];
+                for (int e = 0; e < 5; e++) acc[e] = acc[e] - flu[e];
             }
             if (kn) {
 #pragma unroll
-                for (int e = 0; e < 5; e++) acc[e] = acc[e] - fk1[e];
+                for (int e = 0; e < 5; e++) acc[e] = acc[e] - fk[e];
             }
             res_update(z, a, rop, l, acc);
-#pragma unroll
-            for (int e = 0; e < 5; e++) fk[e] = fk1[e];
         }
     }
 }
@@ -1101,62 +1128,50 @@ static void res_lc(const KZ& z, const RhsArgs& a, bool lamin, dim3 g, hipStream_
 }
 
 template <int KFLU, int SLOPE>
-static void res_kcol(const KZ& z, const RhsArgs& a, bool lamin, hipStream_t st) {
-    const int n = a.kcol_n > 0 ? a.kcol_n : RES_KCOL_N;
-    dim3 g((z.ni + 63) / 64, (z.nj + 3) / 4, (z.nk + n - 1) / n);
+static void res_planes(const KZ& z, const RhsArgs& a, bool lamin, hipStream_t st) {
+    // cells up k per workgroup: two workgroups fit a CU, so they run in rounds of 2 x 256, each round as
+    // long as the 4 n face fluxes of its cells, the k face under the first one and the first planes (about
+    // two faces' time); of the even cuts of nk, the one whose rounds take least
+    const int nx = (z.nj + kPlaneRows - 1) / kPlaneRows * z.nit, nb = (nx + kPlaneCells - 1) / kPlaneCells;
+    int n = a.kcol_n > 0 ? a.kcol_n : z.nk;
+    long best = -1;
+    for (int cuts = 1; a.kcol_n <= 0 && cuts <= z.nk; cuts++) {
+        const int m = (z.nk + cuts - 1) / cuts;
+        if ((cuts - 1) * m >= z.nk) continue;          // (the same m as fewer cuts)
+        const long t = ((long)nb * cuts + kPlaneSlots - 1) / kPlaneSlots * (4 * m + 3);
+        if (best < 0 || t < best) { best = t; n = m; }
+    }
+    dim3 g(nb, (z.nk + n - 1) / n), b(64 * kPlaneRows);
     if (lamin) {
-        if (z.typ == 2) hipLaunchKernelGGL((k_residual_kcol<KFLU, SLOPE, true, true>), g, blk2, 0, st, z, a);
-        else hipLaunchKernelGGL((k_residual_kcol<KFLU, SLOPE, true, false>), g, blk2, 0, st, z, a);
+        if (z.typ == 2) hipLaunchKernelGGL((k_residual_planes<KFLU, SLOPE, true, true>), g, b, 0, st, z, a, n);
+        else hipLaunchKernelGGL((k_residual_planes<KFLU, SLOPE, true, false>), g, b, 0, st, z, a, n);
     } else {
-        if (z.typ == 2) hipLaunchKernelGGL((k_residual_kcol<KFLU, SLOPE, false, true>), g, blk2, 0, st, z, a);
-        else hipLaunchKernelGGL((k_residual_kcol<KFLU, SLOPE, false, false>), g, blk2, 0, st, z, a);
+        if (z.typ == 2) hipLaunchKernelGGL((k_residual_planes<KFLU, SLOPE, false, true>), g, b, 0, st, z, a, n);
+        else hipLaunchKernelGGL((k_residual_planes<KFLU, SLOPE, false, false>), g, b, 0, st, z, a, n);
     }
 }
 
 template <int KFLU, int SLOPE>
-static void res_faces(const KZ& z, const RhsArgs& a, bool lamin, hipStream_t st) {
-    dim3 g((z.ni + 62) / 63, (z.nj + 3) / 4, (z.nk + RES_KC - 1) / RES_KC), b(64, 5);
-    if (lamin) {
-        if (z.typ == 2) hipLaunchKernelGGL((k_residual_faces<KFLU, SLOPE, true, true>), g, b, 0, st, z, a);
-        else hipLaunchKernelGGL((k_residual_faces<KFLU, SLOPE, true, false>), g, b, 0, st, z, a);
-    } else {
-        if (z.typ == 2) hipLaunchKernelGGL((k_residual_faces<KFLU, SLOPE, false, true>), g, b, 0, st, z, a);
-        else hipLaunchKernelGGL((k_residual_faces<KFLU, SLOPE, false, false>), g, b, 0, st, z, a);
-    }
+static void res_scheme(const KZ& z, const RhsArgs& a, hipStream_t st) {
+    const bool lamin = z.iflow == 2;
+    const dim3 g((z.ni + 63) / 64, (z.nj + 3) / 4, z.nk);
+    // The planes are faster but for Cartesian Euler zones of one round of workgroups, whose few operations
+    // a cell do not pay for the planes' barriers: cells / planes at 32 x 24 x 20 7.6 / 8.0 us (Roe 11.1 /
+    // 11.5), 48^3 15.3 / 15.2, 64^3 21.4 / 23.0, 80^3 53 / 34
+    const bool cells = a.schedule == RES_CELLS ||
+                       (a.schedule == RES_AUTO && !lamin && z.typ == 2 && (long)g.x * g.y * g.z <= 1024);
+    if (cells) res_lc<KFLU, SLOPE>(z, a, lamin, g, st);
+    else res_planes<KFLU, SLOPE>(z, a, lamin, st);
 }
 
 int launch_residual(const KZ& z, const RhsArgs& a, hipStream_t st) {
-    bool lamin = z.iflow == 2;
-    if (a.schedule == RES_KCOL) {
-        if (z.kflu == 5) {
-            if (z.slope == 1) res_kcol<5, 1>(z, a, lamin, st);
-            else if (z.slope == 2) res_kcol<5, 2>(z, a, lamin, st);
-            else if (z.slope == 3) res_kcol<5, 3>(z, a, lamin, st);
-            else return -1;
-        } else if (z.kflu == 1 && z.slope == 2) res_kcol<1, 2>(z, a, lamin, st);
-        else if (z.kflu == 2 && z.slope == 2) res_kcol<2, 2>(z, a, lamin, st);
-        else return -1;
-        return 0;
-    }
-    if (a.schedule == RES_FACES && a.ncorr == 0) {
-        if (z.kflu == 5) {
-            if (z.slope == 1) res_faces<5, 1>(z, a, lamin, st);
-            else if (z.slope == 2) res_faces<5, 2>(z, a, lamin, st);
-            else if (z.slope == 3) res_faces<5, 3>(z, a, lamin, st);
-            else return -1;
-        } else if (z.kflu == 1 && z.slope == 2) res_faces<1, 2>(z, a, lamin, st);
-        else if (z.kflu == 2 && z.slope == 2) res_faces<2, 2>(z, a, lamin, st);
-        else return -1;
-        return 0;
-    }
-    dim3 g((z.ni + 63) / 64, (z.nj + 3) / 4, z.nk);
     if (z.kflu == 5) {
-        if (z.slope == 1) res_lc<5, 1>(z, a, lamin, g, st);
-        else if (z.slope == 2) res_lc<5, 2>(z, a, lamin, g, st);
-        else if (z.slope == 3) res_lc<5, 3>(z, a, lamin, g, st);
+        if (z.slope == 1) res_scheme<5, 1>(z, a, st);
+        else if (z.slope == 2) res_scheme<5, 2>(z, a, st);
+        else if (z.slope == 3) res_scheme<5, 3>(z, a, st);
         else return -1;
-    } else if (z.kflu == 1 && z.slope == 2) res_lc<1, 2>(z, a, lamin, g, st);
-    else if (z.kflu == 2 && z.slope == 2) res_lc<2, 2>(z, a, lamin, g, st);
+    } else if (z.kflu == 1 && z.slope == 2) res_scheme<1, 2>(z, a, st);
+    else if (z.kflu == 2 && z.slope == 2) res_scheme<2, 2>(z, a, st);
     else return -1;
     return 0;
 }
@@ -1325,11 +1340,12 @@ __global__ void k_effort(KZ z, EffArgs a) {
         tn[0] = tm[lt]; tn[1] = tm[lt + ndm]; tn[2] = tm[lt + 2 * ndm];
         sn = sqrt(tn[0] * tn[0] + tn[1] * tn[1] + tn[2] * tn[2]);
     }
-    slope_state<SLOPE>(f, rop, nd, l, inc, qm, qp);
-    inviscid_flux<KFLU, CART, D>(f, rop, z.wig, nd, l, tn, sn, qm, qp, fl);
+    const MemCell cell(z, rop, l, lt);
+    slope_state<SLOPE, D>(f, cell, qm, qp);
+    inviscid_flux<KFLU, CART, D>(f, cell, tn, sn, qm, qp, fl);
     if (LAMIN) {
-        if (CART) visc_cart<D>(f, z, rop, z.xmut, l, fl, gv);
-        else visc_full<D>(f, z, rop, z.xmut, l, lt, tn, fl, gv);
+        if (CART) visc_cart<D>(f, cell, fl, gv);
+        else visc_full<D>(f, z, cell, tn, fl, gv);
     }
     const double pinf = z.pinf;
     const double norm = 2. / (z.roinf * (z.vinf * z.vinf));

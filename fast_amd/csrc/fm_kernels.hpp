@@ -23,18 +23,14 @@ struct RhsArgs {
     double coefH, coefW;    // RK coefficients
     int implicit, nitcfg;
     double c1, c2, c3;      // BDF coefficients
-    int schedule;           // RES_CELLS (six faces per cell), RES_FACES (each face once) or
-                            // RES_KCOL (a thread walks kcol_n cells up k, k faces once)
-    int kcol_n;             // RES_KCOL column length (0: RES_KCOL_N)
+    int schedule;           // RES_CELLS (six faces per cell from memory), RES_AUTO (that or the
+                            // planes in LDS, whichever is faster), else the planes
+    int kcol_n;             // cells up k per workgroup of the planes (0: by the zone's size)
     int ncorr;              // Roe: wall faces whose Euler flux is replaced, in BC order
     WallCorr corr[kMaxWallCorr];
     double ck_vent, c_ale;  // shape_tab_mtr.for mesh-motion factors of the wall flux
 };
 enum { RES_CELLS = 0, RES_FACES = 1, RES_KCOL = 2, RES_AUTO = 3 };
-#ifndef FM_RES_KCOL_N
-#define FM_RES_KCOL_N 4
-#endif
-constexpr int RES_KCOL_N = FM_RES_KCOL_N;
 
 struct LuWork;
 struct LuArgs {

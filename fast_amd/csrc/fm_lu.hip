@@ -1090,14 +1090,6 @@ template <bool CART> constexpr int lu_slot_doubles() { return (lu_skf<CART>() + 
 template <bool CART> constexpr int lu_lds_doubles() { return lu_ring<CART>() * lu_slot_doubles<CART>() + 20 * 64; }
 constexpr int kLuStThreads = 6 * 64;
 
-// End of a half step: the LDS writes of every wave are visible to the others.  Only LDS is ordered: a
-// __syncthreads() would also wait for the wave's global stores and loads in flight.
-__device__ __forceinline__ void lu_step_barrier() {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
-    __builtin_amdgcn_s_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
-}
-
 // 1 KB from device memory straight into LDS: lane l copies the 16 bytes at src + 16 l to LDS byte
 // dst + 16 l.  In asm, with no register written, because the compiler would wait for every copy in
 // flight before the wave's next LDS read; lu_copy_wait counts them instead (the wave that copies
@@ -1205,9 +1197,9 @@ __device__ __forceinline__ void lu_sweep_wave(const KZ& z, const LuArgs& a, cons
     // (two barriers before the first step: the first row in place, then read by every wave before its
     // slot is filled again)
     Row cur, nxt;
-    lu_step_barrier();
+    lds_barrier();
     read_row(0, cur);
-    lu_step_barrier();
+    lds_barrier();
     // step s; EDGE: lanes may lack a neighbour
     auto step = [&](int s, auto at_edge) {
         constexpr bool EDGE = decltype(at_edge)::value;
@@ -1247,7 +1239,7 @@ __device__ __forceinline__ void lu_sweep_wave(const KZ& z, const LuArgs& a, cons
         }
 #pragma unroll
         for (int e = 0; e < NE; e++) pc.W[(E0 + e) * 64 + L] = x1[e] * cur.dg;
-        lu_step_barrier();
+        lds_barrier();
         // the solution of the step; while it arrives, the row of the next step is asked for
         double x[5];
 #pragma unroll
@@ -1287,7 +1279,7 @@ __device__ __forceinline__ void lu_sweep_wave(const KZ& z, const LuArgs& a, cons
             }
         }
         cur = nxt;
-        lu_step_barrier();
+        lds_barrier();
     };
     // the steps whose lanes may lack a neighbour, two at a time, then the others
     const int steps = pc.steps(), nedge = edge ? steps : 16;
@@ -1321,14 +1313,14 @@ __device__ __forceinline__ void lu_rows_wave(const LuPencil<CART, LOWER>& pc) {
     };
     for (int q = 0; q < RING; q++) copy_row(q);
     lu_copy_wait<kCopies * (RING - 2)>();
-    lu_step_barrier();
-    lu_step_barrier();
+    lds_barrier();
+    lds_barrier();
     const int steps = pc.steps();
     for (int s = 0; s < steps; s++) {
         copy_row(s + RING);
-        lu_step_barrier();
+        lds_barrier();
         lu_copy_wait<kCopies * (RING - 2)>();
-        lu_step_barrier();
+        lds_barrier();
     }
     lu_copy_wait<0>();
 }
@@ -1397,18 +1389,18 @@ __device__ __forceinline__ void lu_halo_wave(const LuArgs& a, const LuPencil<CAR
     halo(0, 0);
     hand_in(0);
     hload(kLuStHalo, 0);
-    lu_step_barrier();
-    lu_step_barrier();
+    lds_barrier();
+    lds_barrier();
     const int steps = pc.steps();
     for (int s0 = 0; s0 < steps; s0 += 2) {
 #pragma unroll
         for (int q = 0; q < 2; q++) {
             constexpr int H = kLuStHalo;
             halo(s0 + q + 1, (q + 1) % H);
-            lu_step_barrier();
+            lds_barrier();
             hand_in((q + 1) % H);
             hload(s0 + q + 1 + H, (q + 1) % H);
-            lu_step_barrier();
+            lds_barrier();
         }
     }
 }

@@ -203,9 +203,10 @@ int fm_compute_timed(fm_ctx* ctx, int nitrun, int nstep_deb, int nstep_fin, int 
    clears the word (fm_compute itself is asynchronous and returns FM_OK).  With several zones
    and FM_OPT_ZONE_BATCH on, the sweeps of all zones run as one dataflow launch per sweep. */
 #define FM_LU_DATAFLOW 2
-/* FM_LU_STREAM (default): one wave per pencil of 8 x 8 (j, k) lines sweeps the whole i extent as a
-   skewed wavefront (neighbour products move between lanes by DPP and ds_bpermute) and hands its
-   face products to the next pencils through a global exchange (bounded waits, reported as above).
+/* FM_LU_STREAM (default): one workgroup of six waves per pencil of 8 x 8 (j, k) lines sweeps the whole i
+   extent as a skewed wavefront (one equation per wave, then one product per wave; rows copied into
+   LDS ahead) and hands its face products to the next pencils through a global exchange (bounded
+   waits, reported as above).
    Its inputs are first copied into a skewed, pencil-major layout (one contiguous row per step and
    array; on curvilinear zones with the mean face normals) and its results copied back; the zone
    needs 16 (3dcart) or 25 (3dfull) doubles per cell more device memory for that copy.  Inside
@@ -215,11 +216,10 @@ int fm_compute_timed(fm_ctx* ctx, int nitrun, int nstep_deb, int nstep_fin, int 
    zones and FM_OPT_ZONE_BATCH on, the pencils of all zones go through one launch per sweep.  FP32
    sweeps run the dataflow schedule. */
 #define FM_LU_STREAM 3
-/* FM_OPT_RESIDUAL_SCHEDULE: FM_RES_CELLS evaluates the six faces of every cell;
-   FM_RES_FACES evaluates every face flux once and sums them per cell in the reference order;
-   FM_RES_KCOL walks a column of 4 cells up k per thread, evaluating the k faces once;
-   FM_RES_AUTO (default) takes FM_RES_CELLS on Cartesian zones and FM_RES_KCOL on curvilinear
-   ones.  Same results bit for bit. */
+/* FM_OPT_RESIDUAL_SCHEDULE: FM_RES_CELLS evaluates the six faces of every cell from memory;
+   FM_RES_FACES and FM_RES_KCOL walk columns of cells up k with planes of the state in LDS, four face
+   fluxes per cell; FM_RES_AUTO (default) takes the faster of the two for the zone (the planes but
+   on small Cartesian Euler zones).  Same results bit for bit. */
 #define FM_OPT_RESIDUAL_SCHEDULE 2
 #define FM_RES_CELLS 0
 #define FM_RES_AUTO 3
@@ -250,7 +250,7 @@ int fm_compute_timed(fm_ctx* ctx, int nitrun, int nstep_deb, int nstep_fin, int 
    (FM_E_UNSUPPORTED, in either order of setting). */
 #define FM_OPT_LU_GIVE_UP 6
 /* Tile shapes (same results bit for bit, only the speed changes; fast_amd.tune picks them):
-   FM_OPT_RES_KCOL_N: cells per thread column of FM_RES_KCOL (1..64, 0 = built-in 4);
+   FM_OPT_RES_KCOL_N: cells up k per workgroup of the residual's planes (1..64, 0 = by the zone's size);
    FM_OPT_LU_FLOW_GRID: workgroups of a dataflow sweep (0 = as many as can be resident). */
 #define FM_OPT_RES_KCOL_N 7
 #define FM_OPT_LU_FLOW_GRID 8

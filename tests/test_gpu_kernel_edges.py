@@ -22,3 +22,22 @@ def test_lu_stream_tiles(ctxmod, orc, mesh, mode, n):  # noqa: F811
         mk = lambda: H.jittered_box(n, H.numerics("ausmpred", mode), bcs=H.WALL_J)
     zo, zg, _, _ = run_pair(ctxmod, orc, mk, nsub, nsteps=2)
     assert_same(zo, zg, ghosts=True)
+
+
+@pytest.mark.parametrize("kcol", [0, 1, 3, 64])
+@pytest.mark.parametrize("n", [(2, 2, 2), (3, 5, 4), (56, 4, 2), (57, 3, 5), (61, 9, 7), (126, 6, 3)])
+@pytest.mark.parametrize("case", ["ausmpred-lamin-cart", "roe_min-euler-full", "senseur-lamin-full", "roe_kap-lamin-wall"])
+def test_residual_planes_tiles(ctxmod, orc, case, n, kcol):  # noqa: F811
+    """The residual's planes on rows that end before, at and after a wave's 60 cells, on groups of 1 to 4
+    rows, and on columns of one cell, of lengths that do not divide nk and longer than nk."""
+    scheme, flow, mesh = case.split("-")
+    mode = "bdf_ss2" if mesh == "cart" else "explicit" if flow == "euler" else "local"
+    nsub = {"bdf_ss2": 2, "explicit": 3, "local": 1}[mode]
+    num = H.numerics(scheme, mode)
+    if mesh == "cart":
+        mk = lambda: cases.tgv_zone(n, num, perturb=0.02, flow=flow)
+    else:
+        mk = lambda: H.jittered_box(n, num, flow=flow, bcs=H.WALL_J if mesh == "wall" else None)
+    zo, zg, _, _ = run_pair(ctxmod, orc, mk, nsub, options=((ctxmod.OPT_RESIDUAL_SCHEDULE, ctxmod.RES_KCOL),
+                                                            (ctxmod.OPT_RES_KCOL_N, kcol)))
+    assert_same(zo, zg, ghosts=True)
