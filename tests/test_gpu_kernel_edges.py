@@ -41,3 +41,33 @@ def test_residual_planes_tiles(ctxmod, orc, case, n, kcol):  # noqa: F811
     zo, zg, _, _ = run_pair(ctxmod, orc, mk, nsub, options=((ctxmod.OPT_RESIDUAL_SCHEDULE, ctxmod.RES_KCOL),
                                                             (ctxmod.OPT_RES_KCOL_N, kcol)))
     assert_same(zo, zg, ghosts=True)
+
+
+def bc_set(n, kind):
+    """Conditions of a zone of n cells: "split" cuts the j faces into four windows each (10 conditions and
+    more than one launch), "overlap" lets two conditions of a face share cells, where the later one wins."""
+    ni, nj, nk = n
+    a, b = max(1, ni // 2), max(1, nk // 2)
+    per = [("BCautoperiod", f, None) for f in ("imin", "imax", "kmin", "kmax")]
+    if kind == "overlap":
+        return per + [("BCWallViscous", "jmin", None), ("BCFarfield", (3, [1, a, 1, 1, 1, nk]), None),
+                      ("BCOutflow", "jmax", None), ("BCWallViscous", (4, [a, ni, nj, nj, 1, b]), None)]
+    out = [("BCFarfield", "imin", None), ("BCOutflow", "imax", None)] + per[2:]
+    names = ["BCWallViscous", "BCFarfield", "BCExtrapolate", "BCWallInviscid"]
+    for idir, j in ((3, 1), (4, nj)):
+        names = names[1:] + names[:1]
+        q = [[1, a, 1, b], [a + 1, ni, 1, b], [1, a, b + 1, nk], [a + 1, ni, b + 1, nk]]
+        out += [(m, (idir, [w[0], w[1], j, j, w[2], w[3]]), None) for m, w in zip(names, q)]
+    return out
+
+
+@pytest.mark.parametrize("mode", ["explicit", "bdf_ss2", "local"])
+@pytest.mark.parametrize("kind", ["split", "overlap"])
+@pytest.mark.parametrize("n", [(2, 2, 2), (3, 3, 3), (9, 6, 5), (34, 5, 19)])
+def test_bc_sets(ctxmod, orc, n, kind, mode):  # noqa: F811
+    """Boundary conditions sharing a launch, over more than one launch, and one after another where
+    their windows overlap or the zone is two cells wide."""
+    nsub = {"explicit": 3, "bdf_ss2": 2, "local": 1}[mode]
+    mk = lambda: H.jittered_box(n, H.numerics("ausmpred", mode), bcs=bc_set(n, kind))
+    zo, zg, _, _ = run_pair(ctxmod, orc, mk, nsub, nsteps=2)
+    assert_same(zo, zg, ghosts=True)
