@@ -152,7 +152,6 @@ void launch_lu_stream_list(bool cart, const LuZone* zones, int nz, const LuWork*
                            int npack, int nunpack, int* counter, hipStream_t st);
 void launch_lu_flow_list(bool cart, const LuZone* zones, const LuWork* work, int nwork, int* counter,
                          hipStream_t st);
-int lu_pipeline_failed(const LuArgs& a, hipStream_t st);
 // doubles of the tile-boundary exchange buffer the pipelined sweeps of an LU box need
 long lu_exchange_size(int ni, int nj, int nk);
 void launch_copy_box(const KZ& z, const double* src, double* dst, Box b, hipStream_t st);

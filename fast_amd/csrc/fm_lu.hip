@@ -1751,18 +1751,6 @@ void launch_lu(const KZ& z, const LuArgs& a, hipStream_t st) {
 }
 
 // error word of the pipelined sweeps (a bounded wait gave up); clears it
-int lu_pipeline_failed(const LuArgs& a, hipStream_t st) {
-    if ((a.schedule != LU_PIPELINE && a.schedule != LU_DATAFLOW && a.schedule != LU_STREAM) || !a.sync) return 0;
-    int h = 0;
-    if (hipMemcpyAsync(&h, a.sync + 1, sizeof(int), hipMemcpyDeviceToHost, st) != hipSuccess) return -1;
-    if (hipStreamSynchronize(st) != hipSuccess) return -1;
-    if (h) {
-        int zero = 0;
-        (void)hipMemcpy(a.sync + 1, &zero, sizeof(int), hipMemcpyHostToDevice);
-    }
-    return h;
-}
-
 void launch_copy_box(const KZ& z, const double* src, double* dst, Box b, hipStream_t st) {
     int n0 = b.i1 - b.i0 + 1, n1 = b.j1 - b.j0 + 1, n2 = b.k1 - b.k0 + 1;
     if (n0 <= 0 || n1 <= 0 || n2 <= 0) return;

@@ -1,4 +1,5 @@
 """HIP kernels against the oracle, bit for bit, at the sizes where their tilings can go wrong."""
+import numpy as np
 import pytest
 
 from fast_amd import cases
@@ -71,3 +72,19 @@ def test_bc_sets(ctxmod, orc, n, kind, mode):  # noqa: F811
     mk = lambda: H.jittered_box(n, H.numerics("ausmpred", mode), bcs=bc_set(n, kind))
     zo, zg, _, _ = run_pair(ctxmod, orc, mk, nsub, nsteps=2)
     assert_same(zo, zg, ghosts=True)
+
+
+@pytest.mark.parametrize("n", [(3, 4, 5), (46, 46, 37), (46, 46, 38), (80, 80, 55), (80, 80, 56), (90, 90, 90), (90, 90, 91),
+                               (130, 97, 81)])
+def test_field_copies(ctxmod, n):  # noqa: F811
+    """Fields written and read back, at sizes around those where the copy changes its way: 4, 16 and 32 MB,
+    and a last chunk that is short."""
+    z = cases.tgv_zone(n, H.numerics("ausmpred", "explicit"))
+    ctx = ctxmod.Context(0)
+    zid = ctx.add_zone(z)
+    rng = np.random.default_rng(11)
+    for f in (ctxmod.FIELD_RO, ctxmod.FIELD_RO_M1):
+        a = rng.random(z.ro.size)
+        ctx.set(zid, f, a)
+        assert np.array_equal(ctx.get(zid, f, np.zeros_like(a)), a)
+    ctx.close()
