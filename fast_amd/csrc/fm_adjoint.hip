@@ -7,6 +7,7 @@
 //
 // Every floating-point operation follows the order of the oracle's fo_dpj_dpw and
 // fo_residual_vjp, compiled without contraction, so that the two agree bit for bit.
+#include <algorithm>
 #include "fm_device.hpp"
 #include "fm_kernels.hpp"
 
@@ -106,9 +107,13 @@ __device__ __forceinline__ void dpj_mirror(const double n[3], const double g[5],
 
 // One thread per face of the window: J_D = s (cos a F_x + sin a F_y), J_L = s (cos a F_y -
 // sin a F_x), s = sens * surfinv (dpJ_dpW_fluausm_euler_o3_2d.for:359-366, 855-890); the two
-// interior cells of the stencil are assigned their conservative gradients (:958-978).
-template <bool CART, int D>
-__global__ void k_dpj_dpw(KZ z, DpjArgs a) {
+// interior cells of the stencil, A next to the face and B behind it, are assigned their conservative
+// gradients (:958-978): out[(o * 10 + s * 5 + e) * nf + t], o = 0 J_D, 1 J_L, s = 0 A, 1 B, face t.
+// Only these leave the device: whole fields up and down for two layers of cells were 100 MB of a
+// 96 x 80 x 72 zone, 3 ms, against 1.1 MB.  UP is a template argument so that the stencil stays in
+// registers (indexed by a run-time side it went to 576 bytes of scratch: 26 us, now 12).
+template <bool CART, int D, bool up>
+__global__ void __launch_bounds__(64) k_dpj_dpw(KZ z, DpjArgs a) {
     const int n0 = a.w[1] - a.w[0] + 1, n1 = a.w[3] - a.w[2] + 1, n2 = a.w[5] - a.w[4] + 1;
     const long nf = (long)n0 * n1 * n2;
     const long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
@@ -117,7 +122,6 @@ __global__ void k_dpj_dpw(KZ z, DpjArgs a) {
     const FluxConst f = flux_const(z);
     const long l = IDX(z, i, j, k), nd = z.nd, ndm = z.ndm;
     const long inc = D == 0 ? 1 : D == 1 ? z.incj : z.inck;
-    const bool up = (a.idir % 2) == 0;
     const double norm = 2. / (z.roinf * (z.vinf * z.vinf));
     const double sens = up ? norm : -norm;
     const double cc = sens * a.surfinv * a.cosa, cs = sens * a.surfinv * a.sina;
@@ -139,7 +143,7 @@ __global__ void k_dpj_dpw(KZ z, DpjArgs a) {
     for (int s = 0; s < 4; s++)
 #pragma unroll
         for (int e = 0; e < 5; e++) q[s][e] = a.rop[cell[s] + e * nd];
-    const int A = up ? 1 : 2, B = up ? 0 : 3, gA = up ? 2 : 1, gB = up ? 3 : 0;
+    constexpr int A = up ? 1 : 2, B = up ? 0 : 3, gA = up ? 2 : 1, gB = up ? 3 : 0;
 #pragma unroll
     for (int o = 0; o < 2; o++) {
         const double fb[3] = {o == 0 ? cc : -cs, o == 0 ? cs : cc, 0.};
@@ -154,30 +158,35 @@ __global__ void k_dpj_dpw(KZ z, DpjArgs a) {
         double ga[5], gb[5];
         dpj_cons(q[A], cvm, wb[A], ga);
         dpj_cons(q[B], cvm, wb[B], gb);
-        double* out = o == 0 ? a.dcd : a.dcl;
 #pragma unroll
         for (int e = 0; e < 5; e++) {
-            out[cell[A] + e * nd] = ga[e];
-            out[cell[B] + e * nd] = gb[e];
+            a.out[(o * 10 + e) * nf + t] = ga[e];
+            a.out[(o * 10 + 5 + e) * nf + t] = gb[e];
         }
     }
 }
 
-template <bool CART>
+template <bool CART, int D>
 static void dpj_d(const KZ& z, const DpjArgs& a, dim3 g, hipStream_t st) {
+    if (a.idir % 2 == 0) hipLaunchKernelGGL((k_dpj_dpw<CART, D, true>), g, dim3(64), 0, st, z, a);
+    else hipLaunchKernelGGL((k_dpj_dpw<CART, D, false>), g, dim3(64), 0, st, z, a);
+}
+
+template <bool CART>
+static void dpj(const KZ& z, const DpjArgs& a, dim3 g, hipStream_t st) {
     int d = (a.idir - 1) / 2;
-    if (d == 0) hipLaunchKernelGGL((k_dpj_dpw<CART, 0>), g, dim3(256), 0, st, z, a);
-    else if (d == 1) hipLaunchKernelGGL((k_dpj_dpw<CART, 1>), g, dim3(256), 0, st, z, a);
-    else hipLaunchKernelGGL((k_dpj_dpw<CART, 2>), g, dim3(256), 0, st, z, a);
+    if (d == 0) dpj_d<CART, 0>(z, a, g, st);
+    else if (d == 1) dpj_d<CART, 1>(z, a, g, st);
+    else dpj_d<CART, 2>(z, a, g, st);
 }
 
 int launch_dpj_dpw(const KZ& z, const DpjArgs& a, hipStream_t st) {
     if (z.kflu != 1 || z.slope != 2 || z.iflow != 1) return -1;     // option 213 only
     long nf = (long)(a.w[1] - a.w[0] + 1) * (a.w[3] - a.w[2] + 1) * (a.w[5] - a.w[4] + 1);
     if (nf <= 0) return 0;
-    dim3 g((unsigned)((nf + 255) / 256));
-    if (z.typ == 2) dpj_d<true>(z, a, g, st);
-    else dpj_d<false>(z, a, g, st);
+    dim3 g((unsigned)((nf + 63) / 64));
+    if (z.typ == 2) dpj<true>(z, a, g, st);
+    else dpj<false>(z, a, g, st);
     return 0;
 }
 
@@ -194,7 +203,7 @@ int launch_dpj_dpw(const KZ& z, const DpjArgs& a, hipStream_t st) {
 // adds those of the faces c - 1, c, c + 1, c + 2 in that order, then adds the sum to out.
 // Directions run i, j, k.  Kernels:
 // * i: one workgroup per (j, k) row, the row's face contributions staged in LDS;
-// * j, k: one thread per line, marching up the line with the four-cell stencil and the four
+// * j, k: one thread per segment of a line, marching up it with the four-cell stencil and the four
 //   partial sums in registers (a cell is complete, and written, once its last face is done);
 // * rows too long for LDS: face contributions through a global buffer, then a gather pass.
 
@@ -427,27 +436,36 @@ __global__ void __launch_bounds__(256) k_vjp_row(KZ z, VjpArgs a) {
     }
 }
 
-// j or k direction: one thread per line (i fastest across threads), marching the faces of the line
+// j or k direction: one thread per segment of a line (i fastest across threads), marching its faces.
+// Segment s (blockIdx.y) owns cells s len + 1 .. (s + 1) len, the first and the last also the two ghosts
+// before and behind the line; the faces lo - 1 .. hi + 2 of its cells start one face below, and the three
+// cells before its own come out incomplete and are dropped.  A step is one serial chain of some 600
+// instructions and the loads it starts with, 2.5 us; whole lines were 27 workgroups on 96 x 80 x 72, 200 us
+// up j and 179 up k, segments of 5 take 35 and 32.
 template <bool CART, int D>
-__global__ void __launch_bounds__(256) k_vjp_march(KZ z, VjpArgs a) {
+__global__ void __launch_bounds__(256) k_vjp_march(KZ z, VjpArgs a, int len) {
     const int no = D == 1 ? z.nk : z.nj;
     const long nl = (long)z.ni * no;
     const long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
     if (t >= nl) return;
     const int i = 1 + (int)(t % z.ni), o = 1 + (int)(t / z.ni);
     const int n = D == 1 ? z.nj : z.nk;
+    const int lo = (int)blockIdx.y * len + 1;
+    const bool last = blockIdx.y + 1 == gridDim.y;
+    const int f0 = lo == 1 ? 1 : lo - 1, f1 = last ? n + 1 : lo + len + 1;
+    const int first = lo == 1 ? -1 : lo;          // first cell written
     const long nd = z.nd, inc = D == 1 ? z.incj : z.inck;
     const FluxConst f = flux_const(z);
     auto cell = [&](int c) -> long { return D == 1 ? IDX(z, i, c, o) : IDX(z, i, o, c); };
     double q[4][5], acc[4][5], lm[5];
-    const long l0 = cell(1);
+    const long l0 = cell(1), lf = l0 + (long)(f0 - 1) * inc;
 #pragma unroll
     for (int s2 = 0; s2 < 4; s2++)
 #pragma unroll
-        for (int e = 0; e < 5; e++) { q[s2][e] = a.rop[l0 + (s2 - 2) * inc + e * nd]; acc[s2][e] = 0.; }
+        for (int e = 0; e < 5; e++) { q[s2][e] = a.rop[lf + (s2 - 2) * inc + e * nd]; acc[s2][e] = 0.; }
 #pragma unroll
-    for (int e = 0; e < 5; e++) lm[e] = 0.;
-    for (int fi = 1; fi <= n + 1; fi++) {
+    for (int e = 0; e < 5; e++) lm[e] = f0 >= 2 ? a.lam[lf - inc + e * nd] : 0.;
+    for (int fi = f0; fi <= f1; fi++) {
         const long l = l0 + (long)(fi - 1) * inc;
         double lp[5], fb[5];
 #pragma unroll
@@ -463,9 +481,11 @@ __global__ void __launch_bounds__(256) k_vjp_march(KZ z, VjpArgs a) {
 #pragma unroll
             for (int e = 0; e < 5; e++) acc[s2][e] = acc[s2][e] + wb[s2][e];
         // cell fi - 2 has had its last face
-        const long lc = l - 2 * inc;
+        if (fi - 2 >= first) {
+            const long lc = l - 2 * inc;
 #pragma unroll
-        for (int e = 0; e < 5; e++) a.out[lc + e * nd] = a.out[lc + e * nd] + acc[0][e];
+            for (int e = 0; e < 5; e++) a.out[lc + e * nd] = a.out[lc + e * nd] + acc[0][e];
+        }
 #pragma unroll
         for (int e = 0; e < 5; e++) {
             acc[0][e] = acc[1][e]; acc[1][e] = acc[2][e]; acc[2][e] = acc[3][e]; acc[3][e] = 0.;
@@ -477,12 +497,26 @@ __global__ void __launch_bounds__(256) k_vjp_march(KZ z, VjpArgs a) {
             for (int e = 0; e < 5; e++) q[3][e] = a.rop[l + 2 * inc + e * nd];
         }
     }
+    if (!last) return;
     // cells n, n + 1, n + 2
     const long ln = cell(n);
 #pragma unroll
     for (int s2 = 0; s2 < 3; s2++)
 #pragma unroll
         for (int e = 0; e < 5; e++) a.out[ln + s2 * inc + e * nd] = a.out[ln + s2 * inc + e * nd] + acc[s2][e];
+}
+
+// cells of a segment of the march: the steps it takes, len + 3, times how often the segments fill the chip
+// (two waves on each of 1024 SIMDs), at least 4 cells, the last segment as long as any
+static int march_length(long lines, int n) {
+    const long waves = (lines + 255) / 256 * 4;
+    int best = n;
+    long cost = (waves + 2047) / 2048 * (n + 1);
+    for (int len = 4; len < n; len++) {
+        const long segs = (n + len - 1) / len, c = (waves * segs + 2047) / 2048 * (len + 3);
+        if (c < cost) { cost = c; best = len; }
+    }
+    return best;
 }
 
 constexpr int kVjpRowMax = 400;    // longest i row staged in LDS (20 x (ni + 1) doubles <= 64 KiB)
@@ -494,12 +528,16 @@ template <bool CART, int D>
 static void vjp_dir(const KZ& z, const VjpArgs& a, hipStream_t st) {
     if (D == 0 && z.ni <= kVjpRowMax) {
         size_t lds = sizeof(double) * 20 * (size_t)(z.ni + 1);
-        hipLaunchKernelGGL((k_vjp_row<CART>), dim3((unsigned)((long)z.nj * z.nk)), dim3(256), lds, st, z, a);
+        // as many waves as the row has faces for: 256 threads on 97 faces took 41 us, 128 take 32
+        const unsigned w = std::min(256, (z.ni + 1 + 63) / 64 * 64);
+        hipLaunchKernelGGL((k_vjp_row<CART>), dim3((unsigned)((long)z.nj * z.nk)), dim3(w), lds, st, z, a);
         return;
     }
     if (D == 1 || D == 2) {
         long nl = (long)z.ni * (D == 1 ? z.nk : z.nj);
-        hipLaunchKernelGGL((k_vjp_march<CART, D>), dim3((unsigned)((nl + 255) / 256)), dim3(256), 0, st, z, a);
+        const int n = D == 1 ? z.nj : z.nk, len = march_length(nl, n);
+        hipLaunchKernelGGL((k_vjp_march<CART, D>), dim3((unsigned)((nl + 255) / 256), (unsigned)((n + len - 1) / len)),
+                           dim3(256), 0, st, z, a, len);
         return;
     }
     vjp_two_pass<CART, D>(z, a, st);

@@ -1134,21 +1134,34 @@ extern "C" int fm_dpj_dpw(fm_ctx* c, int zone, int level, int idir, const int* w
     int face = idir % 2 == 1 ? 1 : (d == 0 ? k.ni : d == 1 ? k.nj : k.nk) + 1;
     if (window[2 * d] != face) return fail(FM_E_ARG, "fm_dpj_dpw: window is not on the zone face of idir %d", idir);
     HIPCHK(hipSetDevice(c->device));
-    size_t bytes = sizeof(double) * 5 * (size_t)k.nd;
+    const int n0 = window[1] - window[0] + 1, n1 = window[3] - window[2] + 1, n2 = window[5] - window[4] + 1;
+    const size_t nf = (size_t)n0 * n1 * n2, bytes = sizeof(double) * 20 * nf;
     Work wk;
-    HIPCHK(wk.get(c, 2 * bytes));
-    double* buf = wk.p;
-    hipError_t e = link_copy(c, dcd, buf, bytes, true);
-    if (e == hipSuccess) e = link_copy(c, dcl, buf + 5 * k.nd, bytes, true);
+    HIPCHK(wk.get(c, bytes));
     DpjArgs a;
     a.idir = idir;
     for (int q = 0; q < 6; q++) a.w[q] = window[q];
     a.cosa = cosa; a.sina = sina; a.surfinv = surfinv;
-    a.rop = z->ro[level]; a.dcd = buf; a.dcl = buf + 5 * k.nd;
-    if (e == hipSuccess) { launch_dpj_dpw(k, a, c->stream); e = hipGetLastError(); }
-    if (e == hipSuccess) e = link_copy(c, dcd, buf, bytes, false);
-    if (e == hipSuccess) e = link_copy(c, dcl, buf + 5 * k.nd, bytes, false);
+    a.rop = z->ro[level]; a.out = wk.p;
+    std::vector<double> v;
+    double* h = bytes <= kLinkSlot && link_slot(c, 0) ? (double*)c->link_host[0] : nullptr;
+    if (!h) { v.resize(20 * nf); h = v.data(); }
+    launch_dpj_dpw(k, a, c->stream);
+    hipError_t e = hipGetLastError();
+    if (e == hipSuccess) e = hipMemcpyAsync(h, wk.p, bytes, hipMemcpyDeviceToHost, c->stream);
+    if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
     if (e != hipSuccess) return fail(FM_E_HIP, "fm_dpj_dpw: %s", hipGetErrorString(e));
+    // into the two layers of cells next to the face, row by row
+    const long inc = d == 0 ? 1 : d == 1 ? k.incj : k.inck;
+    const long off[2] = {idir % 2 ? 0 : -inc, idir % 2 ? inc : -2 * inc};
+    for (int o = 0; o < 2; o++)
+        for (int q = 0; q < 10; q++) {
+            double* out = (o == 0 ? dcd : dcl) + (q % 5) * k.nd + off[q / 5];
+            const double* src = h + (size_t)(o * 10 + q) * nf;
+            for (int kk = 0; kk < n2; kk++)
+                for (int jj = 0; jj < n1; jj++, src += n0)
+                    memcpy(out + IDX(k, window[0], window[2] + jj, window[4] + kk), src, sizeof(double) * n0);
+        }
     return FM_OK;
 }
 

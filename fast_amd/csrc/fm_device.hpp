@@ -33,7 +33,7 @@ struct KZ {
     double* xmut; double* drodm; double* coe; double* wig;
 };
 
-__device__ __forceinline__ long IDX(const KZ& z, int i, int j, int k) {
+__host__ __device__ __forceinline__ long IDX(const KZ& z, int i, int j, int k) {
     return (long)(i + z.nf - 1) + (long)(j + z.nf - 1) * z.incj + (long)(k + z.nfk - 1) * z.inck;
 }
 __device__ __forceinline__ long MTR(const KZ& z, int i, int j, int k) {

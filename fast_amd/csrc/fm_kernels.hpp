@@ -119,7 +119,8 @@ int launch_effort(const KZ& z, const EffArgs& a, hipStream_t st);
 // sums[0..11] = the 12 contributions of out (33 x nf) summed face by face
 void launch_effort_sum(const double* out, long nf, double* sums, hipStream_t st);
 // gradients of the pressure drag / lift coefficients at a slip-wall window (fm_adjoint.hip)
-struct DpjArgs { int idir, w[6]; double cosa, sina, surfinv; const double* rop; double* dcd; double* dcl; };
+// (out = 20 x nfaces: per face J_D and J_L in the two interior cells next to it, see k_dpj_dpw)
+struct DpjArgs { int idir, w[6]; double cosa, sina, surfinv; const double* rop; double* out; };
 int launch_dpj_dpw(const KZ& z, const DpjArgs& a, hipStream_t st);
 // out += (dR/dW)^T lam for the AUSM+(P) o3 Euler face balance (fm_adjoint.hip); buf holds
 // vjp_buffer_doubles(z) doubles

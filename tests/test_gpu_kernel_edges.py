@@ -88,3 +88,31 @@ def test_field_copies(ctxmod, n):  # noqa: F811
         ctx.set(zid, f, a)
         assert np.array_equal(ctx.get(zid, f, np.zeros_like(a)), a)
     ctx.close()
+
+
+@pytest.mark.parametrize("mesh", ["cart", "full"])
+@pytest.mark.parametrize("n", [(2, 2, 2), (63, 4, 5), (64, 9, 3), (17, 33, 26), (170, 7, 172)])
+def test_adjoint_tiles(ctxmod, orc, n, mesh):  # noqa: F811
+    """The transposed Jacobian's segments (lines no longer than one, of a cell over, of several) and rows
+    ending on a wave; the wall gradients of whole and part faces, beyond one pinned slot on the largest."""
+    num = H.numerics("ausmpred", "bdf")
+    if mesh == "cart":
+        mk = lambda: cases.tgv_zone(n, num, perturb=0.05, seed=3, flow="euler", bcs=H.INVISCID_J)
+    else:
+        mk = lambda: H.jittered_box(n, num, bcs=H.INVISCID_J, flow="euler")
+    zo, zg = mk(), mk()
+    orc.init_metric(zo)
+    orc.apply_bc(zo, zo.ro)
+    ctx = ctxmod.Context(0)
+    zid = ctx.add_zone(zg)
+    ctx.apply_bc(zid, 0)
+    lam = np.random.default_rng(4).standard_normal(5 * zo.nd)
+    assert np.array_equal(ctx.residual_vjp(zid, lam), orc.residual_vjp(zo, lam))
+    ni, nj, nk = n
+    for idir, w in ((3, [1, ni, 1, 1, 1, nk]), (4, [2, ni, nj + 1, nj + 1, 2, nk]), (1, [1, 1, 1, nj, 1, nk]),
+                    (2, [ni + 1, ni + 1, 2, nj, 1, nk]), (5, [1, ni, 1, nj, 1, 1]), (6, [1, ni, 1, 1, nk + 1, nk + 1])):
+        f = [np.full(5 * zo.nd, v) for v in (7.0, -3.0, 7.0, -3.0)]
+        orc.dpj_dpw(zo, idir, np.array(w, dtype=np.int32), 0.9, 0.3, 0.5, dcd=f[0], dcl=f[1])
+        ctx.dpj_dpw(zid, idir, w, 0.9, 0.3, 0.5, f[2], f[3])
+        assert np.array_equal(f[0], f[2]) and np.array_equal(f[1], f[3]), idir
+    ctx.close()
