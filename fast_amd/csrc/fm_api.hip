@@ -104,9 +104,9 @@ struct fm_ctx {
     std::vector<LuList> lu_lists;
     LuZone* lu_tab; int lu_tab_cap;
     LuZone* lu_host[2]; hipEvent_t lu_ev[2]; int lu_slot;
-    // the edge and corner table of several zones, outside graphs (staged as the LU table)
-    CoinsZone* co_tab; int co_cap;
-    CoinsZone* co_host[2]; hipEvent_t co_ev[2]; int co_slot;
+    // tables of several zones outside graphs, staged as the LU table: edges and corners, right-hand sides
+    struct Table { void* dev = nullptr; size_t cap = 0; void* host[2] = {}; hipEvent_t ev[2] = {}; int slot = 0; };
+    Table co_tab, rhs_tab;
     int* flow_ctr;           // block counter of the batched dataflow sweeps
     // several zones: each zone's right-hand side and boundary conditions run on a stream of its
     // own (forked from and joined back to `stream`); `cur` is the stream the zone work goes to
@@ -228,7 +228,11 @@ extern "C" int fm_ctx_destroy(fm_ctx* c) {
         delete g;
     }
     if (c->lu_tab) (void)hipFree(c->lu_tab);
-    if (c->co_tab) (void)hipFree(c->co_tab);
+    for (fm_ctx::Table* t : {&c->co_tab, &c->rhs_tab}) {
+        if (t->dev) (void)hipFree(t->dev);
+        for (void* h : t->host) if (h) (void)hipHostFree(h);
+        for (hipEvent_t e : t->ev) if (e) (void)hipEventDestroy(e);
+    }
     if (c->flow_ctr) (void)hipFree(c->flow_ctr);
     for (char* h : c->link_host) if (h) (void)hipHostFree(h);
     for (hipEvent_t e : c->link_ev) if (e) (void)hipEventDestroy(e);
@@ -240,8 +244,6 @@ extern "C" int fm_ctx_destroy(fm_ctx* c) {
     for (int q = 0; q < 2; q++) {
         if (c->lu_host[q]) (void)hipHostFree(c->lu_host[q]);
         if (c->lu_ev[q]) (void)hipEventDestroy(c->lu_ev[q]);
-        if (c->co_host[q]) (void)hipHostFree(c->co_host[q]);
-        if (c->co_ev[q]) (void)hipEventDestroy(c->co_ev[q]);
     }
     (void)hipEventDestroy(c->e0);
     (void)hipEventDestroy(c->e1);
@@ -867,43 +869,35 @@ static void lu_stream_after(Zone* z, const LuArgs& la) {
 }
 
 // One sub-iteration of one zone (gsdr3.cpp:152-444 with navier_stokes_struct.for and lhs.cpp).
-static int substep(fm_ctx* c, Zone* z, int nitcfg, int first_it, int lssiter_verif, int lexit_lu, int stop,
-                   LuArgs* defer = nullptr) {
-    KZ& k = z->k;
-    hipStream_t st = c->cur;
-    int implicit = k.itypcp <= 1;
+static double* level_ssiter(const Zone* z, int nitcfg) {
+    if (nitcfg == 1) return z->ro[0];
+    if (z->k.itypcp <= 1) return z->ro[2];
+    return nitcfg % 2 == 0 ? z->ro[2] : z->ro[0];
+}
+
+// what the coefficients and the residual of a sub-iteration take
+static int rhs_args(fm_ctx* c, Zone* z, int nitcfg, int first_it, RhsZone& r) {
+    const KZ& k = z->k;
+    const int implicit = k.itypcp <= 1;
     double* ro = z->ro[0]; double* ro_m1 = z->ro[1]; double* ro_p1 = z->ro[2];
-    double *ro_ssiter, *ro_cl;
-    if (nitcfg == 1) { ro_ssiter = ro; ro_cl = ro_p1; }
-    else if (implicit) { ro_ssiter = ro_p1; ro_cl = ro_p1; }
-    else if (nitcfg % 2 == 0) { ro_ssiter = ro_p1; ro_cl = ro; }
-    else { ro_ssiter = ro; ro_cl = ro_p1; }
-    int sdm[6] = {1, k.ni, 1, k.nj, 1, k.nk};
-    int lamin = k.iflow == 2;
-    if (nitcfg == 1) {
-        if (implicit) {
-            Box b = {1 - k.nf, k.ni + k.nf, 1 - k.nf, k.nj + k.nf, 1 - k.nfk, k.nk + k.nfk};
-            launch_coe(k, ro_ssiter, first_it, k.dtloc ? 2 : 1, b, lamin, st);
-        } else {
-            Box b = {0, k.ni + 1, 0, k.nj + 1, 0, k.nk + 1};
-            launch_coe(k, ro_ssiter, first_it, 0, b, lamin, st);
-        }
+    memset(&r, 0, sizeof r);
+    r.z = k;
+    r.first_it = first_it; r.lamin = k.iflow == 2;
+    if (implicit) {
+        r.b = Box{1 - k.nf, k.ni + k.nf, 1 - k.nf, k.nj + k.nf, 1 - k.nfk, k.nk + k.nfk};
+        r.mode = k.dtloc ? 2 : 1;
+    } else {
+        r.b = Box{0, k.ni + 1, 0, k.nj + 1, 0, k.nk + 1};
+        r.mode = 0;
     }
-    // cptst3.for:114-119: CFL monitor at the first sub-iteration of a verification step
-    if (nitcfg == 1 && lssiter_verif) {
-        launch_cfl(k, ro_ssiter, z->norm_part, z->norm_blocks, z->norm_out + 10, st);
-        z->have_cfl = 1;
-    }
-    if (k.kflu == 2 && nitcfg == 1) launch_wiggle(k, ro_ssiter, st);
-    RhsArgs a;
-    memset(&a, 0, sizeof a);
+    RhsArgs& a = r.a;
     a.schedule = c->res_schedule;
     a.kcol_n = c->res_kcol_n;
     if (k.kflu == 5) {
         int rc = wall_corrections(z, a);
         if (rc) return rc;
     }
-    a.rop = ro_ssiter; a.rop_n = ro; a.rop_n1 = ro_m1;
+    a.rop = level_ssiter(z, nitcfg); a.rop_n = ro; a.rop_n1 = ro_m1;
     a.implicit = implicit; a.nitcfg = nitcfg;
     a.zero_init = (implicit || nitcfg == 1);
     a.coefH = 0.;
@@ -916,11 +910,46 @@ static int substep(fm_ctx* c, Zone* z, int nitcfg, int first_it, int lssiter_ver
     else { a.c1 = -1.5; a.c2 = 2.; a.c3 = -0.5; }
     if (nitcfg % 2 == 1) { a.rk_out = ro_p1; a.rk_in = ro; }
     else { a.rk_out = ro; a.rk_in = ro_p1; }
-    if (launch_residual(k, a, st)) return fail(FM_E_UNSUPPORTED, "no residual kernel for this scheme");
-    HIPCHK(hipGetLastError());
+    return FM_OK;
+}
+
+// the right-hand side is (about to be) written
+static void rhs_done(Zone* z) {
     z->dw_pending = 0;
-    if (!implicit) z->w_rows = nullptr;       // the stage update rewrites the state
+    if (z->k.itypcp > 1) z->w_rows = nullptr;       // the stage update rewrites the state
+}
+
+static int substep_rest(fm_ctx* c, Zone* z, int nitcfg, int lssiter_verif, int lexit_lu, int stop, LuArgs* defer);
+
+static int substep(fm_ctx* c, Zone* z, int nitcfg, int first_it, int lssiter_verif, int lexit_lu, int stop,
+                   LuArgs* defer = nullptr) {
+    KZ& k = z->k;
+    hipStream_t st = c->cur;
+    RhsZone r;
+    if (int rc = rhs_args(c, z, nitcfg, first_it, r)) return rc;
+    const double* ro_ssiter = r.a.rop;
+    if (nitcfg == 1) launch_coe(k, ro_ssiter, first_it, r.mode, r.b, r.lamin, st);
+    // cptst3.for:114-119: CFL monitor at the first sub-iteration of a verification step
+    if (nitcfg == 1 && lssiter_verif) {
+        launch_cfl(k, ro_ssiter, z->norm_part, z->norm_blocks, z->norm_out + 10, st);
+        z->have_cfl = 1;
+    }
+    if (k.kflu == 2 && nitcfg == 1) launch_wiggle(k, ro_ssiter, st);
+    if (launch_residual(k, r.a, st)) return fail(FM_E_UNSUPPORTED, "no residual kernel for this scheme");
+    HIPCHK(hipGetLastError());
+    rhs_done(z);
     if (stop == 1) return FM_OK;
+    return substep_rest(c, z, nitcfg, lssiter_verif, lexit_lu, stop, defer);
+}
+
+// a sub-iteration from its right-hand side on
+static int substep_rest(fm_ctx* c, Zone* z, int nitcfg, int lssiter_verif, int lexit_lu, int stop, LuArgs* defer) {
+    KZ& k = z->k;
+    hipStream_t st = c->cur;
+    const int implicit = k.itypcp <= 1;
+    double* ro_p1 = z->ro[2];
+    double* ro_ssiter = level_ssiter(z, nitcfg);
+    double* ro_cl = level_cl(z, nitcfg);
     if (implicit) {
         int shift_lu[6], lcorner = 1;
         bczone(c, z, 1, k.drodm, shift_lu, &lcorner);
@@ -1525,45 +1554,53 @@ static int side_join(fm_ctx* c, size_t ns) {
     return FM_OK;
 }
 
-// The edges and corners of several zones in one launch, after their physical boundary conditions
-// (per zone, gsdr3.cpp:436-439): a zone's edges and corners read only its own face ghosts.  A
-// captured step reads a table of its own (written once before its capture); otherwise the table
-// goes through a pinned buffer that the previous copy from it has released.
-static int coins_batched(fm_ctx* c, const std::vector<CoinsZone>& co, int nblk, fm_ctx::GraphEntry* ge,
-                         int nstep, bool capture) {
-    if (co.empty()) return FM_OK;
+// A table for a launch over several zones.  A captured step reads a table of its own (written once
+// before its capture); otherwise it goes through a pinned buffer that the previous copy from it has released.
+static int table_copy(fm_ctx* c, fm_ctx::Table& t, const void* data, size_t bytes, fm_ctx::GraphEntry* ge, long key,
+                      bool capture, void** out) {
     hipStream_t st = c->stream;
-    const size_t bytes = co.size() * sizeof(CoinsZone);
-    CoinsZone* d = nullptr;
+    void* d = nullptr;
     if (ge) {
-        const long key = -1L - nstep;
-        for (auto& t : ge->tabs) if (t.first == key) d = (CoinsZone*)t.second;
+        for (auto& q : ge->tabs) if (q.first == key) d = q.second;
         if (!d) {
-            if (capture) return fail(FM_E_HIP, "graph capture: corner table missing");
+            if (capture) return fail(FM_E_HIP, "graph capture: zone table missing");
             HIPCHK(hipMalloc(&d, bytes));
             ge->tabs.push_back({key, d});
         }
-        if (!capture) HIPCHK(hipMemcpy(d, co.data(), bytes, hipMemcpyHostToDevice));
+        if (!capture) HIPCHK(hipMemcpy(d, data, bytes, hipMemcpyHostToDevice));
     } else {
-        if ((int)co.size() > c->co_cap) {
+        if (bytes > t.cap) {
             HIPCHK(hipStreamSynchronize(st));
-            if (c->co_tab) HIPCHK(hipFree(c->co_tab));
+            if (t.dev) HIPCHK(hipFree(t.dev));
+            t.dev = nullptr; t.cap = 0;
             for (int q = 0; q < 2; q++) {
-                if (c->co_host[q]) HIPCHK(hipHostFree(c->co_host[q]));
-                HIPCHK(hipHostMalloc(&c->co_host[q], bytes));
-                if (!c->co_ev[q]) HIPCHK(hipEventCreateWithFlags(&c->co_ev[q], hipEventDisableTiming));
+                if (t.host[q]) HIPCHK(hipHostFree(t.host[q]));
+                t.host[q] = nullptr;
+                HIPCHK(hipHostMalloc(&t.host[q], bytes));
+                if (!t.ev[q]) HIPCHK(hipEventCreateWithFlags(&t.ev[q], (unsigned)hipEventDisableTiming));
             }
-            HIPCHK(hipMalloc(&c->co_tab, bytes));
-            c->co_cap = (int)co.size();
+            HIPCHK(hipMalloc(&t.dev, bytes));
+            t.cap = bytes;
         }
-        int q = c->co_slot; c->co_slot ^= 1;
-        HIPCHK(hipEventSynchronize(c->co_ev[q]));
-        memcpy(c->co_host[q], co.data(), bytes);
-        HIPCHK(hipMemcpyAsync(c->co_tab, c->co_host[q], bytes, hipMemcpyHostToDevice, st));
-        HIPCHK(hipEventRecord(c->co_ev[q], st));
-        d = c->co_tab;
+        int q = t.slot; t.slot ^= 1;
+        HIPCHK(hipEventSynchronize(t.ev[q]));
+        memcpy(t.host[q], data, bytes);
+        HIPCHK(hipMemcpyAsync(t.dev, t.host[q], bytes, hipMemcpyHostToDevice, st));
+        HIPCHK(hipEventRecord(t.ev[q], st));
+        d = t.dev;
     }
-    launch_coins_list(d, (int)co.size(), nblk, st);
+    *out = d;
+    return FM_OK;
+}
+
+// The edges and corners of several zones in one launch, after their physical boundary conditions
+// (per zone, gsdr3.cpp:436-439): a zone's edges and corners read only its own face ghosts.
+static int coins_batched(fm_ctx* c, const std::vector<CoinsZone>& co, int nblk, fm_ctx::GraphEntry* ge,
+                         int nstep, bool capture) {
+    if (co.empty()) return FM_OK;
+    void* d;
+    if (int rc = table_copy(c, c->co_tab, co.data(), co.size() * sizeof(CoinsZone), ge, -1L - nstep, capture, &d)) return rc;
+    launch_coins_list((const CoinsZone*)d, (int)co.size(), nblk, c->stream);
     HIPCHK(hipGetLastError());
     return FM_OK;
 }
@@ -1587,10 +1624,37 @@ static int time_step(fm_ctx* c, int first_it, int verif, int n0, int n1, fm_ctx:
         int any = 0;
         std::vector<Zone*> bz;
         std::vector<LuArgs> bl;
-        if (ns) { if (int rc = side_fork(c, ns, capture)) return rc; }
+        // several zones: coefficients and residuals of those that can in one launch each, and streams for
+        // the rest of the sub-iteration only if a zone has work of its own there
+        std::vector<RhsZone> rl;
+        std::vector<char> listed(nz, 0);
+        bool alone = false;
+        if (ns) {
+            for (size_t n = 0; n < nz; n++) {
+                Zone* z = c->zones[n];
+                const bool implicit = z->k.itypcp <= 1;
+                if (implicit && nstep == z->k.nssiter && !verif) continue;
+                RhsZone r;
+                if (!verif) {
+                    if (int rc = rhs_args(c, z, nstep, first_it, r)) return rc;
+                    listed[n] = rhs_listed(r.z, r.a);
+                }
+                if (listed[n]) rl.push_back(r);
+                alone = alone || !listed[n] || (implicit && !(batch && z->bcs.empty()));
+            }
+            if (!rl.empty()) {
+                rhs_plan(rl);
+                void* d;
+                if (int rc = table_copy(c, c->rhs_tab, rl.data(), rl.size() * sizeof(RhsZone), ge, (1L << 32) + nstep,
+                                        capture, &d)) return rc;
+                launch_rhs_list(rl, (const RhsZone*)d, nstep == 1, c->stream);
+                HIPCHK(hipGetLastError());
+            }
+            if (alone) { if (int rc = side_fork(c, ns, capture)) return rc; }
+        }
         for (size_t n = 0; n < nz; n++) {
             Zone* z = c->zones[n];
-            if (ns) c->cur = c->side[n % ns];
+            c->cur = alone ? c->side[n % ns] : c->stream;
             int implicit = z->k.itypcp <= 1;
             int nssiter = z->k.nssiter;
             // souszones_list.cpp:44-84: a verification step computes residuals (and the
@@ -1604,13 +1668,16 @@ static int time_step(fm_ctx* c, int first_it, int verif, int n0, int n1, fm_ctx:
             }
             LuArgs la;
             la.i0 = 1; la.i1 = 0;
-            int rc = substep(c, z, nstep, first_it, lssiter_verif, lexit_lu, 3, batch ? &la : nullptr);
+            if (listed[n]) rhs_done(z);
+            int rc = listed[n] ? substep_rest(c, z, nstep, lssiter_verif, lexit_lu, 3, batch ? &la : nullptr)
+                               : substep(c, z, nstep, first_it, lssiter_verif, lexit_lu, 3, batch ? &la : nullptr);
             if (rc) { c->cur = c->stream; return rc; }
             if (batch && implicit && lexit_lu == 0 && la.i1 >= la.i0) { bz.push_back(z); bl.push_back(la); }
             lexit[n] = lexit_lu;
             any |= lexit_lu == 0;
         }
-        if (ns) { if (int rc = side_join(c, ns)) return rc; }
+        c->cur = c->stream;
+        if (alone) { if (int rc = side_join(c, ns)) return rc; }
         if (!bz.empty()) {
             int rc = lu_batched(c, bz, bl, ge, nstep, capture);
             if (rc) return rc;
@@ -1621,20 +1688,25 @@ static int time_step(fm_ctx* c, int first_it, int verif, int n0, int n1, fm_ctx:
         if (ns) {
             // several zones: their physical boundary conditions side by side, then the edges and
             // corners of all of them in one launch
-            if (int rc2 = side_fork(c, ns, capture)) return rc2;
+            bool any_bc = false;
+            for (size_t n = 0; n < nz; n++) any_bc = any_bc || (lexit[n] == 0 && !c->zones[n]->bcs.empty());
+            if (any_bc) { if (int rc2 = side_fork(c, ns, capture)) return rc2; }
             std::vector<CoinsZone> co;
             int nblk = 0;
             for (size_t n = 0; n < nz; n++) {
                 if (lexit[n] != 0) continue;
                 Zone* z = c->zones[n];
-                c->cur = c->side[n % ns];
                 int shift[6];
-                bczone(c, z, 0, cl[n], shift, nullptr);
+                if (any_bc) {
+                    c->cur = c->side[n % ns];
+                    bczone(c, z, 0, cl[n], shift, nullptr);
+                }
                 const CoinsZone e = {z->k, cl[n], Box{1, z->k.ni, 1, z->k.nj, 1, z->k.nk}};
                 co.push_back(e);
                 nblk = std::max(nblk, coins_blocks(e.z, e.L));
             }
-            if (int rc2 = side_join(c, ns)) return rc2;
+            c->cur = c->stream;
+            if (any_bc) { if (int rc2 = side_join(c, ns)) return rc2; }
             if (int rc2 = coins_batched(c, co, nblk, ge, nstep, capture)) return rc2;
         } else {
             for (size_t n = 0; n < nz; n++)

@@ -1,5 +1,6 @@
 // Kernels of the FastS structured NS iteration for MI355X (gfx950).  One thread per cell
 // (or per ghost cell, per plane cell); i is the fastest, coalesced index everywhere.
+#include <algorithm>
 #include "fm_device.hpp"
 #include "fm_kernels.hpp"
 
@@ -98,11 +99,8 @@ __global__ void k_metric_cart(KZ z) {
 // tstb3c.for; tstb3_impli.for + dtloc.for).  mode: 0 explicit (mu on box, coe1 = DTC/vol on
 // the interior), 1 implicit global, 2 implicit local.
 template <bool CART>
-__global__ void k_coe(KZ z, const double* __restrict__ rop, int first_it, int mode, Box b, int lamin) {
-    int i = blockIdx.x * blockDim.x + threadIdx.x + b.i0;
-    int j = blockIdx.y * blockDim.y + threadIdx.y + b.j0;
-    int k = blockIdx.z + b.k0;
-    if (i > b.i1 || j > b.j1 || k > b.k1) return;
+__device__ __forceinline__ void coe_cell(const KZ& z, const double* __restrict__ rop, int first_it, int mode, int lamin,
+                                         int i, int j, int k) {
     long nd = z.nd, l = IDX(z, i, j, k);
     double T = rop[l + 4 * nd];
     double mu = 0.;
@@ -171,6 +169,45 @@ __global__ void k_coe(KZ z, const double* __restrict__ rop, int first_it, int mo
     }
     z.coe[l] = c1; z.coe[l + nd] = c2; z.coe[l + 2 * nd] = c3; z.coe[l + 3 * nd] = c4;
     z.coe[l + 4 * nd] = xid + c1 * (c2 + c3 + c4) * 0.5;
+}
+template <bool CART>
+__global__ void k_coe(KZ z, const double* __restrict__ rop, int first_it, int mode, Box b, int lamin) {
+    int i = blockIdx.x * blockDim.x + threadIdx.x + b.i0;
+    int j = blockIdx.y * blockDim.y + threadIdx.y + b.j0;
+    int k = blockIdx.z + b.k0;
+    if (i > b.i1 || j > b.j1 || k > b.k1) return;
+    coe_cell<CART>(z, rop, first_it, mode, lamin, i, j, k);
+}
+
+// Several zones in one launch: workgroups [zones[n].*first, zones[n + 1].*first) are zone n's. On streams
+// of their own the zones' kernels overlapped a few at a time, between a fork and a join: a step of eight
+// zones of 16 to 28 cells a side took 250 us, now 185; of 64 zones of 18 to 92 cells, whose kernels fill
+// the chip, 6.07 ms, now 5.95.
+// The table is read as constant memory: scalar loads, and pointers known to be to global memory (else they
+// would take the slower loads that may go to LDS as well).
+typedef const __attribute__((address_space(4))) RhsZone RhsTable;
+template <int RhsZone::* FIRST>
+__device__ __forceinline__ RhsTable* listed_zone(const RhsZone* zones, int nz, int block) {
+    RhsTable* t = (RhsTable*)(unsigned long)zones;
+    int lo = 0, hi = nz - 1;
+    while (lo < hi) {
+        const int m = (lo + hi + 1) / 2;
+        if (t[m].*FIRST <= block) lo = m; else hi = m - 1;
+    }
+    return t + lo;
+}
+template <bool CART>
+__global__ void __launch_bounds__(256) k_coe_list(const RhsZone* zones, int nz) {
+    RhsTable* t = listed_zone<&RhsZone::coe_first>(zones, nz, blockIdx.x);
+    KZ z;
+    Box b;
+    __builtin_memcpy(&z, (const void*)&t->z, sizeof z);
+    __builtin_memcpy(&b, (const void*)&t->b, sizeof b);
+    const int n0 = b.i1 - b.i0 + 1, n1 = b.j1 - b.j0 + 1, n2 = b.k1 - b.k0 + 1;
+    const unsigned c = (unsigned)((int)blockIdx.x - t->coe_first) * 256 + threadIdx.x, r = c / n0, k = r / n1;
+    if (k >= (unsigned)n2) return;
+    coe_cell<CART>(z, t->a.rop, t->first_it, t->mode, t->lamin, b.i0 + (int)(c - r * n0),
+                   b.j0 + (int)(r - k * n1), b.k0 + (int)k);
 }
 
 // SENSEUR sensor (SENSOR/wiggle2001.for): interior cells plus the max faces
@@ -452,22 +489,40 @@ __device__ __forceinline__ long apart(long lt) {
     return lt;
 }
 
-template <int KFLU, int SLOPE, bool LAMIN, bool CART>
-__global__ void __launch_bounds__(64 * kPlaneRows) __attribute__((amdgpu_waves_per_eu(2))) k_residual_planes(KZ z, RhsArgs a, int kcol) {
+// Consecutive workgroups go to the eight XCDs in turn; on 3dcart this gives XCD c the c-th of eight
+// near-equal ranges of workgroups, so that the rows two neighbours share are in its L2 (256^3 1152 -> 1143
+// us, 161 x 97 x 75 108 -> 103; curvilinear zones, whose metric fills it, lose: 513 x 257 x 65 1819 -> 2062)
+__device__ __forceinline__ int by_xcd(int id, int n) {
+    const int c = id % 8, per = n / 8, rem = n % 8;
+    return c * per + (c < rem ? c : rem) + id / 8;
+}
+
+// (LIST: the workgroups of several zones, z, a and kcol from the table; a zone's start at a multiple of
+// eight, so that their XCDs are those of a launch of its own.  One kernel, not a body with two callers: the
+// compiler spills what it inlines from there.)
+template <int KFLU, int SLOPE, bool LAMIN, bool CART, bool LIST>
+__global__ void __launch_bounds__(64 * kPlaneRows) __attribute__((amdgpu_waves_per_eu(2)))
+k_residual_planes(KZ z, RhsArgs a, int kcol, const RhsZone* zones, int nz) {
+    int bx = blockIdx.x, by = blockIdx.y;
+    if (LIST) {
+        RhsTable* t = listed_zone<&RhsZone::res_first>(zones, nz, blockIdx.x);
+        const int ngx = t->ngx, n = ngx * t->ngy, id = (int)blockIdx.x - t->res_first;
+        if (id >= n) return;
+        const int q = CART ? by_xcd(id, n) : id;
+        by = __builtin_amdgcn_readfirstlane(q / ngx); bx = q - by * ngx;
+        __builtin_memcpy(&z, (const void*)&t->z, sizeof z);
+        a.rop = t->a.rop; a.rop_n = t->a.rop_n; a.rop_n1 = t->a.rop_n1; a.rk_in = t->a.rk_in; a.rk_out = t->a.rk_out;
+        a.zero_init = t->a.zero_init; a.coefH = t->a.coefH; a.coefW = t->a.coefW;
+        a.implicit = t->a.implicit; a.nitcfg = t->a.nitcfg; a.c1 = t->a.c1; a.c2 = t->a.c2; a.c3 = t->a.c3;
+        kcol = t->kcol;           // (zones with corrected wall fluxes are launched by themselves)
+    } else if (CART) {
+        const int q = by_xcd(bx + gridDim.x * by, gridDim.x * gridDim.y);
+        by = q / gridDim.x; bx = q % gridDim.x;
+    }
     constexpr int NA = LAMIN ? 6 : 5, PLANE = NA * kPlaneTile * 64;
     __shared__ double P[3 * PLANE + 4];              // (the first and last lanes read two places out)
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
     const int nx = (z.nj + kPlaneRows - 1) / kPlaneRows * z.nit;
-    int bx = blockIdx.x, by = blockIdx.y;
-    if (CART) {
-        // consecutive workgroups go to the eight XCDs in turn; this gives XCD c the c-th of eight
-        // near-equal ranges of workgroups, so that the rows two neighbours share are in its L2 (256^3
-        // 1152 -> 1143 us, 161 x 97 x 75 108 -> 103; curvilinear zones, whose metric fills it, lose:
-        // 513 x 257 x 65 1819 -> 2062)
-        const int n = gridDim.x * gridDim.y, id = bx + gridDim.x * by, c = id % 8, per = n / 8, rem = n % 8;
-        const int q = c * per + (c < rem ? c : rem) + id / 8;
-        by = q / gridDim.x; bx = q % gridDim.x;
-    }
     const int x0 = bx * kPlaneCells + lane - 2, x = x0 < 0 ? 0 : x0 < nx ? x0 : nx - 1;
     const int g = x / z.nit, i = x - g * z.nit - 1, j0 = g * kPlaneRows + w + 1, j = j0 < z.nj ? j0 : z.nj;
     const bool own = lane >= 2 && lane < 2 + kPlaneCells && x0 < nx && i >= 1 && i <= z.ni && j0 <= z.nj;
@@ -556,7 +611,7 @@ __global__ void __launch_bounds__(64 * kPlaneRows) __attribute__((amdgpu_waves_p
             for (int e = 0; e < 5; e++) acc[e] = acc[e] - fk[e];
         }
         if (own) {
-            if (KFLU == 5 && a.ncorr > 0) wall_correction<SLOPE, CART>(f, z, rop, a, i, j, k, acc);
+            if (KFLU == 5 && !LIST && a.ncorr > 0) wall_correction<SLOPE, CART>(f, z, rop, a, i, j, k, acc);
             if (jn) {
 #pragma unroll
                 for (int e = 0; e < 5; e++) acc[e] = acc[e] - flu[e];
@@ -1135,12 +1190,18 @@ static void res_lc(const KZ& z, const RhsArgs& a, bool lamin, dim3 g, hipStream_
     }
 }
 
+// workgroups of a level of planes
+static int planes_blocks(const KZ& z) {
+    const int nx = (z.nj + kPlaneRows - 1) / kPlaneRows * z.nit;
+    return (nx + kPlaneCells - 1) / kPlaneCells;
+}
+
 template <int KFLU, int SLOPE>
 static void res_planes(const KZ& z, const RhsArgs& a, bool lamin, hipStream_t st) {
     // cells up k per workgroup: two workgroups fit a CU, so they run in rounds of 2 x 256, each round as
     // long as the 4 n face fluxes of its cells, the k face under the first one and the first planes (about
     // two faces' time); of the even cuts of nk, the one whose rounds take least
-    const int nx = (z.nj + kPlaneRows - 1) / kPlaneRows * z.nit, nb = (nx + kPlaneCells - 1) / kPlaneCells;
+    const int nb = planes_blocks(z);
     int n = a.kcol_n > 0 ? a.kcol_n : z.nk;
     long best = -1;
     for (int cuts = 1; a.kcol_n <= 0 && cuts <= z.nk; cuts++) {
@@ -1151,24 +1212,28 @@ static void res_planes(const KZ& z, const RhsArgs& a, bool lamin, hipStream_t st
     }
     dim3 g(nb, (z.nk + n - 1) / n), b(64 * kPlaneRows);
     if (lamin) {
-        if (z.typ == 2) hipLaunchKernelGGL((k_residual_planes<KFLU, SLOPE, true, true>), g, b, 0, st, z, a, n);
-        else hipLaunchKernelGGL((k_residual_planes<KFLU, SLOPE, true, false>), g, b, 0, st, z, a, n);
+        if (z.typ == 2) hipLaunchKernelGGL((k_residual_planes<KFLU, SLOPE, true, true, false>), g, b, 0, st, z, a, n, nullptr, 0);
+        else hipLaunchKernelGGL((k_residual_planes<KFLU, SLOPE, true, false, false>), g, b, 0, st, z, a, n, nullptr, 0);
     } else {
-        if (z.typ == 2) hipLaunchKernelGGL((k_residual_planes<KFLU, SLOPE, false, true>), g, b, 0, st, z, a, n);
-        else hipLaunchKernelGGL((k_residual_planes<KFLU, SLOPE, false, false>), g, b, 0, st, z, a, n);
+        if (z.typ == 2) hipLaunchKernelGGL((k_residual_planes<KFLU, SLOPE, false, true, false>), g, b, 0, st, z, a, n, nullptr, 0);
+        else hipLaunchKernelGGL((k_residual_planes<KFLU, SLOPE, false, false, false>), g, b, 0, st, z, a, n, nullptr, 0);
     }
+}
+
+static bool res_cells(const KZ& z, const RhsArgs& a) {
+    const dim3 g((z.ni + 63) / 64, (z.nj + 3) / 4, z.nk);
+    // The planes are faster but for Cartesian Euler zones of one round of workgroups, whose few operations
+    // a cell do not pay for the planes' barriers: cells / planes at 32 x 24 x 20 7.6 / 8.0 us (Roe 11.1 /
+    // 11.5), 48^3 15.3 / 15.2, 64^3 21.4 / 23.0, 80^3 53 / 34
+    return a.schedule == RES_CELLS ||
+           (a.schedule == RES_AUTO && z.iflow != 2 && z.typ == 2 && (long)g.x * g.y * g.z <= 1024);
 }
 
 template <int KFLU, int SLOPE>
 static void res_scheme(const KZ& z, const RhsArgs& a, hipStream_t st) {
     const bool lamin = z.iflow == 2;
     const dim3 g((z.ni + 63) / 64, (z.nj + 3) / 4, z.nk);
-    // The planes are faster but for Cartesian Euler zones of one round of workgroups, whose few operations
-    // a cell do not pay for the planes' barriers: cells / planes at 32 x 24 x 20 7.6 / 8.0 us (Roe 11.1 /
-    // 11.5), 48^3 15.3 / 15.2, 64^3 21.4 / 23.0, 80^3 53 / 34
-    const bool cells = a.schedule == RES_CELLS ||
-                       (a.schedule == RES_AUTO && !lamin && z.typ == 2 && (long)g.x * g.y * g.z <= 1024);
-    if (cells) res_lc<KFLU, SLOPE>(z, a, lamin, g, st);
+    if (res_cells(z, a)) res_lc<KFLU, SLOPE>(z, a, lamin, g, st);
     else res_planes<KFLU, SLOPE>(z, a, lamin, st);
 }
 
@@ -1182,6 +1247,82 @@ int launch_residual(const KZ& z, const RhsArgs& a, hipStream_t st) {
     else if (z.kflu == 2 && z.slope == 2) res_scheme<2, 2>(z, a, st);
     else return -1;
     return 0;
+}
+
+// Zones whose coefficients and residual can go into a list: those that run the planes, with no sensor
+// between the two and no corrected wall flux (whose table is indexed at run time).
+bool rhs_listed(const KZ& z, const RhsArgs& a) {
+    const bool scheme = z.kflu == 5 ? z.slope >= 1 && z.slope <= 3 : z.kflu == 1 && z.slope == 2;
+    return scheme && a.ncorr == 0 && !res_cells(z, a);
+}
+
+static int rhs_kind(const RhsZone& t) {
+    return ((t.z.kflu == 5 ? t.z.slope : 0) * 2 + (t.z.iflow == 2)) * 2 + (t.z.typ == 2);
+}
+
+// Orders the zones by kernel, and gives each its workgroups: of the residual, columns of as many cells up k
+// (within a zone even cuts) as take the rounds of all zones of the kernel the least time, by the model of
+// one zone's.
+void rhs_plan(std::vector<RhsZone>& l) {
+    std::stable_sort(l.begin(), l.end(), [](const RhsZone& a, const RhsZone& b) { return rhs_kind(a) < rhs_kind(b); });
+    for (size_t p = 0, e; p < l.size(); p = e) {
+        int nk = 0;
+        for (e = p; e < l.size() && rhs_kind(l[e]) == rhs_kind(l[p]); e++) nk = std::max(nk, l[e].z.nk);
+        auto blocks = [&](int m) {
+            long b = 0;
+            for (size_t q = p; q < e; q++) b += (long)planes_blocks(l[q].z) * ((l[q].z.nk + m - 1) / m);
+            return b;
+        };
+        int n = l[p].a.kcol_n;
+        long best = -1;
+        for (int m = 1; l[p].a.kcol_n <= 0 && m <= nk; m++) {
+            const long t = (blocks(m) + kPlaneSlots - 1) / kPlaneSlots * (4 * m + 3);
+            if (best < 0 || t < best) { best = t; n = m; }
+        }
+        int coe = 0, res = 0;
+        for (size_t q = p; q < e; q++) {
+            RhsZone& t = l[q];
+            const Box& b = t.b;
+            const int cuts = (t.z.nk + n - 1) / n;
+            t.kcol = l[p].a.kcol_n > 0 ? n : (t.z.nk + cuts - 1) / cuts;
+            t.ngx = planes_blocks(t.z); t.ngy = (t.z.nk + t.kcol - 1) / t.kcol;
+            t.coe_first = coe; t.res_first = res;
+            coe += (int)(((long)(b.i1 - b.i0 + 1) * (b.j1 - b.j0 + 1) * (b.k1 - b.k0 + 1) + 255) / 256);
+            res += (t.ngx * t.ngy + 7) / 8 * 8;
+            t.coe_end = coe; t.res_end = res;
+        }
+    }
+}
+
+template <int KFLU, int SLOPE>
+static void rhs_list(const RhsZone& t, const RhsZone* d, int nz, int blocks, hipStream_t st) {
+    const dim3 g(blocks), b(64 * kPlaneRows);
+    if (t.z.iflow == 2) {
+        if (t.z.typ == 2) hipLaunchKernelGGL((k_residual_planes<KFLU, SLOPE, true, true, true>), g, b, 0, st, t.z, t.a, 0, d, nz);
+        else hipLaunchKernelGGL((k_residual_planes<KFLU, SLOPE, true, false, true>), g, b, 0, st, t.z, t.a, 0, d, nz);
+    } else {
+        if (t.z.typ == 2) hipLaunchKernelGGL((k_residual_planes<KFLU, SLOPE, false, true, true>), g, b, 0, st, t.z, t.a, 0, d, nz);
+        else hipLaunchKernelGGL((k_residual_planes<KFLU, SLOPE, false, false, true>), g, b, 0, st, t.z, t.a, 0, d, nz);
+    }
+}
+
+void launch_rhs_list(const std::vector<RhsZone>& l, const RhsZone* dev, bool coe, hipStream_t st) {
+    for (size_t p = 0, e; p < l.size(); p = e) {
+        for (e = p; e < l.size() && rhs_kind(l[e]) == rhs_kind(l[p]);) e++;
+        const RhsZone &t = l[p], &last = l[e - 1];
+        const int nz = (int)(e - p);
+        if (coe) {
+            if (t.z.typ == 2) hipLaunchKernelGGL(k_coe_list<true>, dim3(last.coe_end), dim3(256), 0, st, dev + p, nz);
+            else hipLaunchKernelGGL(k_coe_list<false>, dim3(last.coe_end), dim3(256), 0, st, dev + p, nz);
+        }
+        if (t.z.kflu == 5) {
+            if (t.z.slope == 1) rhs_list<5, 1>(t, dev + p, nz, last.res_end, st);
+            else if (t.z.slope == 2) rhs_list<5, 2>(t, dev + p, nz, last.res_end, st);
+            else rhs_list<5, 3>(t, dev + p, nz, last.res_end, st);
+        } else {
+            rhs_list<1, 2>(t, dev + p, nz, last.res_end, st);
+        }
+    }
 }
 
 // Conditions that can share a launch: each fills whole ghost layers next to its face from the cells

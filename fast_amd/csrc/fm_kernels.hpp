@@ -32,6 +32,20 @@ struct RhsArgs {
 };
 enum { RES_CELLS = 0, RES_FACES = 1, RES_KCOL = 2, RES_AUTO = 3 };
 
+// several zones' coefficients and residuals in one launch each: what a zone's own two launches take, and
+// the workgroups rhs_plan gives it (by kernel, from 0)
+struct RhsZone {
+    KZ z;
+    RhsArgs a;
+    Box b;                        // of the coefficients, with first_it, mode and lamin as launch_coe
+    int first_it, mode, lamin;
+    int kcol, ngx, ngy;           // the residual's columns and grid
+    int coe_first, coe_end, res_first, res_end;
+};
+bool rhs_listed(const KZ& z, const RhsArgs& a);
+void rhs_plan(std::vector<RhsZone>& l);
+void launch_rhs_list(const std::vector<RhsZone>& l, const RhsZone* dev, bool coe, hipStream_t st);
+
 struct LuWork;
 struct LuArgs {
     int i0, i1, j0, j1, k0, k1;   // LU range (shift_lu)
