@@ -475,8 +475,8 @@ __device__ __forceinline__ void face_flux_at(const FluxConst& f, const KZ& z, co
     }
     slope_state<SLOPE, D>(f, cell, qm, qp);
     inviscid_flux<KFLU, CART, D>(f, cell, tn, sn, qm, qp, flu);
-    if (LAMIN) {
-        if (CART) visc_cart<D>(f, cell, flu);
+    if constexpr (LAMIN) {
+        if constexpr (CART) visc_cart<D>(f, cell, flu);
         else visc_full<D>(f, z, cell, tn, flu);
     }
 }

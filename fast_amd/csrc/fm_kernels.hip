@@ -444,34 +444,45 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(FM_RES
 // 60 of 64 lanes with a cell of their own: the lanes lost are the ghosts and 4 a wave whatever ni is.
 // The workgroup walks kcol cells up k with the planes k - 1, k and k + 1 of its rows and of the two rows on
 // each side in LDS and plane k + 2 on its way in registers; a thread keeps the k face between two of
-// its cells.  Per cell: four faces, summed in the reference order.
+// its cells. Without viscous fluxes only the plane k is in LDS, the thread's column in registers (COLUMN).
+// Per cell: four faces, summed in the reference order; or (SHARE) three and a quarter, the j face above a
+// cell being the one under the row above, read from its wave, and the waves taking turns at the one above
+// the rows.
 //
 // Why: a 64-lane load of 8 bytes takes the CU's vector memory path 16 cycles whether or not it hits, an
 // LDS read 4.  k_residual's 153 loads a cell kept that path busy for 79 % of its time (256^3, AUSM+(P)
 // laminar; vector units 42 %), and on curvilinear zones, with ~380, the registers it held them in spilled.
-// Here a cell costs 12 loads for the planes and 22 for its own update, and four face fluxes instead of six
+// Here a cell costs 12 loads for the planes and 22 for its own update, and fewer face fluxes than six
 // (five for columns of cells).  us before (six faces on 3dcart, columns on 3dfull) and now, laminar:
-// AUSM+(P) 256^3 1778 -> 1143, 161 x 97 x 75 136 -> 80, 64^3 28 -> 29; SENSEUR 161 x 97 x 75 155 -> 78;
-// Roe o3 128^3 493 -> 230, minmod 667 -> 250; curvilinear AUSM+(P) 257 x 129 x 33 436 -> 242,
-// 513 x 257 x 65 3006 -> 1875, 80 x 50 x 20 98 -> 34, Roe 257 x 129 x 33 695 -> 275; Euler 192 x 180 x 168
-// 445 -> 340.  What bounds it now: instruction issue, at two waves a SIMD.
+// AUSM+(P) 256^3 1778 -> 1083, 161 x 97 x 75 136 -> 79, 64^3 28 -> 27; SENSEUR 161 x 97 x 75 155 -> 76;
+// Roe o3 128^3 493 -> 229, minmod 667 -> 245; curvilinear AUSM+(P) 257 x 129 x 33 436 -> 242,
+// 513 x 257 x 65 3006 -> 1878, 80 x 50 x 20 98 -> 34, Roe 257 x 129 x 33 695 -> 280; Euler 192 x 180 x 168
+// 445 -> 266 (the column in registers and three waves a SIMD: 340 before them).  Sharing j fluxes gives 3 to
+// 5 %: a quarter of the waves, in turn, still has four faces between two barriers.  On curvilinear
+// laminar zones it costs 16 %: what bounds them is the latency of the metric, some 45 loads a face that
+// the caches hold little of (waves wait 73 % of their time, vector units 30 %), so the longest chain
+// counts.  What bounds the others: instruction issue (75 %), at two waves a SIMD.
 constexpr int kPlaneRows = 4, kPlaneCells = 60, kPlaneTile = kPlaneRows + 4;
-constexpr int kPlaneSlots = 512;      // workgroups at work at once (two of 74 KB of LDS on each of 256 CUs)
 
 // what a face flux at (0, DJ0, DK0) from the thread's cell reads: state and viscosity from the planes
 // (two cells up k: the thread's own values on their way), the metric from memory at the lane's own i and
 // from the neighbouring lanes at i +- 1
-template <int DJ0, int DK0>
+template <int DJ0, int DK0, bool COLUMN, bool SHARE>
 struct PlaneCell {
     const KZ& z;
     const double* m1; const double* p0; const double* p1;     // planes k - 1, k, k + 1 at the thread's cell
     const double* up;                                         // plane k + 2, the thread's cell
+    // (COLUMN: m1 and p1 point to the thread's own values, all there is of the planes k - 1 and k + 1)
     long l, lt;
     template <int DI, int DJ, int DK> __device__ __forceinline__ double get(int e) const {
         constexpr int K = DK0 + DK;
         static_assert(K >= -1 && (K <= 1 || (K == 2 && DI == 0 && DJ0 + DJ == 0)), "outside the planes held");
+        static_assert(!COLUMN || K == 0 || (DI == 0 && DJ0 + DJ == 0), "outside the column");
         if (K == 2) return up[e];
-        return (K < 0 ? m1 : K > 0 ? p1 : p0)[(e * kPlaneTile + DJ0 + DJ) * 64 + DI];
+        if (COLUMN && K != 0) return K < 0 ? m1[e] : p1[e];
+        // (SHARE: viscosity is kept of the rows next to the workgroup's only)
+        static_assert(DJ0 + DJ >= -2 && DJ0 + DJ <= 2, "outside the rows held");
+        return (K < 0 ? m1 : K > 0 ? p1 : p0)[(e * kPlaneTile - (SHARE && e == 5) + DJ0 + DJ) * 64 + DI];
     }
     template <int DI, int DJ, int DK> __device__ __forceinline__ double q(int e) const { return get<DI, DJ, DK>(e); }
     template <int DI, int DJ, int DK> __device__ __forceinline__ double mu() const { return get<DI, DJ, DK>(5); }
@@ -480,6 +491,29 @@ struct PlaneCell {
         return from_lane<DI>(t[lt + (DJ0 + DJ) * z.mj + (DK0 + DK) * z.mk + m * z.ndm]);
     }
 };
+
+// what the k face above the cell before the next one reads where there is no viscous flux: the thread's own
+// column, and the metric at the lane's own place
+struct ColumnCell {
+    const KZ& z;
+    const double* c0; const double* c1; const double* c2; const double* c3;      // k - 1 to k + 2
+    long l, lt;
+    template <int DI, int DJ, int DK> __device__ __forceinline__ double q(int e) const {
+        static_assert(DI == 0 && DJ == 0 && DK >= -2 && DK <= 1, "outside the column");
+        return (DK == -2 ? c0 : DK == -1 ? c1 : DK == 0 ? c2 : c3)[e];
+    }
+    template <int DI, int DJ, int DK> __device__ __forceinline__ double mu() const { return 0.; }
+    __device__ __forceinline__ double wig(int d) const { return z.wig[l + z.inck + d * z.nd]; }
+    template <int DI, int DJ, int DK> __device__ __forceinline__ double met(const double* __restrict__ t, int m) const {
+        return from_lane<DI>(t[lt + DJ * z.mj + (1 + DK) * z.mk + m * z.ndm]);
+    }
+};
+
+// which kernels hand j fluxes between their waves: all but the curvilinear laminar ones
+template <bool LAMIN, bool CART> constexpr bool plane_share() { return CART || !LAMIN; }
+
+// waves a SIMD the registers are allocated for: 3 where they suffice without spills
+template <int KFLU, bool LAMIN> constexpr int plane_waves() { return LAMIN || KFLU == 5 ? 2 : 3; }
 
 // the metric index of another face: hides from the compiler that it equals the last face's, so that the
 // face vectors two faces share are read again (from the caches) rather than held in registers
@@ -501,7 +535,7 @@ __device__ __forceinline__ int by_xcd(int id, int n) {
 // eight, so that their XCDs are those of a launch of its own.  One kernel, not a body with two callers: the
 // compiler spills what it inlines from there.)
 template <int KFLU, int SLOPE, bool LAMIN, bool CART, bool LIST>
-__global__ void __launch_bounds__(64 * kPlaneRows) __attribute__((amdgpu_waves_per_eu(2)))
+__global__ void __launch_bounds__(64 * kPlaneRows) __attribute__((amdgpu_waves_per_eu(plane_waves<KFLU, LAMIN>())))
 k_residual_planes(KZ z, RhsArgs a, int kcol, const RhsZone* zones, int nz) {
     int bx = blockIdx.x, by = blockIdx.y;
     if (LIST) {
@@ -519,22 +553,27 @@ k_residual_planes(KZ z, RhsArgs a, int kcol, const RhsZone* zones, int nz) {
         const int q = by_xcd(bx + gridDim.x * by, gridDim.x * gridDim.y);
         by = q / gridDim.x; bx = q % gridDim.x;
     }
-    constexpr int NA = LAMIN ? 6 : 5, PLANE = NA * kPlaneTile * 64;
-    __shared__ double P[3 * PLANE + 4];              // (the first and last lanes read two places out)
-    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    constexpr bool COLUMN = !LAMIN, SHARE = plane_share<LAMIN, CART>();
+    constexpr int NA = LAMIN ? 6 : 5, PLANE = (NA * kPlaneTile - (LAMIN && SHARE ? 2 : 0)) * 64;
+    __shared__ double P[(COLUMN ? 1 : 3) * PLANE + 4];       // (the first and last lanes read two places out)
+    __shared__ double X[SHARE ? kPlaneRows : 1][5][64];      // fluxes of the j faces above the rows
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, ws = __builtin_amdgcn_readfirstlane(w);
     const int nx = (z.nj + kPlaneRows - 1) / kPlaneRows * z.nit;
     const int x0 = bx * kPlaneCells + lane - 2, x = x0 < 0 ? 0 : x0 < nx ? x0 : nx - 1;
-    const int g = x / z.nit, i = x - g * z.nit - 1, j0 = g * kPlaneRows + w + 1, j = j0 < z.nj ? j0 : z.nj;
+    const int g = x / z.nit, i = x - g * z.nit - 1, j0 = g * kPlaneRows + w + 1, j = j0 <= z.nj ? j0 : z.nj + 1;
     const bool own = lane >= 2 && lane < 2 + kPlaneCells && x0 < nx && i >= 1 && i <= z.ni && j0 <= z.nj;
     const int k0 = by * kcol + 1, k1 = k0 + kcol - 1 < z.nk ? k0 + kcol - 1 : z.nk;
     const double* __restrict__ rop = a.rop;
     const long nd = z.nd;
     const FluxConst f = flux_const(z);
     const bool jn = cb_next(j, z.cbj, z.nbj);
+    // from the thread's cell to the one above the workgroup's rows: cells, and rows of the tile
+    const int jx = g * kPlaneRows + kPlaneRows + 1, dj = (jx <= z.nj ? jx : z.nj + 1) - j;
+    const long lx = dj * z.incj, ltx = CART ? 0 : dj * z.mj;
     // the two rows this wave brings in: its own (row w + 2 of the tile) and one of the four around
     const int hr = w < 2 ? w : w + 4;
     auto row_j = [&](int r) { const int jr = g * kPlaneRows - 1 + r; return jr < z.nj + 2 ? jr : z.nj + 2; };
-    long lo = IDX(z, i, row_j(w + 2), k0 - 2), lh = IDX(z, i, row_j(hr), k0 - 2);
+    long lo = IDX(z, i, row_j(w + 2), k0 - 2), lh = IDX(z, i, row_j(hr), COLUMN ? k0 : k0 - 2);
     double vo[NA], vh[NA];
     auto fetch = [&]() {
 #pragma unroll
@@ -547,33 +586,59 @@ k_residual_planes(KZ z, RhsArgs a, int kcol, const RhsZone* zones, int nz) {
     auto keep = [&](double* p) {
 #pragma unroll
         for (int e = 0; e < NA; e++) {
-            p[2 + (e * kPlaneTile + w + 2) * 64 + lane] = vo[e];
-            p[2 + (e * kPlaneTile + hr) * 64 + lane] = vh[e];
+            p[2 + (e * kPlaneTile - (SHARE && e == 5) + w + 2) * 64 + lane] = vo[e];
+            if (!SHARE || e < 5 || (hr > 0 && hr < kPlaneTile - 1))
+                p[2 + (e * kPlaneTile - (SHARE && e == 5) + hr) * 64 + lane] = vh[e];
         }
     };
-    double *s0 = P, *s1 = P + PLANE, *s2 = P + 2 * PLANE;
-    fetch(); keep(s0);
-    fetch(); keep(s1);
-    fetch(); keep(s2);
-    fetch();
-    lds_barrier();
     // the k face under the first cell, from the cell before it, then cell by cell
     long l = IDX(z, i, j, k0 - 1), lt = CART ? 0 : MTR(z, i, j, k0 - 1);
     double fk[5];
     const int mine = 2 + (w + 2) * 64 + lane;
     const double *m1, *p0, *p1;
+    double *s0 = P, *s1 = P + PLANE, *s2 = P + 2 * PLANE;
+    double c0[COLUMN ? 5 : 1], c1[COLUMN ? 5 : 1], c2[COLUMN ? 5 : 1];
+    auto own_ahead = [&](double* v) {
+#pragma unroll
+        for (int e = 0; e < 5; e++) v[e] = rop[lo + e * nd];
+        lo += z.inck;
+    };
     auto planes = [&]() { m1 = s0 + mine; p0 = s1 + mine; p1 = s2 + mine; };
     auto advance = [&]() {
+        if constexpr (COLUMN) {
+#pragma unroll
+            for (int e = 0; e < 5; e++) {
+                c0[e] = c1[e]; c1[e] = c2[e]; c2[e] = vo[e];
+                P[2 + (e * kPlaneTile + w + 2) * 64 + lane] = c1[e];
+                P[2 + (e * kPlaneTile + hr) * 64 + lane] = vh[e];
+            }
+            fetch();
+            l += z.inck; lt += z.mk;
+        } else {
+            if constexpr (!SHARE) lds_barrier();
+            keep(s0);
+            fetch();
+            double* t = s0; s0 = s1; s1 = s2; s2 = t;
+            l += z.inck; lt += z.mk;
+        }
         lds_barrier();
-        keep(s0);
+        if constexpr (!COLUMN) planes();
+    };
+    if constexpr (COLUMN) {
+        m1 = c0; p0 = P + mine; p1 = c2;
+        own_ahead(c0); own_ahead(c1); own_ahead(c2);
         fetch();
-        double* t = s0; s0 = s1; s1 = s2; s2 = t;
-        l += z.inck; lt += z.mk;
+        face_flux_at<KFLU, SLOPE, LAMIN, CART, 2>(f, z, ColumnCell{z, c0, c1, c2, vo, l, lt}, fk);
+    } else {
+        fetch(); keep(s0);
+        fetch(); keep(s1);
+        fetch(); keep(s2);
+        fetch();
         lds_barrier();
         planes();
-    };
-    planes();
-    face_flux_at<KFLU, SLOPE, LAMIN, CART, 2>(f, z, PlaneCell<0, 1>{z, m1, p0, p1, vo, l, lt}, fk);
+        face_flux_at<KFLU, SLOPE, LAMIN, CART, 2>(f, z, PlaneCell<0, 1, COLUMN, SHARE>{z, m1, p0, p1, vo, l, lt}, fk);
+        if constexpr (SHARE) lds_barrier();
+    }
     for (int k = k0; k <= k1; k++) {
         advance();
         double flu[5], acc[5];
@@ -586,25 +651,62 @@ k_residual_planes(KZ z, RhsArgs a, int kcol, const RhsZone* zones, int nz) {
         }
 #pragma unroll
         for (int e = 0; e < 5; e++) acc[e] = acc[e] + fk[e];
+        // the j face under the cell; SHARE: handed to the row below, and one wave, another one each cell, also
+        // does the one above the rows (in a loop, so that there is one copy of the flux)
         // (what the faces of a cell share is read again, not held in registers)
-        __builtin_amdgcn_sched_barrier(0);
-        face_flux_at<KFLU, SLOPE, LAMIN, CART, 1>(f, z, PlaneCell<0, 0>{z, m1, p0, p1, vo, l, apart<CART>(lt)}, flu);
+        if constexpr (SHARE) {
+            int rows = 0;
+#pragma clang loop unroll(disable)
+            for (;;) {
+                __builtin_amdgcn_sched_barrier(0);
+                asm volatile("" : "+s"(rows));
+                const int o = rows * 64;
+                face_flux_at<KFLU, SLOPE, LAMIN, CART, 1>(
+                    f, z, PlaneCell<0, 0, COLUMN, SHARE>{z, COLUMN ? m1 : m1 + o, p0 + o, COLUMN ? p1 : p1 + o, vo, rows ? l + lx : l,
+                                                  apart<CART>(rows ? lt + ltx : lt)}, flu);
+                if (rows == 0) {
 #pragma unroll
-        for (int e = 0; e < 5; e++) acc[e] = acc[e] + flu[e];
+                    for (int e = 0; e < 5; e++) acc[e] = acc[e] + flu[e];
+                }
+                if (ws + rows > 0) {
+#pragma unroll
+                    for (int e = 0; e < 5; e++) X[ws + rows - 1][e][lane] = flu[e];
+                }
+                if (rows || ws != (k & (kPlaneRows - 1))) break;
+                rows = kPlaneRows - ws;
+            }
+        } else {
+            __builtin_amdgcn_sched_barrier(0);
+            face_flux_at<KFLU, SLOPE, LAMIN, CART, 1>(f, z, PlaneCell<0, 0, COLUMN, SHARE>{z, m1, p0, p1, vo, l, apart<CART>(lt)}, flu);
+#pragma unroll
+            for (int e = 0; e < 5; e++) acc[e] = acc[e] + flu[e];
+        }
         __builtin_amdgcn_sched_barrier(0);
-        face_flux_at<KFLU, SLOPE, LAMIN, CART, 0>(f, z, PlaneCell<0, 0>{z, m1, p0, p1, vo, l, apart<CART>(lt)}, flu);
+        face_flux_at<KFLU, SLOPE, LAMIN, CART, 0>(f, z, PlaneCell<0, 0, COLUMN, SHARE>{z, m1, p0, p1, vo, l, apart<CART>(lt)}, flu);
 #pragma unroll
         for (int e = 0; e < 5; e++) acc[e] = acc[e] + flu[e];
 #pragma unroll
         for (int e = 0; e < 5; e++) acc[e] = acc[e] - from_lane<1>(flu[e]);
         __builtin_amdgcn_sched_barrier(0);
-        face_flux_at<KFLU, SLOPE, LAMIN, CART, 1>(f, z, PlaneCell<1, 0>{z, m1, p0, p1, vo, l, apart<CART>(lt)}, flu);
-        if (!jn) {
+        if constexpr (!SHARE) {
+            face_flux_at<KFLU, SLOPE, LAMIN, CART, 1>(f, z, PlaneCell<1, 0, COLUMN, SHARE>{z, m1, p0, p1, vo, l, apart<CART>(lt)}, flu);
+            if (!jn) {
 #pragma unroll
-            for (int e = 0; e < 5; e++) acc[e] = acc[e] - flu[e];
+                for (int e = 0; e < 5; e++) acc[e] = acc[e] - flu[e];
+            }
+            __builtin_amdgcn_sched_barrier(0);
         }
-        __builtin_amdgcn_sched_barrier(0);
-        face_flux_at<KFLU, SLOPE, LAMIN, CART, 2>(f, z, PlaneCell<0, 1>{z, m1, p0, p1, vo, l, apart<CART>(lt)}, fk);
+        if constexpr (COLUMN) face_flux_at<KFLU, SLOPE, LAMIN, CART, 2>(f, z, ColumnCell{z, c0, c1, c2, vo, l, apart<CART>(lt)}, fk);
+        else face_flux_at<KFLU, SLOPE, LAMIN, CART, 2>(f, z, PlaneCell<0, 1, COLUMN, SHARE>{z, m1, p0, p1, vo, l, apart<CART>(lt)}, fk);
+        if constexpr (SHARE) {
+            lds_barrier();
+#pragma unroll
+            for (int e = 0; e < 5; e++) flu[e] = X[ws][e][lane];
+            if (!jn) {
+#pragma unroll
+                for (int e = 0; e < 5; e++) acc[e] = acc[e] - flu[e];
+            }
+        }
         const bool kn = cb_next(k, z.cbk, z.nbk);
         if (!kn) {
 #pragma unroll
@@ -1196,18 +1298,26 @@ static int planes_blocks(const KZ& z) {
     return (nx + kPlaneCells - 1) / kPlaneCells;
 }
 
+// time of nb workgroups of m cells up k: as many as fit the CUs (two, or three of three waves a SIMD) run in
+// rounds, each round as long as its 4 m face fluxes (3 1/4 m where the j fluxes are shared), the k face
+// under the first cell and the first planes (about two faces' time)
+static long planes_time(const KZ& z, long nb, int m) {
+    const bool lamin = z.iflow == 2, share = lamin ? (z.typ == 2 ? plane_share<true, true>() : plane_share<true, false>())
+                                                   : (z.typ == 2 ? plane_share<false, true>() : plane_share<false, false>());
+    const long slots = 256 * (z.kflu == 5 ? plane_waves<5, false>() : lamin ? plane_waves<1, true>() : plane_waves<1, false>());
+    return (nb + slots - 1) / slots * ((share ? 13 : 16) * m + 12);
+}
+
 template <int KFLU, int SLOPE>
 static void res_planes(const KZ& z, const RhsArgs& a, bool lamin, hipStream_t st) {
-    // cells up k per workgroup: two workgroups fit a CU, so they run in rounds of 2 x 256, each round as
-    // long as the 4 n face fluxes of its cells, the k face under the first one and the first planes (about
-    // two faces' time); of the even cuts of nk, the one whose rounds take least
+    // cells up k per workgroup: of the even cuts of nk, the one whose rounds take least
     const int nb = planes_blocks(z);
     int n = a.kcol_n > 0 ? a.kcol_n : z.nk;
     long best = -1;
     for (int cuts = 1; a.kcol_n <= 0 && cuts <= z.nk; cuts++) {
         const int m = (z.nk + cuts - 1) / cuts;
         if ((cuts - 1) * m >= z.nk) continue;          // (the same m as fewer cuts)
-        const long t = ((long)nb * cuts + kPlaneSlots - 1) / kPlaneSlots * (4 * m + 3);
+        const long t = planes_time(z, (long)nb * cuts, m);
         if (best < 0 || t < best) { best = t; n = m; }
     }
     dim3 g(nb, (z.nk + n - 1) / n), b(64 * kPlaneRows);
@@ -1220,20 +1330,13 @@ static void res_planes(const KZ& z, const RhsArgs& a, bool lamin, hipStream_t st
     }
 }
 
-static bool res_cells(const KZ& z, const RhsArgs& a) {
-    const dim3 g((z.ni + 63) / 64, (z.nj + 3) / 4, z.nk);
-    // The planes are faster but for Cartesian Euler zones of one round of workgroups, whose few operations
-    // a cell do not pay for the planes' barriers: cells / planes at 32 x 24 x 20 7.6 / 8.0 us (Roe 11.1 /
-    // 11.5), 48^3 15.3 / 15.2, 64^3 21.4 / 23.0, 80^3 53 / 34
-    return a.schedule == RES_CELLS ||
-           (a.schedule == RES_AUTO && z.iflow != 2 && z.typ == 2 && (long)g.x * g.y * g.z <= 1024);
-}
-
 template <int KFLU, int SLOPE>
 static void res_scheme(const KZ& z, const RhsArgs& a, hipStream_t st) {
     const bool lamin = z.iflow == 2;
     const dim3 g((z.ni + 63) / 64, (z.nj + 3) / 4, z.nk);
-    if (res_cells(z, a)) res_lc<KFLU, SLOPE>(z, a, lamin, g, st);
+    // (the planes are faster at every size measured, 16^3 to 256^3, but for Roe Euler zones of 260 000 cells,
+    // the same or 3 % slower)
+    if (a.schedule == RES_CELLS) res_lc<KFLU, SLOPE>(z, a, lamin, g, st);
     else res_planes<KFLU, SLOPE>(z, a, lamin, st);
 }
 
@@ -1253,7 +1356,7 @@ int launch_residual(const KZ& z, const RhsArgs& a, hipStream_t st) {
 // between the two and no corrected wall flux (whose table is indexed at run time).
 bool rhs_listed(const KZ& z, const RhsArgs& a) {
     const bool scheme = z.kflu == 5 ? z.slope >= 1 && z.slope <= 3 : z.kflu == 1 && z.slope == 2;
-    return scheme && a.ncorr == 0 && !res_cells(z, a);
+    return scheme && a.ncorr == 0 && a.schedule != RES_CELLS;
 }
 
 static int rhs_kind(const RhsZone& t) {
@@ -1276,7 +1379,7 @@ void rhs_plan(std::vector<RhsZone>& l) {
         int n = l[p].a.kcol_n;
         long best = -1;
         for (int m = 1; l[p].a.kcol_n <= 0 && m <= nk; m++) {
-            const long t = (blocks(m) + kPlaneSlots - 1) / kPlaneSlots * (4 * m + 3);
+            const long t = planes_time(l[p].z, blocks(m), m);
             if (best < 0 || t < best) { best = t; n = m; }
         }
         int coe = 0, res = 0;
