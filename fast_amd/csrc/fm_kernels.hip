@@ -1489,12 +1489,20 @@ void launch_coins_list(const CoinsZone* zones, int nz, int nblk, hipStream_t st)
     hipLaunchKernelGGL(k_coins_list, dim3((unsigned)nblk, 13, (unsigned)nz), dim3(256), 0, st, zones);
 }
 
+// Workgroups of a reduction that have a cell, of nblk: the others' results leave the total as it is, and the
+// second pass goes through them one by one (512 of them 16 us, the 60 of 32 x 24 x 20 cells 4).
+static int reduce_count(const KZ& z, int nblk) {
+    return (int)std::min((long)nblk, ((long)z.ni * z.nj * z.nk + 255) / 256);
+}
+
 void launch_norms(const KZ& z, const double* dr, double* part, int nblk, double* out, hipStream_t st) {
+    nblk = reduce_count(z, nblk);
     hipLaunchKernelGGL(k_norm_partial, dim3(nblk), dim3(256), 0, st, z, dr, part);
     hipLaunchKernelGGL(k_norm_final, dim3(1), dim3(kFinalThreads), 0, st, part, nblk, out);
 }
 
 void launch_cfl(const KZ& z, const double* rop, double* part, int nblk, double* out, hipStream_t st) {
+    nblk = reduce_count(z, nblk);
     hipLaunchKernelGGL(k_cfl_partial, dim3(nblk), dim3(256), 0, st, z, rop, part);
     hipLaunchKernelGGL(k_cfl_final, dim3(1), dim3(kFinalThreads), 0, st, part, nblk, out);
 }

@@ -2,7 +2,7 @@
 import numpy as np
 import pytest
 
-from fast_amd import cases
+from fast_amd import cases, params as P
 from tests import helpers as H
 from tests.test_gpu_parity import assert_same, ctxmod, orc, run_pair  # noqa: F401  (fixtures)
 
@@ -155,3 +155,16 @@ def test_zones_in_one_launch(ctxmod, mode):  # noqa: F811
         assert np.isfinite(together[1][n]).all()
         for s, one in enumerate(run([m])):
             assert np.array_equal(one[0], together[s][n], equal_nan=True), (n, s)
+
+
+@pytest.mark.parametrize("n", [(2, 2, 2), (4, 8, 8), (257, 3, 5), (64, 64, 32), (67, 52, 39)])
+def test_norm_blocks(ctxmod, orc, n):  # noqa: F811
+    """Residual norms of fewer cells than a block, of one block, of blocks and one cell over, of as many
+    blocks as there can be and of more cells than those hold at once."""
+    mk = lambda: cases.tgv_zone(n, H.numerics("ausmpred", "bdf"), perturb=0.02)
+    zo, zg, rdm, norms = run_pair(ctxmod, orc, mk, 1, stop=2)
+    r = rdm.reshape(-1, 2, 5, int(zo.param_int[P.NSSITER]))
+    dtc = zo.param_real[P.DTC]
+    # (positive terms summed in another order: at most their number times 2^-53 apart, taken at 1e-12)
+    np.testing.assert_allclose(norms[:5], np.sqrt(r[:, 0, :, 0].sum(axis=0) / np.prod(n)) / dtc, rtol=1e-12, atol=0)
+    assert np.array_equal(norms[5:], r[:, 1, :, 0].max(axis=0) / dtc)
