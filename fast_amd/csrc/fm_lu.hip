@@ -998,8 +998,14 @@ __device__ __forceinline__ void lu_copy_tile(int& t, int& y) {
     t = w / ny; y = w % ny;
 }
 
+// (the packs come before both sweeps and set their pencil counters back: [0] lower, [2] upper)
+__device__ __forceinline__ void lu_reset_counters(int* counter) {
+    if (blockIdx.x == 0 && blockIdx.y == 0 && blockIdx.z == 0 && threadIdx.x == 0) counter[0] = counter[2] = 0;
+}
+
 __global__ __launch_bounds__(256) void k_lu_pack(KZ z, LuArgs a, int ntj) {
     __shared__ double T[64][65];
+    lu_reset_counters(a.sync);
     // with a.w_ready the state rows hold the state already (arrays 5-9 skipped)
     const int f = a.w_ready && blockIdx.z >= 5 ? blockIdx.z + 5 : blockIdx.z;
     int t, y;
@@ -1010,8 +1016,10 @@ __global__ __launch_bounds__(256) void k_lu_pack(KZ z, LuArgs a, int ntj) {
 // The skewed copies of several zones: workgroup (w, y, c) packs the c-th array its zone needs
 // (as in k_lu_pack: the state rows are skipped with a.w_ready, the normal rows with a.n_ready) of
 // rows [64 y, 64 y + 64) of pencil work[w].
-__global__ __launch_bounds__(256) void k_lu_pack_list(const LuZone* __restrict__ zones, const LuWork* __restrict__ work) {
+__global__ __launch_bounds__(256) void k_lu_pack_list(const LuZone* __restrict__ zones, const LuWork* __restrict__ work,
+                                                       int* counter) {
     __shared__ double T[64][65];
+    lu_reset_counters(counter);
     const LuWork w = work[blockIdx.x];
     const KZ& z = zones[w.zone].z;
     const LuArgs& a = zones[w.zone].a;
@@ -1071,16 +1079,6 @@ __global__ __launch_bounds__(256) void k_lu_unpack_list(const LuZone* __restrict
     const int f = lu_unpack_first(a) + (int)blockIdx.z;
     if (r0 >= R || f >= lu_unpack_end(a)) return;
     lu_unpack_rows(z, a, ntj, w.bj + ntj * w.bk, r0, f, T);
-}
-
-// The pencil exchanges of several zones filled with the pending pattern (and the shared pencil
-// counter reset): workgroup (n, c) fills chunk c of zone n's exchange.
-__global__ __launch_bounds__(256) void k_lu_fill_list(const LuZone* __restrict__ zones, int* counter) {
-    const LuArgs& a = zones[blockIdx.x].a;
-    if (blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x == 0) *counter = 0;
-    const long n = lu_stream_exchange_size(a.i1 - a.i0 + 1, a.j1 - a.j0 + 1, a.k1 - a.k0 + 1);
-    for (long e = (long)blockIdx.y * blockDim.x + threadIdx.x; e < n; e += (long)gridDim.y * blockDim.x)
-        a.stx[e] = __longlong_as_double(kLuPending);
 }
 
 // LDS of a pencil, in doubles: the rows in flight (lu_ring() slots of lu_skf() arrays, rounded up to
@@ -1258,6 +1256,17 @@ __device__ __forceinline__ void lu_sweep_wave(const KZ& z, const LuArgs& a, cons
 #pragma unroll
                 for (int e = 0; e < 5; e++) pc.P[(5 * ROLE + e) * 64 + to] = p[e];
             }
+            if (ROLE == 0) {
+                // the products of this step were read from the exchange during the last one: their slots go
+                // back to the pending pattern, by the wave that hands none on (slots without a line
+                // hold it anyway)
+                const int m = LOWER ? s : pc.R - 8 - s;
+                if ((unsigned)m < (unsigned)(ni + 7) && L < 40) {
+                    lu_gdouble* back = pc.X + ((long)pc.tileid * (ni + 7) + m) * 40;
+                    lu_stg(back + L, __longlong_as_double(kLuPending));
+                    lu_stg(back + (long)pc.ntile * (ni + 7) * 40 + L, __longlong_as_double(kLuPending));
+                }
+            }
             if (ROLE > 0) {
                 const int m = LOWER ? s - 7 : pc.R - 1 - s;
                 if (put && pc.active(s)) {
@@ -1426,7 +1435,7 @@ __global__ void __launch_bounds__(kLuStThreads) __attribute__((amdgpu_waves_per_
     const int ntile = ntj * ntk;
     for (;;) {
         // (the waves have read the last ticket before the first step of its pencil)
-        if (threadIdx.x == 0) ticket = atomicAdd(a.sync, 1);
+        if (threadIdx.x == 0) ticket = atomicAdd(a.sync + (LOWER ? 0 : 2), 1);
         __syncthreads();
         const int t = __builtin_amdgcn_readfirstlane(ticket);
         if (t >= ntile) break;
@@ -1447,7 +1456,7 @@ k_lu_stream_list(const LuZone* __restrict__ zones, const LuWork* __restrict__ wo
     __shared__ __align__(16) double S[lu_lds_doubles<CART>()];
     __shared__ int ticket;
     for (;;) {
-        if (threadIdx.x == 0) ticket = atomicAdd(counter, 1);
+        if (threadIdx.x == 0) ticket = atomicAdd(counter + (LOWER ? 0 : 2), 1);
         __syncthreads();
         const int t = __builtin_amdgcn_readfirstlane(ticket);
         if (t >= nwork) break;
@@ -1536,14 +1545,14 @@ void fill_exchange(const LuArgs& a, long n, hipStream_t st) {
     hipLaunchKernelGGL(k_fill_lin, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, a.xch, n, kLuPending, a.sync);
 }
 
-// Streaming sweeps of a zone: the skewed copy of the inputs, then for each sweep the exchange filled
-// with the pending pattern (and the tile counter reset) and one launch with as many workgroups as
-// can be resident at once (at most one per pencil).
+// Streaming sweeps of a zone: the skewed copy of the inputs, then for each sweep one launch with as many
+// workgroups as can be resident at once (at most one per pencil).  The exchange holds the pending pattern
+// between sweeps: each step gives back the slots it was handed, 1 to 17 us of a sweep against a launch of 2
+// to 26 us each that filled it (128^3 the same in all, 256^3 34 us less, 32 x 24 x 20 8 us).
 template <bool CART>
 void stream(const KZ& z, const LuArgs& a, hipStream_t st) {
     int ni = a.i1 - a.i0 + 1, nj = a.j1 - a.j0 + 1, nk = a.k1 - a.k0 + 1;
     int ntj = (nj + 7) / 8, ntk = (nk + 7) / 8;
-    const long nx = lu_stream_exchange_size(ni, nj, nk);
     hipLaunchKernelGGL(k_lu_pack, dim3((unsigned)(ntj * ntk), (unsigned)((ni + 14 + 63) / 64), (unsigned)lu_pack_count(CART, a)),
                        dim3(256), 0, st, z, a, ntj);
     int cus = 0, dev = 0, per = 0;
@@ -1553,9 +1562,7 @@ void stream(const KZ& z, const LuArgs& a, hipStream_t st) {
         per = 1;
     long cap = (long)per * cus;
     unsigned grid = (unsigned)((long)ntj * ntk < cap ? (long)ntj * ntk : cap);
-    hipLaunchKernelGGL(k_fill_lin, dim3((unsigned)((nx + 255) / 256)), dim3(256), 0, st, a.stx, nx, kLuPending, a.sync);
     hipLaunchKernelGGL((k_lu_stream<CART, true>), dim3(grid), dim3(kLuStThreads), 0, st, z, a, ntj, ntk);
-    hipLaunchKernelGGL(k_fill_lin, dim3((unsigned)((nx + 255) / 256)), dim3(256), 0, st, a.stx, nx, kLuPending, a.sync);
     hipLaunchKernelGGL((k_lu_stream<CART, false>), dim3(grid), dim3(kLuStThreads), 0, st, z, a, ntj, ntk);
     // dW back only if asked (inside fm_compute it is copied once, after the last time step)
     const int f0 = lu_unpack_first(a), f1 = lu_unpack_end(a);
@@ -1658,9 +1665,8 @@ void lu_pencil_list(const std::vector<Box>& boxes, std::vector<LuWork>& work, in
             }
 }
 
-// Streaming LU-SGS of several zones of one mesh kind: the skewed copies, then for each sweep the
-// exchanges filled (and the pencil counter reset) and one launch over the pencil list, then the
-// results back.
+// Streaming LU-SGS of several zones of one mesh kind: the skewed copies, then for each sweep one launch
+// over the pencil list, then the results back.
 void launch_lu_stream_list(bool cart, const LuZone* zones, int nz, const LuWork* work, int nwork, int maxrb,
                            int npack, int nunpack, int* counter, hipStream_t st) {
     if (nwork <= 0 || nz <= 0) return;
@@ -1671,11 +1677,9 @@ void launch_lu_stream_list(bool cart, const LuZone* zones, int nz, const LuWork*
     if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, kfn, kLuStThreads, 0) != hipSuccess || per < 1) per = 1;
     const long cap = (long)per * cus;
     const unsigned grid = (unsigned)(nwork < cap ? nwork : cap);
-    if (npack > 0)
-        hipLaunchKernelGGL(k_lu_pack_list, dim3((unsigned)nwork, (unsigned)maxrb, (unsigned)npack), dim3(256), 0, st,
-                           zones, work);
+    hipLaunchKernelGGL(k_lu_pack_list, dim3((unsigned)nwork, (unsigned)maxrb, (unsigned)npack), dim3(256), 0, st,
+                       zones, work, counter);
     for (int lower = 1; lower >= 0; lower--) {
-        hipLaunchKernelGGL(k_lu_fill_list, dim3((unsigned)nz, 64), dim3(256), 0, st, zones, counter);
         if (cart) {
             if (lower) hipLaunchKernelGGL((k_lu_stream_list<true, true>), dim3(grid), dim3(kLuStThreads), 0, st, zones, work, nwork, counter);
             else hipLaunchKernelGGL((k_lu_stream_list<true, false>), dim3(grid), dim3(kLuStThreads), 0, st, zones, work, nwork, counter);
