@@ -33,7 +33,7 @@ HBM_PEAK_GBS = 8000.0
 BYTES_PER_CELL = {"coe": 88.0, "residual": 120.0, "lu": 240.0, "bc": 0.0, "iteration": 400.0}
 KERNELS = {"coe": "k_coe", "bc": "k_bcs",
            "residual": {"cells": "k_residual", "faces": "k_residual_planes", "kcol": "k_residual_planes",
-                        "auto": "k_residual_planes (planes of the state in LDS; small Euler zones k_residual)"},
+                        "auto": "k_residual_planes (planes of the state in LDS)"},
            "lu": {"blocks": "k_lu_block (lower + upper sweeps, one launch per block diagonal)",
                   "pipeline": "k_lu_pipe (lower + upper sweeps)",
                   "dataflow": "k_lu_flow (lower + upper sweeps, one launch each)",
@@ -510,7 +510,7 @@ def main():
     roofline = {"bound": "hbm", "kernel": kname, "achieved": round(achieved, 1),
                 "peak": HBM_PEAK_GBS, "unit": "GB/s", "frac": round(achieved / HBM_PEAK_GBS, 4),
                 "traffic": traffic_from_profiles(dom + "/" + (a.lu if dom == "lu" else
-                                                              "cells" if a.residual == "auto" else a.residual)),
+                                                              "cells" if a.residual == "cells" else "planes")),
                 "bytes_per_cell": BYTES_PER_CELL[dom],
                 "launch_ms": round(dom_ms, 4),
                 "phase_gbs": {k: round(BYTES_PER_CELL[k] * ncell / (v * 1e-3) / 1e9, 1)
