@@ -6,6 +6,7 @@
 #include <cstdio>
 #include <cstring>
 #include <algorithm>
+#include <atomic>
 #include <condition_variable>
 #include <cstdarg>
 #include <exception>
@@ -135,11 +136,16 @@ struct fm_ctx {
         // corners (key -1 - sub-iteration)
         std::vector<std::pair<long, void*>> tabs;
     };
+    // What calls of several threads on one context share: held from the first use of any of it to the last
+    // (a call that reads a field while another computes an effort, or two that read fields, at once).
+    std::recursive_mutex shared;
     // fields between host and device: pinned slots the copies go through (see link_copy)
     char* link_host[4]; hipEvent_t link_ev[4];
     double* work; size_t work_cap;      // device workspace of the adjoint and effort entry points
-    int lu_unchecked;                   // sweeps may have run since the error words were last read
     int* lu_flags;                      // pinned: the error words as read
+    // sweeps may have run since the error words were last read: set once a sweep is on the stream, and
+    // taken back before the words are read, so that no sweep goes unread
+    std::atomic<int> lu_unchecked;
     int graph_on;
     long graph_epoch;                   // bumped by anything a captured kernel argument depends on
     std::vector<GraphEntry*> graphs;
@@ -483,8 +489,11 @@ static hipError_t link_copy(fm_ctx* c, void* host, void* dev, size_t bytes, bool
     const size_t chunk = bytes < 4 * kLinkSlot ? kLinkHalf : kLinkSlot;
     const long n = (long)((bytes + chunk - 1) / chunk);
     int slots = 0;
-    if (bytes >= (up ? kLinkUp : kLinkDown))
+    std::unique_lock<std::recursive_mutex> hold(c->shared, std::defer_lock);
+    if (bytes >= (up ? kLinkUp : kLinkDown)) {
+        hold.lock();
         while (slots < 4 && slots < n && link_slot(c, slots)) slots++;
+    }
     std::vector<std::thread> th;
     std::mutex m;
     std::condition_variable cv;
@@ -558,13 +567,16 @@ static hipError_t link_copy(fm_ctx* c, void* host, void* dev, size_t bytes, bool
 }
 
 // Device workspace of one call: the context's own, grown as needed, up to kWorkKeep (an allocation and its
-// release took 51 us); larger ones go back with the call.  Calls of a context share its stream.
+// release took 51 us); larger ones go back with the call.  Calls of a context share its stream; those of other
+// threads wait for the workspace until this one has given it back.
 constexpr size_t kWorkKeep = (size_t)256 << 20;
 struct Work {
     double* p = nullptr;
     bool own = false;
+    std::unique_lock<std::recursive_mutex> hold;
     hipError_t get(fm_ctx* c, size_t bytes) {
         if (bytes > kWorkKeep) { own = true; return hipMalloc(&p, bytes); }
+        hold = std::unique_lock<std::recursive_mutex>(c->shared);
         if (c->work_cap < bytes) {
             if (c->work) (void)hipFree(c->work);
             c->work = nullptr; c->work_cap = 0;
@@ -986,8 +998,8 @@ static int substep_rest(fm_ctx* c, Zone* z, int nitcfg, int lssiter_verif, int l
             // (a batched zone: lu_batched sets the copies it skips, with its rows)
             lu_stream_flags(c, z, la);
             if (defer) { *defer = la; return FM_OK; }
-            c->lu_unchecked = 1;
             launch_lu(k, la, st);
+            c->lu_unchecked = 1;
             HIPCHK(hipGetLastError());
             lu_stream_after(z, la);
             if (la.out == z->ro_scratch) {
@@ -1003,11 +1015,20 @@ static int substep_rest(fm_ctx* c, Zone* z, int nitcfg, int lssiter_verif, int l
     return FM_OK;
 }
 
+// error words to be read (again) once the scope it stands in is left
+struct LuUnread {
+    fm_ctx* c;
+    explicit LuUnread(fm_ctx* c_) : c(c_) {}
+    ~LuUnread() { if (c) c->lu_unchecked = 1; }
+};
+
 // An LU sweep whose bounded waits gave up has produced garbage: report it.  The error words are read only
 // if sweeps may have run since they were last found clear, all of them before one wait (a wait for each of
 // 64 zones took 1.4 ms, at every field read).
 static int check_lu(fm_ctx* c) {
-    if (!c->lu_unchecked) return FM_OK;
+    std::lock_guard<std::recursive_mutex> hold(c->shared);
+    if (!c->lu_unchecked.exchange(0)) return FM_OK;
+    LuUnread unread(c);
     const size_t most = 1024, nz = c->zones.size();
     if (!c->lu_flags && hipHostMalloc((void**)&c->lu_flags, most * sizeof(int)) != hipSuccess) {
         c->lu_flags = nullptr;
@@ -1039,7 +1060,7 @@ static int check_lu(fm_ctx* c) {
             return fail(FM_E_HIP, "LU-SGS sweep timed out waiting for a neighbour tile or block");
         }
     }
-    c->lu_unchecked = 0;
+    unread.c = nullptr;
     return FM_OK;
 }
 
@@ -1393,7 +1414,7 @@ extern "C" int fm_apply_bc(fm_ctx* c, int zone, int level, int nstep) {
 // zones updated in place.  Same blocks and the same per-block work as the per-zone sweeps.
 static int lu_batched(fm_ctx* c, const std::vector<Zone*>& zs, const std::vector<LuArgs>& las,
                       fm_ctx::GraphEntry* ge = nullptr, int nstep = 0, bool capture = false) {
-    c->lu_unchecked = 1;
+    LuUnread unread(c);
     hipStream_t st = c->stream;
     // FP64 streaming: one launch per sweep over the pencils of all zones; FP64 dataflow: one launch
     // per sweep over the blocks of all zones, each zone with its own face exchange; otherwise (blocks
@@ -1774,7 +1795,7 @@ static int compute_steps(fm_ctx* c, int nitrun, int nstep_deb, int nstep_fin, in
                     if (e != hipSuccess) return fail(FM_E_HIP, "graph instantiate: %s", hipGetErrorString(e));
                     ge->state = 2;
                 }
-                c->lu_unchecked = 1;
+                LuUnread unread(c);
                 HIPCHK(hipGraphLaunch(ge->exec, c->stream));
                 // the host state a replayed step leaves is the one the eager step left
                 for (size_t n = 0; n < c->zones.size() && n < ge->dw_pending.size(); n++) {
@@ -1887,9 +1908,9 @@ extern "C" int fm_ctx_set_option(fm_ctx* c, int option, int value) {
         return FM_OK;
     }
     if (option == FM_OPT_LU_GIVE_UP) {
-        c->lu_unchecked = 1;
         // failure-handling test hook: set every zone's LU error word as a wait that gave up would
         if (value != 1) return fail(FM_E_ARG, "LU give-up %d", value);
+        LuUnread unread(c);
         HIPCHK(hipSetDevice(c->device));
         HIPCHK(hipStreamSynchronize(c->stream));
         int one = 1;
@@ -2029,8 +2050,8 @@ extern "C" int fm_time_phase(fm_ctx* c, int zone, int phase, int reps, float* ms
             if (launch_residual(k, a, st)) return fail(FM_E_UNSUPPORTED, "no residual kernel");
         } else if (phase == FM_PHASE_LU) {
             if (!implicit) return fail(FM_E_ARG, "LU phase needs an implicit zone");
-            c->lu_unchecked = 1;
             launch_lu(k, la, st);
+            c->lu_unchecked = 1;
         } else if (phase == FM_PHASE_BC) {
             int shift[6], sdm[6] = {1, k.ni, 1, k.nj, 1, k.nk};
             bczone(c, z, 0, z->ro_scratch, shift, nullptr);
