@@ -1030,6 +1030,7 @@ static int check_lu(fm_ctx* c) {
     if (!c->lu_unchecked.exchange(0)) return FM_OK;
     LuUnread unread(c);
     const size_t most = 1024, nz = c->zones.size();
+    long gave_up = 0;
     if (!c->lu_flags && hipHostMalloc((void**)&c->lu_flags, most * sizeof(int)) != hipSuccess) {
         c->lu_flags = nullptr;
         return fail(FM_E_HIP, "reading the LU error word failed");
@@ -1047,21 +1048,27 @@ static int check_lu(fm_ctx* c) {
         if (e != hipSuccess || e2 != hipSuccess) return fail(FM_E_HIP, "reading the LU error word failed");
         for (size_t n = n0; n < n1; n++) {
             if (!c->lu_flags[n - n0]) continue;
-            // a sweep that gave up may leave handed-over values in the exchanges
+            // A sweep that gave up may leave handed-over values in the exchanges, and while its word is
+            // set the zone's next sweeps give up as well: every such zone is put right before any is
+            // reported, so that what is computed next is right for all of them.
+            gave_up++;
             Zone* z = c->zones[n];
             const KZ& k = z->k;
             int zero = 0;
-            (void)hipMemcpy(z->lu_sync + 1, &zero, sizeof(int), hipMemcpyHostToDevice);
+            e = hipMemcpy(z->lu_sync + 1, &zero, sizeof(int), hipMemcpyHostToDevice);
             if (z->lu_stx)
                 fill_pending(z->lu_stx, lu_stream_exchange_size(k.ni + 2, k.nj + 2, k.nk + 2), c->stream);
             if (z->lu_fx)
                 fill_pending(z->lu_fx, lu_flow_exchange_size(k.typ == 2, k.ni + 2, k.nj + 2, k.nk + 2), c->stream);
-            (void)hipStreamSynchronize(c->stream);
-            return fail(FM_E_HIP, "LU-SGS sweep timed out waiting for a neighbour tile or block");
+            if (e != hipSuccess) return fail(FM_E_HIP, "clearing the LU error word failed");
         }
     }
     unread.c = nullptr;
-    return FM_OK;
+    if (gave_up == 0) return FM_OK;
+    HIPCHK(hipGetLastError());
+    HIPCHK(hipStreamSynchronize(c->stream));
+    return fail(FM_E_HIP, "LU-SGS sweep timed out waiting for a neighbour tile or block (%ld of %ld zones)", gave_up,
+                (long)nz);
 }
 
 extern "C" int fm_zone_substep(fm_ctx* c, int zone, int nitcfg, int nitrun, int first_it,

@@ -199,8 +199,9 @@ int fm_compute_timed(fm_ctx* ctx, int nitrun, int nstep_deb, int nstep_fin, int 
    each starts as soon as its three neighbour blocks have handed over their face products.  The
    waits are bounded: one that gives up sets an error word, the sweeps still run to their end
    (with wrong values), and the next call that waits for the stream -- fm_sync, fm_zone_substep,
-   fm_zone_get_field, fm_residual_norms, fm_compute_timed, fm_time_phase -- returns FM_E_HIP and
-   clears the word (fm_compute itself is asynchronous and returns FM_OK).  With several zones
+   fm_zone_get_field, fm_residual_norms, fm_compute_timed, fm_time_phase -- returns FM_E_HIP, once
+   for all zones, and clears their words and exchanges: the state is wrong, what is computed from a
+   state set again is right (fm_compute itself is asynchronous and returns FM_OK).  With several zones
    and FM_OPT_ZONE_BATCH on, the sweeps of all zones run as one dataflow launch per sweep. */
 #define FM_LU_DATAFLOW 2
 /* FM_LU_STREAM (default): one workgroup of six waves per pencil of 8 x 8 (j, k) lines sweeps the whole i
