@@ -471,6 +471,8 @@ static double* field_ptr(Zone* z, int field, long* n) {
 // link gives.  From the sizes on where it is faster (measured: 4 MB down 0.24 -> 0.20 ms, 300 MB 18.2 -> 6.8
 // ms; up 25 MB the same, 300 MB 11.0 -> 6.8 ms) the copy goes through four pinned slots of the context, up
 // to 4 MB at a time, two threads moving slots to or from the caller's array while others cross the link.
+// Pinned arrays go directly at every size: 58 GB/s (12 MB down 0.26 ms, 0.45 through the slots; 300 MB 6.0
+// and 7.4).
 constexpr size_t kLinkSlot = (size_t)4 << 20, kLinkHalf = (size_t)2 << 20;
 constexpr size_t kLinkDown = (size_t)4 << 20, kLinkUp = (size_t)32 << 20;
 constexpr int kLinkThreads = 2;
@@ -484,13 +486,21 @@ static bool link_slot(fm_ctx* c, int s) {
     return false;
 }
 
+// memory the runtime knows (pinned, managed or of a device), which the link reaches without help
+static bool known_memory(const void* p) {
+    hipPointerAttribute_t at;
+    if (hipPointerGetAttributes(&at, p) == hipSuccess) return at.type != hipMemoryTypeUnregistered;
+    (void)hipGetLastError();
+    return false;
+}
+
 static hipError_t link_copy(fm_ctx* c, void* host, void* dev, size_t bytes, bool up) {
     const hipMemcpyKind kind = up ? hipMemcpyHostToDevice : hipMemcpyDeviceToHost;
     const size_t chunk = bytes < 4 * kLinkSlot ? kLinkHalf : kLinkSlot;
     const long n = (long)((bytes + chunk - 1) / chunk);
     int slots = 0;
     std::unique_lock<std::recursive_mutex> hold(c->shared, std::defer_lock);
-    if (bytes >= (up ? kLinkUp : kLinkDown)) {
+    if (bytes >= (up ? kLinkUp : kLinkDown) && !known_memory(host)) {
         hold.lock();
         while (slots < 4 && slots < n && link_slot(c, slots)) slots++;
     }
