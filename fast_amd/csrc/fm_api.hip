@@ -141,6 +141,7 @@ struct fm_ctx {
     std::recursive_mutex shared;
     // fields between host and device: pinned slots the copies go through (see link_copy)
     char* link_host[4]; hipEvent_t link_ev[4];
+    size_t link_direct, faces_direct;   // bytes that went directly, to be paid for before slots are made
     double* work; size_t work_cap;      // device workspace of the adjoint and effort entry points
     int* lu_flags;                      // pinned: the error words as read
     // sweeps may have run since the error words were last read: set once a sweep is on the stream, and
@@ -187,6 +188,7 @@ extern "C" int fm_ctx_create(fm_ctx** out, int device) {
     c->lu_fp32 = 0;
     c->graph_on = 1;
     for (int q = 0; q < 4; q++) { c->link_host[q] = nullptr; c->link_ev[q] = nullptr; }
+    c->link_direct = c->faces_direct = 0;
     c->work = nullptr; c->work_cap = 0;
     c->lu_unchecked = 1; c->lu_flags = nullptr;
     c->cur = nullptr;
@@ -477,6 +479,12 @@ constexpr size_t kLinkSlot = (size_t)4 << 20, kLinkHalf = (size_t)2 << 20;
 constexpr size_t kLinkDown = (size_t)4 << 20, kLinkUp = (size_t)32 << 20;
 constexpr int kLinkThreads = 2;
 
+// The slots cost 0.1 to 0.2 ms a MB to make, what they save is 0.025 ms a MB (of the faces' values in slot 0:
+// 0.04): they are made once as many bytes have gone directly as pay for them, so that a program that reads a
+// field once does not pay more than it gains (12.6 MB read once: 0.8 ms, 2.1 to 2.7 if slots are made for it;
+// 33 MB 1.9 and 5.1; 4.4 MB 0.28 and 1.1 to 1.5).
+constexpr size_t kLinkPaid = (size_t)64 << 20, kFacesPaid = (size_t)12 << 20;
+
 static bool link_slot(fm_ctx* c, int s) {
     if (!c->link_ev[s] && hipEventCreateWithFlags(&c->link_ev[s], (unsigned)hipEventDisableTiming) != hipSuccess)
         c->link_ev[s] = nullptr;
@@ -484,6 +492,13 @@ static bool link_slot(fm_ctx* c, int s) {
     if (c->link_ev[s] && c->link_host[s]) return true;
     (void)hipGetLastError();
     return false;
+}
+
+// slot 0 for the values of a window's faces, by a call that holds the workspace; nullptr: an array of its own
+static double* faces_slot(fm_ctx* c, size_t bytes) {
+    if (bytes > kLinkSlot) return nullptr;
+    if (!c->link_host[0]) c->faces_direct += bytes;
+    return (c->link_host[0] || c->faces_direct >= kFacesPaid) && link_slot(c, 0) ? (double*)c->link_host[0] : nullptr;
 }
 
 // memory the runtime knows (pinned, managed or of a device), which the link reaches without help
@@ -502,7 +517,8 @@ static hipError_t link_copy(fm_ctx* c, void* host, void* dev, size_t bytes, bool
     std::unique_lock<std::recursive_mutex> hold(c->shared, std::defer_lock);
     if (bytes >= (up ? kLinkUp : kLinkDown) && !known_memory(host)) {
         hold.lock();
-        while (slots < 4 && slots < n && link_slot(c, slots)) slots++;
+        if (!c->link_host[1]) c->link_direct += bytes;
+        while (c->link_direct >= kLinkPaid && slots < 4 && slots < n && link_slot(c, slots)) slots++;
     }
     std::vector<std::thread> th;
     std::mutex m;
@@ -510,7 +526,7 @@ static hipError_t link_copy(fm_ctx* c, void* host, void* dev, size_t bytes, bool
     long issued = 0;                 // copies of chunks below this are on the stream
     hipError_t err = hipSuccess;
     // chunks handed over by the threads: filled (up) or emptied (down); both take them in turn
-    std::vector<char> moved(slots > 1 ? n : 0, 0);
+    std::vector<char> moved;
     auto size_of = [&](long i) { return std::min(chunk, bytes - (size_t)i * chunk); };
     auto work = [&](int w) {
         hipError_t e = hipSetDevice(c->device);
@@ -537,6 +553,7 @@ static hipError_t link_copy(fm_ctx* c, void* host, void* dev, size_t bytes, bool
     };
     if (slots > 1) {
         try {
+            moved.assign(n, 0);
             th.reserve(kLinkThreads);
             for (int w = 0; w < kLinkThreads; w++) th.emplace_back(work, w);
         } catch (const std::exception&) {
@@ -1129,7 +1146,7 @@ extern "C" int fm_wall_effort(fm_ctx* c, int zone, int level, int idir, const in
     // into a pinned slot where they fit one (the runtime's staging and a fresh host array took longer
     // than the kernel)
     std::vector<double> v;
-    double* h = bytes <= kLinkSlot && link_slot(c, 0) ? (double*)c->link_host[0] : nullptr;
+    double* h = faces_slot(c, bytes);
     if (!h) { v.resize((size_t)33 * nf); h = v.data(); }
     hipError_t e = hipMemcpyAsync(h, wk.p, bytes, hipMemcpyDeviceToHost, c->stream);
     if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
@@ -1211,7 +1228,7 @@ extern "C" int fm_dpj_dpw(fm_ctx* c, int zone, int level, int idir, const int* w
     a.cosa = cosa; a.sina = sina; a.surfinv = surfinv;
     a.rop = z->ro[level]; a.out = wk.p;
     std::vector<double> v;
-    double* h = bytes <= kLinkSlot && link_slot(c, 0) ? (double*)c->link_host[0] : nullptr;
+    double* h = faces_slot(c, bytes);
     if (!h) { v.resize(20 * nf); h = v.data(); }
     launch_dpj_dpw(k, a, c->stream);
     hipError_t e = hipGetLastError();

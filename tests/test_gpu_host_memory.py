@@ -28,3 +28,45 @@ def test_pinned_and_pageable_arrays(ctxmod, n):  # noqa: F811
             dst[:] = 0.0
             assert np.array_equal(ctx.get(0, ctxmod.FIELD_RO, dst), want)
     ctx.close()
+
+
+@pytest.mark.parametrize("moved", [0, 48, 80])
+def test_copies_before_and_after_the_slots(ctxmod, moved):  # noqa: F811
+    """Fields of 4 to 41 MB, and one below, written and read in a context that has moved that many MB
+    before: directly, from some copy on through the pinned slots, and through them from the start."""
+    sizes = [(3, 4, 5), (46, 46, 37), (46, 46, 38), (80, 80, 55), (80, 80, 56), (90, 90, 90), (90, 90, 91), (130, 97, 81)]
+    ctx = ctxmod.Context(0)
+    zs = [cases.tgv_zone(n, H.numerics("ausmpred", "explicit")) for n in sizes]
+    for z in zs:
+        ctx.add_zone(z)
+    step = zs[2].ro.nbytes
+    for _ in range(moved * 10**6 // step):
+        ctx.get(2, ctxmod.FIELD_RO, np.zeros_like(zs[2].ro))
+    rng = np.random.default_rng(6)
+    for q, z in enumerate(zs):
+        a = rng.random(z.ro.size)
+        ctx.set(q, ctxmod.FIELD_RO_M1, a)
+        assert np.array_equal(ctx.get(q, ctxmod.FIELD_RO_M1, np.zeros_like(a)), a), sizes[q]
+    ctx.close()
+
+
+@pytest.mark.parametrize("n", [(33, 8, 17), (257, 8, 33), (400, 8, 39), (410, 8, 39)])
+def test_efforts_before_and_after_the_slot(ctxmod, n):  # noqa: F811
+    """Wall efforts and wall gradients, again and again: the first through arrays of their own, later ones
+    through the pinned slot where the window's faces fit it (the last size is above)."""
+    z = cases.tgv_zone(n, H.numerics("ausmpred", "bdf"), perturb=0.02, flow="euler", bcs=H.INVISCID_J)
+    ctx = ctxmod.Context(0)
+    ctx.add_zone(z)
+    ctx.apply_bc(0, 0)
+    w = [1, n[0], 1, 1, 1, n[2]]
+
+    def both():
+        g = np.full(5 * z.nd, 3.0), np.full(5 * z.nd, -2.0)
+        ctx.dpj_dpw(0, 3, w, 0.9, 0.3, 0.5, *g)
+        return ctx.wall_effort(0, 3, w) + g
+
+    first = both()
+    for _ in range(12):
+        for a, b in zip(both(), first):
+            assert np.array_equal(a, b)
+    ctx.close()

@@ -43,6 +43,9 @@ def test_threads_share_a_context(ctxmod, n):  # noqa: F811
     for q, z in enumerate(zs):
         ctx.add_zone(z)
         ctx.apply_bc(q, 0)
+    # (the copies' pinned slots are made after 64 MB)
+    for _ in range(64 * 2**20 // zs[0].ro.nbytes + 1):
+        ctx.get(0, ctxmod.FIELD_RO, np.zeros_like(zs[0].ro))
     lam = [np.random.default_rng(q).standard_normal(5 * z.nd) for q, z in enumerate(zs)]
 
     def fields(q):
