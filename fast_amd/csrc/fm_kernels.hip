@@ -1343,9 +1343,13 @@ template <int KFLU, int SLOPE>
 static void res_scheme(const KZ& z, const RhsArgs& a, hipStream_t st) {
     const bool lamin = z.iflow == 2;
     const dim3 g((z.ni + 63) / 64, (z.nj + 3) / 4, z.nk);
-    // (the planes are faster at every size measured, 16^3 to 256^3, but for Roe Euler zones of 260 000 cells,
-    // the same or 3 % slower)
-    if (a.schedule == RES_CELLS) res_lc<KFLU, SLOPE>(z, a, lamin, g, st);
+    // RES_AUTO: the planes, but on zones of one row, and of two rows without viscous fluxes: three (two) of
+    // four waves of a group of rows would have no cell, where k_residual's leave at once.  us, planes and
+    // cells, 1024 x 1 x 128: AUSM+(P) laminar 35 and 20, Euler 27 and 14, Roe Euler 44 and 24, 3dfull AUSM+(P)
+    // 102 and 71; x 2 x: Euler 28 and 22, Roe 45 and 42, 3dfull 36 and 27, but laminar 35 and 35, 106 and 122;
+    // x 3 x: Euler 30 and 29, Roe 47 and 46.  (Small zones take 9 us either way.)
+    const bool few = z.nj == 1 || (z.nj == 2 && !lamin);
+    if (a.schedule == RES_CELLS || (a.schedule == RES_AUTO && few)) res_lc<KFLU, SLOPE>(z, a, lamin, g, st);
     else res_planes<KFLU, SLOPE>(z, a, lamin, st);
 }
 

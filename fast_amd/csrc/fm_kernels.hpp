@@ -23,7 +23,8 @@ struct RhsArgs {
     double coefH, coefW;    // RK coefficients
     int implicit, nitcfg;
     double c1, c2, c3;      // BDF coefficients
-    int schedule;           // RES_CELLS (six faces per cell from memory), else the planes in LDS
+    int schedule;           // RES_CELLS (six faces per cell from memory), else the planes in LDS (RES_AUTO:
+                            // by the zone's rows)
     int kcol_n;             // cells up k per workgroup of the planes (0: by the zone's size)
     int ncorr;              // Roe: wall faces whose Euler flux is replaced, in BC order
     WallCorr corr[kMaxWallCorr];

@@ -218,8 +218,9 @@ int fm_compute_timed(fm_ctx* ctx, int nitrun, int nstep_deb, int nstep_fin, int 
    sweeps run the dataflow schedule. */
 #define FM_LU_STREAM 3
 /* FM_OPT_RESIDUAL_SCHEDULE: FM_RES_CELLS evaluates the six faces of every cell from memory;
-   FM_RES_FACES, FM_RES_KCOL and FM_RES_AUTO (default) walk columns of cells up k with planes of the
-   state in LDS, three to four face fluxes per cell.  Same results bit for bit. */
+   FM_RES_FACES and FM_RES_KCOL walk columns of cells up k with planes of the state in LDS, three to
+   four face fluxes per cell; FM_RES_AUTO (default) does that too, but for a zone of one row j, or of
+   two without viscous fluxes, launched by itself.  Same results bit for bit. */
 #define FM_OPT_RESIDUAL_SCHEDULE 2
 #define FM_RES_CELLS 0
 #define FM_RES_AUTO 3
