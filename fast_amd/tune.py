@@ -2,10 +2,11 @@
 one of its zones and keeps the fastest, then the tile shapes of the schedules it kept.  Every
 choice gives the same results bit for bit, so it only affects speed.
 
-Knobs (fm_ctx_set_option): the residual schedule (six faces per cell / every face once /
-columns of cells up k) and the LU-SGS schedule (block diagonals / persistent pipelined tiles /
-dataflow blocks / streaming pencils); tile shapes: the k-column length of the column residual
-and the number of workgroups of a dataflow sweep."""
+Knobs (fm_ctx_set_option): the residual schedule (six faces per cell from memory / planes of the
+state in LDS, which "faces" and "kcol" both name) and the LU-SGS schedule (block diagonals /
+persistent pipelined tiles / dataflow blocks / streaming pencils); tile shapes: the cells up k per
+workgroup of the planes and the number of workgroups of a dataflow sweep.  The values a context
+starts with are among those of each tile shape, so that the shape kept is never the slower one."""
 from . import _lib
 
 KNOBS = (
@@ -16,11 +17,11 @@ KNOBS = (
       ("stream", _lib.LU_STREAM))),
 )
 
-# (tile knob, schedule knob, schedule it shapes, option, phase, values)
+# (tile knob, schedule knob, schedules it shapes, option, phase, values)
 TILES = (
-    ("kcol_n", "residual", "kcol", _lib.OPT_RES_KCOL_N, _lib.PHASE_RESIDUAL,
-     (("2", 2), ("4", 4), ("8", 8))),
-    ("flow_grid", "lu", "dataflow", _lib.OPT_LU_FLOW_GRID, _lib.PHASE_LU,
+    ("kcol_n", "residual", ("faces", "kcol"), _lib.OPT_RES_KCOL_N, _lib.PHASE_RESIDUAL,
+     (("auto", 0), ("2", 2), ("4", 4), ("8", 8))),
+    ("flow_grid", "lu", ("dataflow",), _lib.OPT_LU_FLOW_GRID, _lib.PHASE_LU,
      (("resident", 0), ("256", 256), ("384", 384))),
 )
 
@@ -43,7 +44,7 @@ def autotune(ctx, zone, reps=3, knobs=KNOBS, tiles=TILES):
     out = {}
     for name, opt, phase, values in knobs:
         out[name] = _pick(ctx, zone, opt, phase, values, reps)
-    for name, knob, sched, opt, phase, values in tiles:
-        if knob in out and out[knob][0] == sched:
+    for name, knob, scheds, opt, phase, values in tiles:
+        if knob in out and out[knob][0] in scheds:
             out[name] = _pick(ctx, zone, opt, phase, values, reps)
     return out

@@ -100,3 +100,33 @@ def test_autotune_shapes_the_schedule_it_kept():
     assert out["residual"][0] == "kcol" and out["kcol_n"][0] == "8"
     assert out["lu"][0] == "dataflow" and out["flow_grid"][0] == "256"
     assert c.opts[_lib.OPT_RES_KCOL_N] == 8 and c.opts[_lib.OPT_LU_FLOW_GRID] == 256
+
+
+@pytest.mark.parametrize("winner", ["faces", "kcol"])
+@pytest.mark.parametrize("best", [0, 2, 8])
+def test_autotune_can_leave_the_columns_to_the_zone(winner, best):
+    """The length chosen from the zone's size (0) is among those tried, under either name of the planes, so
+    that what the tuner ends on is never slower than what the context had."""
+    from fast_amd import tune, _lib
+
+    class FakeCtx:
+        def __init__(self):
+            self.opts = {_lib.OPT_RES_KCOL_N: 4, _lib.OPT_LU_FLOW_GRID: 0}
+
+        def set_option(self, opt, v):
+            self.opts[opt] = v
+
+        def time_phase(self, zone, phase, reps=1):
+            if phase != _lib.PHASE_RESIDUAL:
+                return 1.0
+            sched = self.opts[_lib.OPT_RESIDUAL_SCHEDULE]
+            if sched == _lib.RES_CELLS:
+                return 5.0
+            # (one kernel under two names: noise decides)
+            t = 2.0 if sched == (_lib.RES_FACES if winner == "faces" else _lib.RES_KCOL) else 2.01
+            return t - (0.5 if self.opts[_lib.OPT_RES_KCOL_N] == best else 0.0)
+
+    c = FakeCtx()
+    out = tune.autotune(c, 0)
+    assert out["residual"][0] == winner
+    assert c.opts[_lib.OPT_RES_KCOL_N] == best and out["kcol_n"][1]["auto" if best == 0 else str(best)] == min(out["kcol_n"][1].values())
