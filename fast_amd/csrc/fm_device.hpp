@@ -107,15 +107,21 @@ struct MemCell {
     long l, lt;
     __device__ __forceinline__ MemCell(const KZ& z_, const double* rop_, long l_, long lt_) : z(z_), rop(rop_), l(l_), lt(lt_) {}
     template <int DI, int DJ, int DK> __device__ __forceinline__ long at() const { return l + DI + DJ * z.incj + DK * z.inck; }
-    // (the neighbour's distance added last, as an index that is the same for all lanes: with one sum of
-    // indexes k_residual had 8 to 18 registers spilled on 3dcart laminar, 128^3 AUSM+(P) 251 us; so 209)
-    template <int DI, int DJ, int DK> __device__ __forceinline__ double q(int e) const {
-        return (rop + (l + e * z.nd))[DI + DJ * z.incj + DK * z.inck];
-    }
+    template <int DI, int DJ, int DK> __device__ __forceinline__ double q(int e) const { return rop[at<DI, DJ, DK>() + e * z.nd]; }
     template <int DI, int DJ, int DK> __device__ __forceinline__ double mu() const { return z.xmut[at<DI, DJ, DK>()]; }
     __device__ __forceinline__ double wig(int d) const { return z.wig[l + d * z.nd]; }
     template <int DI, int DJ, int DK> __device__ __forceinline__ double met(const double* __restrict__ t, int m) const {
         return t[lt + DI * z.mi + DJ * z.mj + DK * z.mk + m * z.ndm];
+    }
+};
+
+// the same with the neighbour's distance added last, as an index that is one for all lanes: k_residual on 3dcart,
+// where the one sum of indexes spills 8 to 18 registers of the laminar kernels (128^3 AUSM+(P) 251 us; so 209),
+// and SENSEUR Euler on 3dfull (128^3 225 us; so 203).  The others on 3dfull are 5 to 15 % faster with the sum.
+struct MemCellApart : MemCell {
+    using MemCell::MemCell;
+    template <int DI, int DJ, int DK> __device__ __forceinline__ double q(int e) const {
+        return (rop + (l + e * z.nd))[DI + DJ * z.incj + DK * z.inck];
     }
 };
 
@@ -485,10 +491,10 @@ __device__ __forceinline__ void face_flux_at(const FluxConst& f, const KZ& z, co
     }
 }
 // the same of cell (i, j, k), read from memory
-template <int KFLU, int SLOPE, bool LAMIN, bool CART, int D>
+template <int KFLU, int SLOPE, bool LAMIN, bool CART, int D, typename Cell = MemCell>
 __device__ __forceinline__ void face_flux(const FluxConst& f, const KZ& z, const double* __restrict__ rop,
                                           int i, int j, int k, double flu[5]) {
-    face_flux_at<KFLU, SLOPE, LAMIN, CART, D>(f, z, MemCell(z, rop, IDX(z, i, j, k), CART ? 0 : MTR(z, i, j, k)), flu);
+    face_flux_at<KFLU, SLOPE, LAMIN, CART, D>(f, z, Cell(z, rop, IDX(z, i, j, k), CART ? 0 : MTR(z, i, j, k)), flu);
 }
 
 }  // namespace fm

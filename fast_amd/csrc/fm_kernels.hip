@@ -1,6 +1,7 @@
 // Kernels of the FastS structured NS iteration for MI355X (gfx950).  One thread per cell
 // (or per ghost cell, per plane cell); i is the fastest, coalesced index everywhere.
 #include <algorithm>
+#include <type_traits>
 #include "fm_device.hpp"
 #include "fm_kernels.hpp"
 
@@ -400,26 +401,27 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(FM_RES
 #pragma unroll
         for (int e = 0; e < 5; e++) acc[e] = z.drodm[l + e * nd] * a.coefH;
     }
-    face_flux<KFLU, SLOPE, LAMIN, CART, 2>(f, z, rop, i, j, k, flu);
+    using Cell = std::conditional_t<CART || (KFLU == 2 && !LAMIN), MemCellApart, MemCell>;
+    face_flux<KFLU, SLOPE, LAMIN, CART, 2, Cell>(f, z, rop, i, j, k, flu);
 #pragma unroll
     for (int e = 0; e < 5; e++) acc[e] = acc[e] + flu[e];
-    face_flux<KFLU, SLOPE, LAMIN, CART, 1>(f, z, rop, i, j, k, flu);
+    face_flux<KFLU, SLOPE, LAMIN, CART, 1, Cell>(f, z, rop, i, j, k, flu);
 #pragma unroll
     for (int e = 0; e < 5; e++) acc[e] = acc[e] + flu[e];
-    face_flux<KFLU, SLOPE, LAMIN, CART, 0>(f, z, rop, i, j, k, flu);
+    face_flux<KFLU, SLOPE, LAMIN, CART, 0, Cell>(f, z, rop, i, j, k, flu);
 #pragma unroll
     for (int e = 0; e < 5; e++) acc[e] = acc[e] + flu[e];
-    face_flux<KFLU, SLOPE, LAMIN, CART, 0>(f, z, rop, i + 1, j, k, flu);
+    face_flux<KFLU, SLOPE, LAMIN, CART, 0, Cell>(f, z, rop, i + 1, j, k, flu);
 #pragma unroll
     for (int e = 0; e < 5; e++) acc[e] = acc[e] - flu[e];
     const bool jn = cb_next(j, z.cbj, z.nbj), kn = cb_next(k, z.cbk, z.nbk);
     double fj1[5];
-    face_flux<KFLU, SLOPE, LAMIN, CART, 1>(f, z, rop, i, j + 1, k, fj1);
+    face_flux<KFLU, SLOPE, LAMIN, CART, 1, Cell>(f, z, rop, i, j + 1, k, fj1);
     if (!jn) {
 #pragma unroll
         for (int e = 0; e < 5; e++) acc[e] = acc[e] - fj1[e];
     }
-    face_flux<KFLU, SLOPE, LAMIN, CART, 2>(f, z, rop, i, j, k + 1, flu);
+    face_flux<KFLU, SLOPE, LAMIN, CART, 2, Cell>(f, z, rop, i, j, k + 1, flu);
     if (!kn) {
 #pragma unroll
         for (int e = 0; e < 5; e++) acc[e] = acc[e] - flu[e];
