@@ -137,11 +137,8 @@ struct fm_ctx {
         std::vector<std::pair<long, void*>> tabs;
     };
     // What calls of several threads on one context share: held from the first use of any of it to the last
-    // (a call that reads a field while another computes an effort, or two that read fields, at once).
+    // (two calls that compute efforts, gradients or products at once).
     std::recursive_mutex shared;
-    // fields between host and device: pinned slots the copies go through (see link_copy)
-    char* link_host[4]; hipEvent_t link_ev[4];
-    size_t link_direct, faces_direct;   // bytes that went directly, to be paid for before slots are made
     double* work; size_t work_cap;      // device workspace of the adjoint and effort entry points
     int* lu_flags;                      // pinned: the error words as read
     // sweeps may have run since the error words were last read: set once a sweep is on the stream, and
@@ -177,6 +174,27 @@ static int resolve_scratch(int device) {
     return FM_OK;
 }
 
+// Pinned slots that large copies between host and device go through (see link_copy): those of a device,
+// shared by its contexts, one copy at a time (another one meanwhile goes directly), given back with the last
+// context.
+constexpr int kLinkSlots = 4;
+struct LinkPool {
+    std::mutex m;
+    char* host[kLinkSlots] = {};
+    hipEvent_t ev[kLinkSlots] = {};
+    size_t direct = 0, faces = 0;       // bytes that went directly, to be paid for before slots are made
+    int users = 0;
+};
+static LinkPool g_link[kMaxDevices];
+
+static void link_leave(int device) {
+    LinkPool& p = g_link[device];
+    std::lock_guard<std::mutex> hold(p.m);
+    if (--p.users > 0) return;
+    for (char*& h : p.host) { if (h) (void)hipHostFree(h); h = nullptr; }
+    for (hipEvent_t& e : p.ev) { if (e) (void)hipEventDestroy(e); e = nullptr; }
+}
+
 extern "C" int fm_ctx_create(fm_ctx** out, int device) {
     if (!out) return fail(FM_E_ARG, "null output");
     HIPCHK(hipSetDevice(device));
@@ -187,8 +205,6 @@ extern "C" int fm_ctx_create(fm_ctx** out, int device) {
     c->lu_batch = 1;
     c->lu_fp32 = 0;
     c->graph_on = 1;
-    for (int q = 0; q < 4; q++) { c->link_host[q] = nullptr; c->link_ev[q] = nullptr; }
-    c->link_direct = c->faces_direct = 0;
     c->work = nullptr; c->work_cap = 0;
     c->lu_unchecked = 1; c->lu_flags = nullptr;
     c->cur = nullptr;
@@ -202,6 +218,10 @@ extern "C" int fm_ctx_create(fm_ctx** out, int device) {
     c->cur = c->stream;
     HIPCHK(hipEventCreate(&c->e0));
     HIPCHK(hipEventCreate(&c->e1));
+    {
+        std::lock_guard<std::mutex> hold(g_link[device].m);
+        g_link[device].users++;
+    }
     *out = c;
     return FM_OK;
 }
@@ -242,8 +262,7 @@ extern "C" int fm_ctx_destroy(fm_ctx* c) {
         for (hipEvent_t e : t->ev) if (e) (void)hipEventDestroy(e);
     }
     if (c->flow_ctr) (void)hipFree(c->flow_ctr);
-    for (char* h : c->link_host) if (h) (void)hipHostFree(h);
-    for (hipEvent_t e : c->link_ev) if (e) (void)hipEventDestroy(e);
+    link_leave(c->device);
     if (c->work) (void)hipFree(c->work);
     if (c->lu_flags) (void)hipHostFree(c->lu_flags);
     for (hipStream_t s2 : c->side) (void)hipStreamDestroy(s2);
@@ -471,7 +490,7 @@ static double* field_ptr(Zone* z, int field, long* n) {
 // A copy between host and device memory on the context's stream, complete on return.  The runtime moves
 // pageable memory through its own pinned buffers with one thread: 17 GB/s down, 29 GB/s up, of the 50 the
 // link gives.  From the sizes on where it is faster (measured: 4 MB down 0.24 -> 0.20 ms, 300 MB 18.2 -> 6.8
-// ms; up 25 MB the same, 300 MB 11.0 -> 6.8 ms) the copy goes through four pinned slots of the context, up
+// ms; up 25 MB the same, 300 MB 11.0 -> 6.8 ms) the copy goes through four pinned slots of the device, up
 // to 4 MB at a time, two threads moving slots to or from the caller's array while others cross the link.
 // Pinned arrays go directly at every size: 58 GB/s (12 MB down 0.26 ms, 0.45 through the slots; 300 MB 6.0
 // and 7.4).
@@ -479,27 +498,36 @@ constexpr size_t kLinkSlot = (size_t)4 << 20, kLinkHalf = (size_t)2 << 20;
 constexpr size_t kLinkDown = (size_t)4 << 20, kLinkUp = (size_t)32 << 20;
 constexpr int kLinkThreads = 2;
 
-// The slots cost 0.1 to 0.2 ms a MB to make, what they save is 0.025 ms a MB (of the faces' values in slot 0:
-// 0.04): they are made once as many bytes have gone directly as pay for them, so that a program that reads a
-// field once does not pay more than it gains (12.6 MB read once: 0.8 ms, 2.1 to 2.7 if slots are made for it;
-// 33 MB 1.9 and 5.1; 4.4 MB 0.28 and 1.1 to 1.5).
+// A new slot costs 0.35 to 1 ms, what it saves is 0.025 ms a MB (of the faces' values in slot 0: 0.04): slots are
+// made once as many bytes have gone directly on the device as pay for them, so that a program that reads a
+// field once does not pay more than it gains.  First read of 12.6 MB: 0.8 ms, 2.1 to 2.7 if slots are made
+// for it; 33 MB 1.9 and 5.1; 4.4 MB 0.28 and 1.1 to 1.5.  Smaller slots (4 x 1 MB) still cost 1.2 ms and move 12.6
+// MB in 0.50 instead of 0.45 ms.
 constexpr size_t kLinkPaid = (size_t)64 << 20, kFacesPaid = (size_t)12 << 20;
 
-static bool link_slot(fm_ctx* c, int s) {
-    if (!c->link_ev[s] && hipEventCreateWithFlags(&c->link_ev[s], (unsigned)hipEventDisableTiming) != hipSuccess)
-        c->link_ev[s] = nullptr;
-    if (!c->link_host[s] && hipHostMalloc((void**)&c->link_host[s], kLinkSlot) != hipSuccess) c->link_host[s] = nullptr;
-    if (c->link_ev[s] && c->link_host[s]) return true;
+// (the pool is held by the caller)
+static bool link_slot(LinkPool& p, int s) {
+    if (!p.ev[s] && hipEventCreateWithFlags(&p.ev[s], (unsigned)hipEventDisableTiming) != hipSuccess) p.ev[s] = nullptr;
+    if (!p.host[s] && hipHostMalloc((void**)&p.host[s], kLinkSlot) != hipSuccess) p.host[s] = nullptr;
+    if (p.ev[s] && p.host[s]) return true;
     (void)hipGetLastError();
     return false;
 }
 
-// slot 0 for the values of a window's faces, by a call that holds the workspace; nullptr: an array of its own
-static double* faces_slot(fm_ctx* c, size_t bytes) {
-    if (bytes > kLinkSlot) return nullptr;
-    if (!c->link_host[0]) c->faces_direct += bytes;
-    return (c->link_host[0] || c->faces_direct >= kFacesPaid) && link_slot(c, 0) ? (double*)c->link_host[0] : nullptr;
-}
+// slot 0 for the values of a window's faces, held until the call returns; nullptr: an array of its own
+struct FacesSlot {
+    std::unique_lock<std::mutex> hold;
+    double* get(fm_ctx* c, size_t bytes) {
+        if (bytes > kLinkSlot) return nullptr;
+        LinkPool& p = g_link[c->device];
+        hold = std::unique_lock<std::mutex>(p.m, std::try_to_lock);
+        if (!hold.owns_lock()) return nullptr;
+        if (p.host[0] || (p.faces += bytes) >= kFacesPaid)
+            if (link_slot(p, 0)) return (double*)p.host[0];
+        hold.unlock();
+        return nullptr;
+    }
+};
 
 // memory the runtime knows (pinned, managed or of a device), which the link reaches without help
 static bool known_memory(const void* p) {
@@ -514,11 +542,12 @@ static hipError_t link_copy(fm_ctx* c, void* host, void* dev, size_t bytes, bool
     const size_t chunk = bytes < 4 * kLinkSlot ? kLinkHalf : kLinkSlot;
     const long n = (long)((bytes + chunk - 1) / chunk);
     int slots = 0;
-    std::unique_lock<std::recursive_mutex> hold(c->shared, std::defer_lock);
-    if (bytes >= (up ? kLinkUp : kLinkDown) && !known_memory(host)) {
-        hold.lock();
-        if (!c->link_host[1]) c->link_direct += bytes;
-        while (c->link_direct >= kLinkPaid && slots < 4 && slots < n && link_slot(c, slots)) slots++;
+    LinkPool& p = g_link[c->device];
+    std::unique_lock<std::mutex> hold(p.m, std::defer_lock);
+    if (bytes >= (up ? kLinkUp : kLinkDown) && !known_memory(host) && hold.try_lock()) {
+        if (p.direct < kLinkPaid) p.direct += bytes;
+        while (p.direct >= kLinkPaid && slots < kLinkSlots && slots < n && link_slot(p, slots)) slots++;
+        if (slots <= 1) hold.unlock();
     }
     std::vector<std::thread> th;
     std::mutex m;
@@ -538,11 +567,11 @@ static hipError_t link_copy(fm_ctx* c, void* host, void* dev, size_t bytes, bool
                 cv.wait(l, [&] { return issued >= need || err != hipSuccess; });
                 if (err != hipSuccess) return;
             }
-            if (e == hipSuccess && need > 0) e = hipEventSynchronize(c->link_ev[s]);
+            if (e == hipSuccess && need > 0) e = hipEventSynchronize(p.ev[s]);
             if (e == hipSuccess) {
                 char* h = (char*)host + (size_t)i * chunk;
-                if (up) memcpy(c->link_host[s], h, size_of(i));
-                else memcpy(h, c->link_host[s], size_of(i));
+                if (up) memcpy(p.host[s], h, size_of(i));
+                else memcpy(h, p.host[s], size_of(i));
             }
             std::lock_guard<std::mutex> l(m);
             if (e != hipSuccess && err == hipSuccess) err = e;
@@ -578,8 +607,8 @@ static hipError_t link_copy(fm_ctx* c, void* host, void* dev, size_t bytes, bool
             if (err != hipSuccess) break;
         }
         char* d = (char*)dev + (size_t)i * chunk;
-        hipError_t e = hipMemcpyAsync(up ? d : c->link_host[s], up ? c->link_host[s] : d, size_of(i), kind, c->stream);
-        if (e == hipSuccess) e = hipEventRecord(c->link_ev[s], c->stream);
+        hipError_t e = hipMemcpyAsync(up ? d : p.host[s], up ? p.host[s] : d, size_of(i), kind, c->stream);
+        if (e == hipSuccess) e = hipEventRecord(p.ev[s], c->stream);
         {
             std::lock_guard<std::mutex> l(m);
             if (e != hipSuccess && err == hipSuccess) err = e;
@@ -1146,7 +1175,8 @@ extern "C" int fm_wall_effort(fm_ctx* c, int zone, int level, int idir, const in
     // into a pinned slot where they fit one (the runtime's staging and a fresh host array took longer
     // than the kernel)
     std::vector<double> v;
-    double* h = faces_slot(c, bytes);
+    FacesSlot slot;
+    double* h = slot.get(c, bytes);
     if (!h) { v.resize((size_t)33 * nf); h = v.data(); }
     hipError_t e = hipMemcpyAsync(h, wk.p, bytes, hipMemcpyDeviceToHost, c->stream);
     if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
@@ -1228,7 +1258,8 @@ extern "C" int fm_dpj_dpw(fm_ctx* c, int zone, int level, int idir, const int* w
     a.cosa = cosa; a.sina = sina; a.surfinv = surfinv;
     a.rop = z->ro[level]; a.out = wk.p;
     std::vector<double> v;
-    double* h = faces_slot(c, bytes);
+    FacesSlot slot;
+    double* h = slot.get(c, bytes);
     if (!h) { v.resize(20 * nf); h = v.data(); }
     launch_dpj_dpw(k, a, c->stream);
     hipError_t e = hipGetLastError();

@@ -33,7 +33,8 @@ def test_pinned_and_pageable_arrays(ctxmod, n):  # noqa: F811
 @pytest.mark.parametrize("moved", [0, 48, 80])
 def test_copies_before_and_after_the_slots(ctxmod, moved):  # noqa: F811
     """Fields of 4 to 41 MB, and one below, written and read in a context that has moved that many MB
-    before: directly, from some copy on through the pinned slots, and through them from the start."""
+    before: in a process that has moved none, directly, from some copy on through the pinned slots, and
+    through them from the start."""
     sizes = [(3, 4, 5), (46, 46, 37), (46, 46, 38), (80, 80, 55), (80, 80, 56), (90, 90, 90), (90, 90, 91), (130, 97, 81)]
     ctx = ctxmod.Context(0)
     zs = [cases.tgv_zone(n, H.numerics("ausmpred", "explicit")) for n in sizes]
@@ -52,8 +53,9 @@ def test_copies_before_and_after_the_slots(ctxmod, moved):  # noqa: F811
 
 @pytest.mark.parametrize("n", [(33, 8, 17), (257, 8, 33), (400, 8, 39), (410, 8, 39)])
 def test_efforts_before_and_after_the_slot(ctxmod, n):  # noqa: F811
-    """Wall efforts and wall gradients, again and again: the first through arrays of their own, later ones
-    through the pinned slot where the window's faces fit it (the last size is above)."""
+    """Wall efforts and wall gradients, again and again: in a process that has computed none, the first
+    through arrays of their own, later ones through the pinned slot where the window's faces fit it (the
+    last size is above)."""
     z = cases.tgv_zone(n, H.numerics("ausmpred", "bdf"), perturb=0.02, flow="euler", bcs=H.INVISCID_J)
     ctx = ctxmod.Context(0)
     ctx.add_zone(z)

@@ -1,4 +1,4 @@
-"""Calls of several host threads on one context: what each would get alone."""
+"""Calls of several host threads on one context and on several: what each would get alone."""
 import threading
 
 import numpy as np
@@ -43,7 +43,7 @@ def test_threads_share_a_context(ctxmod, n):  # noqa: F811
     for q, z in enumerate(zs):
         ctx.add_zone(z)
         ctx.apply_bc(q, 0)
-    # (the copies' pinned slots are made after 64 MB)
+    # (the copies' pinned slots are made after 64 MB, whoever moved them)
     for _ in range(64 * 2**20 // zs[0].ro.nbytes + 1):
         ctx.get(0, ctxmod.FIELD_RO, np.zeros_like(zs[0].ro))
     lam = [np.random.default_rng(q).standard_normal(5 * z.nd) for q, z in enumerate(zs)]
@@ -79,3 +79,31 @@ def test_threads_share_a_context(ctxmod, n):  # noqa: F811
 
     at_once([fields(q) for q in range(len(zs))] + [adjoint(q) for q in range(len(zs))])
     ctx.close()
+
+
+@pytest.mark.parametrize("n", [(46, 46, 38), (96, 90, 90)])
+def test_contexts_of_several_threads(ctxmod, n):  # noqa: F811
+    """Four contexts, a thread each: one copy at a time goes through the device's pinned slots, the others
+    directly; contexts closed while others copy."""
+    num = H.numerics("ausmpred", "bdf")
+    made = []
+
+    def call(q):
+        def f():
+            z = cases.tgv_zone(n, num, perturb=0.02, seed=q, flow="euler", bcs=H.INVISCID_J)
+            ctx = ctxmod.Context(0)
+            ctx.add_zone(z)
+            a = np.random.default_rng(q).random(z.ro.size)
+            for _ in range(5):
+                a += 1.0
+                ctx.set(0, ctxmod.FIELD_RO_M1, a)
+                assert np.array_equal(ctx.get(0, ctxmod.FIELD_RO_M1, np.zeros_like(a)), a), q
+            w = [1, n[0], 1, 1, 1, n[2]]
+            one, two = ctx.wall_effort(0, 3, w), ctx.wall_effort(0, 3, w)
+            assert np.array_equal(one[0], two[0]) and np.array_equal(one[1], two[1]), q
+            ctx.close()
+            made.append(q)
+        return f
+
+    at_once([call(q) for q in range(4)])
+    assert len(made) == 24
