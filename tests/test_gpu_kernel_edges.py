@@ -168,3 +168,37 @@ def test_norm_blocks(ctxmod, orc, n):  # noqa: F811
     # (positive terms summed in another order: at most their number times 2^-53 apart, taken at 1e-12)
     np.testing.assert_allclose(norms[:5], np.sqrt(r[:, 0, :, 0].sum(axis=0) / np.prod(n)) / dtc, rtol=1e-12, atol=0)
     assert np.array_equal(norms[5:], r[:, 1, :, 0].max(axis=0) / dtc)
+
+
+@pytest.mark.parametrize("mode", ["local", "bdf_ss2"])
+def test_lu_stream_more_pencils_than_fit(ctxmod, orc, mode):  # noqa: F811
+    """A curvilinear zone of 625 pencils, more than the workgroups that are resident at once (some 512): a
+    workgroup takes a second pencil with its rows, products and ticket still in LDS from the first."""
+    mk = lambda: H.jittered_box((3, 200, 200), H.numerics("ausmpred", mode), bcs=H.WALL_J)
+    zo, zg, _, _ = run_pair(ctxmod, orc, mk, 2 if mode == "bdf_ss2" else 1, nsteps=2)
+    assert_same(zo, zg, ghosts=True)
+
+
+def test_lu_stream_list_more_pencils_than_fit(ctxmod):  # noqa: F811
+    """The same over two curvilinear zones in one launch, 840 pencils, against each zone alone."""
+    num = H.numerics("ausmpred", "local")
+    mks = [lambda: H.jittered_box((4, 160, 168), num, seed=1, bcs=H.WALL_J), lambda: H.jittered_box((5, 160, 168), num, seed=2)]
+
+    def run(ms):
+        ctx = ctxmod.Context(0)
+        zs = [m() for m in ms]
+        for n, z in enumerate(zs):
+            ctx.add_zone(z)
+            ctx.apply_bc(n, 0)
+            for f in (ctxmod.FIELD_RO_M1, ctxmod.FIELD_RO_P1):
+                ctx.set(n, f, ctx.get(n, ctxmod.FIELD_RO, np.zeros_like(z.ro)))
+        ctx.compute(0, 1, 1, nit_c=4, modulo_verif=0, first_it=0)
+        out = [[ctx.get(n, f, np.zeros_like(z.ro)) for f in (ctxmod.FIELD_RO, ctxmod.FIELD_DRODM)] for n, z in enumerate(zs)]
+        ctx.close()
+        return out
+
+    both = run(mks)
+    for n, m in enumerate(mks):
+        one = run([m])[0]
+        assert all(np.isfinite(a).all() for a in one)
+        assert all(np.array_equal(a, b) for a, b in zip(one, both[n])), n
