@@ -83,7 +83,7 @@ struct Zone {
 
 struct fm_ctx {
     int device;
-    int lu_schedule;         // LU_PIPELINE or LU_BLOCKS
+    int lu_schedule;         // LU_STREAM, LU_DATAFLOW, LU_BLOCKS or LU_PIPELINE
     int res_schedule;        // RES_CELLS, RES_FACES, RES_KCOL or RES_AUTO
     hipStream_t stream;
     std::vector<Zone*> zones;
@@ -119,10 +119,10 @@ struct fm_ctx {
     int lu_fp32;             // mixed precision: LU-SGS sweep arithmetic in FP32 (default off)
     int res_kcol_n;          // tile shapes: cells up k per residual workgroup (0: by the zone's size)
     int lu_flow_grid;        //   workgroups of a dataflow sweep (0: all that are resident)
-    // time steps captured as HIP graphs (FM_OPT_GRAPH): one per distinct configuration
     // inside fm_compute: the streaming LU-SGS leaves dW in its skewed rows (copied back once at
     // the end: within a time step nothing reads it before the next residual overwrites it)
     int defer_dw;
+    // time steps captured as HIP graphs (FM_OPT_GRAPH): one per distinct configuration
     struct GraphEntry {
         std::vector<const void*> ptrs;  // every zone's three level pointers
         std::vector<int> dw_pending;    // per zone, after the time step
@@ -133,7 +133,7 @@ struct fm_ctx {
         int state;                      // 1: ran once eagerly, 2: captured
         hipGraphExec_t exec;
         // device tables a captured step reads: LU (key 2 sub-iteration + mesh kind), edges and
-        // corners (key -1 - sub-iteration)
+        // corners (key -1 - sub-iteration), right-hand sides (key 2^32 + sub-iteration)
         std::vector<std::pair<long, void*>> tabs;
     };
     // What calls of several threads on one context share: held from the first use of any of it to the last
@@ -769,8 +769,6 @@ static int ensure_exchange(fm_ctx* c, Zone* z) {
     return FM_OK;
 }
 
-// Dataflow LU schedule: the face exchange (sized for the largest LU box, interior plus a wall
-// layer per side) and the block order of the LU box b (rebuilt when the box changes).
 // Streaming LU schedule of a zone: the pencil exchange, sized for the largest LU box and
 // filled with the pending pattern once (the sweeps leave it that way).
 static bool uses_stream(const fm_ctx* c, const Zone* z) {
@@ -813,6 +811,8 @@ static int ensure_flow_exchange(fm_ctx* c, Zone* z) {
     return FM_OK;
 }
 
+// Dataflow LU schedule: the face exchange and the block order of the LU box b (rebuilt when the box
+// changes).
 static int ensure_dataflow(fm_ctx* c, Zone* z, const Box& b, LuArgs& la) {
     // the dataflow schedule, and what the streaming schedule falls back to (curvilinear zones,
     // FP32 sweeps)
@@ -936,7 +936,7 @@ static void lu_stream_after(Zone* z, const LuArgs& la) {
     }
 }
 
-// One sub-iteration of one zone (gsdr3.cpp:152-444 with navier_stokes_struct.for and lhs.cpp).
+// gsdr3.cpp:152-173: the level a sub-iteration starts from
 static double* level_ssiter(const Zone* z, int nitcfg) {
     if (nitcfg == 1) return z->ro[0];
     if (z->k.itypcp <= 1) return z->ro[2];
@@ -989,6 +989,7 @@ static void rhs_done(Zone* z) {
 
 static int substep_rest(fm_ctx* c, Zone* z, int nitcfg, int lssiter_verif, int lexit_lu, int stop, LuArgs* defer);
 
+// One sub-iteration of one zone (gsdr3.cpp:152-444 with navier_stokes_struct.for and lhs.cpp).
 static int substep(fm_ctx* c, Zone* z, int nitcfg, int first_it, int lssiter_verif, int lexit_lu, int stop,
                    LuArgs* defer = nullptr) {
     KZ& k = z->k;
@@ -1697,10 +1698,7 @@ static int coins_batched(fm_ctx* c, const std::vector<CoinsZone>& co, int nblk, 
 // One time step of every zone: sub-iterations n0..n1 (gsdr3 per sub-iteration).
 static int time_step(fm_ctx* c, int first_it, int verif, int n0, int n1, fm_ctx::GraphEntry* ge, bool capture) {
     const size_t nz = c->zones.size();
-    // several zones: their LU-SGS sweeps share one launch per block diagonal
-    // several zones: the batched blocks schedule (one launch per diagonal for all zones) also
-    // stands in for the dataflow schedule, whose per-zone launches and exchange fills cost more
-    // than they save on many small zones
+    // several zones: their LU-SGS sweeps share launches (one per sweep; blocks schedule: one per diagonal)
     const bool batch = nz > 1 && c->lu_batch &&
                        (c->lu_schedule == LU_BLOCKS || c->lu_schedule == LU_DATAFLOW || c->lu_schedule == LU_STREAM);
     std::vector<int> lexit(nz);

@@ -380,7 +380,7 @@ __device__ void wall_correction(const FluxConst& f, const KZ& z, const double* _
 __device__ __forceinline__ bool cb_next(int c, int size, int nb) { return c % size == 0 && c / size < nb; }
 // Update: core3as2.for (implicit, writes the Newton residual into drodm) or core3ark3.for
 // (explicit, keeps drodm and writes the new stage state).
-// FM_RES_WAVES: waves per SIMD the register allocation of k_residual aims at (2: no spills)
+// FM_RES_WAVES: waves per SIMD the register allocation of k_residual aims at (2: spills only with laminar Roe)
 #ifndef FM_RES_WAVES
 #define FM_RES_WAVES 2
 #endif

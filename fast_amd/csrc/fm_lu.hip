@@ -877,10 +877,14 @@ __global__ __launch_bounds__(64) void k_lu_pipe(KZ z, LuArgs a, const double* __
 //  * Pencils hand their j-face (k-face) products to the next pencil in sweep order through a
 //    global exchange, one value per (pencil, lane, variable, cell), with agent-scope stores; wave 5 of
 //    the consumer loads them two steps ahead and re-reads values that are still the pending
-//    pattern (bounded waits, error word).  A hand-over costs the 8 steps of the pencil's lines and
-//    about 3 us.  The exchange is filled with the pending pattern before each sweep (one fill kernel:
-//    cheaper than agent-scope stores giving every slot back, whose write-through holds up the loads
-//    issued after them).
+//    pattern (bounded waits, error word).  A hand-over costs 6.0 us of a sweep (3dfull 7.0): the 8 steps of
+//    the pencil's lines and 2.8 us.  So a sweep alone takes 4.4 + 0.405 (ni + 14) us (3dfull 0.53 a step), 8 more
+//    once any pencil waits, and 6.0 a pencil diagonal: 128 x 8 x 256 257 us, 128 x 64 x 64 158 as this gives.
+//    With more pencils at once the steps get slower: 128 x 128 x 64 218 for 202, 128^3 323 for 250, 512 x 64 x 64
+//    412 for 309 (each pencil then waits for the slower of two; not taken apart further).  The exchange holds the pending pattern between sweeps, whatever box they have: it is filled
+//    once when allocated and again after a wait gave up (check_lu), and wave 0 gives back the slots of step s in
+//    the second half of step s, wave 5 having read them before its end of step s - 1.  (Given back by wave 5
+//    itself, the write-through stores held up its loads of the next steps.)
 //  * Pencils are taken from a counter in diagonal order (reversed for the upper sweep): a pencil
 //    only waits on pencils handed out before it, so there is no deadlock whatever the dispatch
 //    order.
@@ -912,9 +916,6 @@ long lu_skew_size(bool cart, int ni, int nj, int nk) {
     long nt = (long)((nj + 7) / 8) * ((nk + 7) / 8);
     return nt * (ni + 14) * (cart ? 16 : 25) * 64;
 }
-
-// arrays the pack copies, in launch order: the right-hand side, the state (unless a.w_ready), the
-// coefficients, the normals (3dfull, unless a.n_ready)
 
 // Exchange: value e of cell ii on line l8 of the j (face 0) or k (face 1) side of consuming pencil t
 // at (((face ntile + t) (ni + 7) + ii + l8) 5 + e) 8 + l8.  The eight lines of a face handle cells with
@@ -1516,7 +1517,6 @@ void flow(const KZ& z, const LuArgs& a, hipStream_t st) {
     constexpr int CI = lu_ci<CART>();
     int ni = a.i1 - a.i0 + 1, nj = a.j1 - a.j0 + 1, nk = a.k1 - a.k0 + 1;
     int nbi = (ni + CI - 1) / CI, nbj = (nj + 7) / 8, nbk = (nk + 7) / 8;
-    long nx = lu_flow_exchange_size(CART, ni, nj, nk);
     // as many workgroups as can be resident at once (measured: 512 on a Cartesian zone beat 1024
     // and 2048, whose extra workgroups only queue behind the resident ones)
     int cus = 0, dev = 0, per = 0;
@@ -1530,7 +1530,6 @@ void flow(const KZ& z, const LuArgs& a, hipStream_t st) {
     unsigned grid = (unsigned)(a.flow_n < cap ? a.flow_n : cap);
     // the exchange is pending before a sweep (filled when allocated, and every slot a sweep writes
     // is read and given back by its consumer): only the block counter is reset
-    (void)nx;
     hipLaunchKernelGGL(k_fill_lin, dim3(1), dim3(64), 0, st, a.fx, 0L, kLuPending, a.sync);
     if (a.fp32) hipLaunchKernelGGL((k_lu_flow<CART, true, CI, float>), dim3(grid), dim3(256), 0, st, z, a, nbi, nbj, nbk);
     else if (a.flow_step) hipLaunchKernelGGL((k_lu_flow<CART, true, CI, double, true>), dim3(grid), dim3(256), 0, st, z, a, nbi, nbj, nbk);
@@ -1754,7 +1753,6 @@ void launch_lu(const KZ& z, const LuArgs& a, hipStream_t st) {
     else { sweep<false, true>(z, a, st); sweep<false, false>(z, a, st); }
 }
 
-// error word of the pipelined sweeps (a bounded wait gave up); clears it
 void launch_copy_box(const KZ& z, const double* src, double* dst, Box b, hipStream_t st) {
     int n0 = b.i1 - b.i0 + 1, n1 = b.j1 - b.j0 + 1, n2 = b.k1 - b.k0 + 1;
     if (n0 <= 0 || n1 <= 0 || n2 <= 0) return;
