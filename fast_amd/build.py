@@ -1,8 +1,8 @@
 """Build the fastmi HIP library (libfastmi.so) in-tree for gfx950.
 
 Floating-point contraction is disabled (``-ffp-contract=off``) so that the kernels reproduce
-the reference FastS kernels bit for bit; packed FP32 instructions are disabled as required on
-this hardware pool.
+the reference FastS kernels bit for bit; packed FP32 instructions are disabled (some of their
+forms have given wrong results).
 """
 import os
 import subprocess

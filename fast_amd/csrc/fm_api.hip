@@ -814,8 +814,7 @@ static int ensure_flow_exchange(fm_ctx* c, Zone* z) {
 // Dataflow LU schedule: the face exchange and the block order of the LU box b (rebuilt when the box
 // changes).
 static int ensure_dataflow(fm_ctx* c, Zone* z, const Box& b, LuArgs& la) {
-    // the dataflow schedule, and what the streaming schedule falls back to (curvilinear zones,
-    // FP32 sweeps)
+    // the dataflow schedule, and what the streaming schedule falls back to (FP32 sweeps)
     if (c->lu_schedule != LU_DATAFLOW && !(c->lu_schedule == LU_STREAM && !uses_stream(c, z))) return FM_OK;
     const KZ& k = z->k;
     if (int rc = ensure_flow_exchange(c, z)) return rc;

@@ -866,7 +866,7 @@ __global__ __launch_bounds__(64) void k_lu_pipe(KZ z, LuArgs a, const double* __
 //    (one barrier a step) took 0.55 us; rows loaded into registers by each wave 0.57 us (four waves
 //    reading the same rows kept the CU's vector memory path busy for half of the step).
 //    Lower + upper sweep, one wave -> this: 256 x 8 x 8 0.60 -> 0.23 ms, 256 x 128 x 128 1.56 -> 0.81,
-//    256^3 2.93 -> 1.97 ms (there 180 + 238 bytes a cell at 3.2 and 3.8 TB/s bound it), channel
+//    256^3 2.93 -> 1.97 ms (there 189 + 247 bytes a cell at 3.3 and 3.9 TB/s bound it), channel
 //    257 x 129 x 33 (3dfull) 1.58 -> 0.68, 513 x 257 x 65 3.23 -> 1.77 ms.
 //  * Inputs come from a skewed, pencil-major copy made before the sweeps (k_lu_pack): row r of a
 //    pencil holds, for each lane, the cell r - jj - kk of its line (right-hand side, state, the
