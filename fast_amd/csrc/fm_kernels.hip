@@ -1349,7 +1349,9 @@ static void res_scheme(const KZ& z, const RhsArgs& a, hipStream_t st) {
     // four waves of a group of rows would have no cell, where k_residual's leave at once.  us, planes and
     // cells, 1024 x 1 x 128: AUSM+(P) laminar 35 and 20, Euler 27 and 14, Roe Euler 44 and 24, 3dfull AUSM+(P)
     // 102 and 71; x 2 x: Euler 28 and 22, Roe 45 and 42, 3dfull 36 and 27, but laminar 35 and 35, 106 and 122;
-    // x 3 x: Euler 30 and 29, Roe 47 and 46.  (Small zones take 9 us either way.)
+    // x 3 x: Euler 30 and 29, Roe 47 and 46.  (Small zones take 9 us either way.  Left to the planes: Roe Euler
+    // zones of 260 000 cells whose rows are whole waves, 35 to 37 us and 31 implicit, 32 and 30 explicit: at 150 000
+    // and 520 000 cells the two are alike, and rows of 60 or 66 cells take 27 and 31, 35 and 74.)
     const bool few = z.nj == 1 || (z.nj == 2 && !lamin);
     if (a.schedule == RES_CELLS || (a.schedule == RES_AUTO && few)) res_lc<KFLU, SLOPE>(z, a, lamin, g, st);
     else res_planes<KFLU, SLOPE>(z, a, lamin, st);
